@@ -26,9 +26,9 @@ import sys
 import numpy as np
 import torch
 
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-if os.path.join(ROOT, "mini-caffe_amd") not in sys.path:
-    sys.path.insert(0, os.path.join(ROOT, "mini-caffe_amd"))
+# the package of the tree this file is run for: its root is the working folder
+if os.path.join(os.getcwd(), "mini-caffe_amd") not in sys.path:
+    sys.path.insert(0, os.path.join(os.getcwd(), "mini-caffe_amd"))
 
 import minicaffe as mc  # noqa: E402
 from minicaffe import craft, zoo  # noqa: E402
