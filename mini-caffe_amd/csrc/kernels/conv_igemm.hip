@@ -38,7 +38,10 @@ constexpr int LDK = BK + 4;  // LDS row pitch in floats
 
 typedef float acc16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-constexpr int kModeMasks = 0, kModeOneMask = 1, kModePointwise = 2, kModePointwiseQuad = 3;
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+constexpr int kModeMasks = 0, kModeOneMask = 1, kModePointwise = 2;
 // Buffer descriptor word 3 for raw dword access on gfx9-family CDNA parts
 // (32-bit data format, no swizzle, offsets checked against num_records).
 constexpr int kBufferFlags = 0x00020000;
@@ -48,7 +51,8 @@ constexpr unsigned kNoElement = 0x80000000u;
 
 struct IgemmArgs {
   const float* __restrict__ x;
-  const float* __restrict__ wt;
+  const float* __restrict__ wt;           // packed filter, fp32 (pack_weights_kernel), or null
+  const uint16_t* __restrict__ wt_split;  // packed filter, three bf16 planes, or null
   float* __restrict__ y;
   const int4* __restrict__ ktab;  // [Kpad] {byte offset, row-tap index, column-tap index, 0}
   const int* __restrict__ tap_dh;  // bottom row offset of row-tap index b
@@ -117,6 +121,200 @@ __device__ __forceinline__ float apply_act(float v, int act, float slope) {
   }
 }
 
+// What follows the K loop: the sum over K slices inside the launch, then the layer's
+// epilogue and the store.  `factors`: (scale, shift) of tile row r at factors + r * FPITCH
+// bytes, in LDS; `arrived`: one int of LDS that no wavefront needs any more after a barrier.
+template <int BM, int BN, int TM, int TN, int FPITCH, int AHEAD>
+__device__ __forceinline__ void finish_tile(const IgemmArgs& a, int slices, int sub_index, int kslice, int g,
+                                            int mt, int nt, int wm0, int wn0, acc16 (&acc)[TM][TN],
+                                            const char* factors, int* arrived, const float* scale_ptr,
+                                            const float* shift_ptr, float* __restrict__ yout) {
+  const int tid = threadIdx.x;
+  const int l32 = tid & 31, lhi = (tid & 63) >> 5;
+  // What the epilogue reads from the argument block is fetched here in one batch:
+  // fetched where it is first used, the fields cost the wavefront four or five
+  // scalar-memory round trips after the last MFMA, one after the other.  (Before the K
+  // loop they would not fit the scalar registers the loop needs.)
+  struct {
+    int* counters;
+    const float* residual;
+    unsigned y_bytes, div_hw_mul, div_hw_shift, div_w_mul, div_w_shift;
+    int y_cstride, y_nstride, Wo, out_sh, out_sw, out_oh, out_ow, M, P, HqWq, Wq, act;
+    float slope;
+  } e = {a.counters, a.residual, a.y_bytes, a.div_hw_mul, a.div_hw_shift, a.div_w_mul, a.div_w_shift,
+         a.y_cstride, a.y_nstride, a.Wo, a.out_sh, a.out_sw, a.out_oh, a.out_ow, a.M, a.P, a.HqWq, a.Wq,
+         a.act, a.slope};
+  asm volatile("" ::"s"(e.counters), "s"(e.residual), "s"(e.y_bytes), "s"(e.div_hw_mul), "s"(e.div_hw_shift),
+               "s"(e.div_w_mul), "s"(e.div_w_shift), "s"(e.y_cstride), "s"(e.y_nstride), "s"(e.Wo),
+               "s"(e.out_sh), "s"(e.out_sw), "s"(e.out_oh), "s"(e.out_ow), "s"(e.M), "s"(e.P), "s"(e.HqWq),
+               "s"(e.Wq), "s"(e.act), "s"(e.slope));
+
+  if (e.counters != nullptr) {
+    // K slices summed here: see IgemmArgs::partial.  The partial sums and the
+    // counter are accessed with device-scope atomic operations only (relaxed
+    // stores and loads that go past the per-XCD L2, which is not coherent with
+    // the other seven), so no cache write-back or invalidation is needed: a
+    // workgroup waits until its own stores have completed and then counts.
+    // What this rests on is particular to the parts it is built for: a store with
+    // device scope (sc1) is written through to the memory side, where all XCDs meet,
+    // and vmcnt counts it down only when that write has been acknowledged; an
+    // atomic on the counter issued after the wait is therefore ordered behind the
+    // partial sums at the one place every later device-scope load reads from.  The
+    // language's memory model promises none of this for relaxed accesses.
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx942__) && !defined(__gfx950__)
+#error "the in-launch sum of K slices relies on gfx942 / gfx950 device-scope write-through"
+#endif
+    const int tile_id = (sub_index * gridDim.y + g) * gridDim.x + blockIdx.x;
+    constexpr int kRegs = TM * TN * 16;  // accumulator registers per thread
+    float* mine = a.partial +
+                  (static_cast<size_t>(kslice) * a.partial_tiles + tile_id) * (kRegs * 256) + tid;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          __hip_atomic_store(mine + ((i * TN + j) * 16 + r) * 256, acc[i][j][r], __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's partial sums have arrived
+    __syncthreads();  // ... every thread's, and every wave is done with the tiles in LDS
+    if (tid == 0)
+      arrived[0] = __hip_atomic_fetch_add(&e.counters[tile_id], 1, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (arrived[0] != slices - 1) return;  // uniform over the workgroup
+    // the next launch on this stream starts from zero
+    if (tid == 0)
+      __hip_atomic_store(&e.counters[tile_id], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // Slices are added in slice order, the loads of AHEAD of them together (as many as the
+    // registers hold): one at a time each costs a round trip to memory (2048 -> 512 1x1
+    // on one 7x7 map, eight slices: 12.9 us, four at a time 11.8).
+    const float* part = a.partial + static_cast<size_t>(tile_id) * (kRegs * 256) + tid;
+    const size_t slice_elems = static_cast<size_t>(a.partial_tiles) * (kRegs * 256);
+#pragma unroll
+    for (int r = 0; r < kRegs; ++r)
+      acc[r / 16 / TN][r / 16 % TN][r % 16] =
+          __hip_atomic_load(part + r * 256, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int z = 1; z < slices; z += AHEAD) {
+      float v[AHEAD][kRegs];
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u) {
+        // (a slice past the last one is read as the last one and not added)
+        const float* from = part + min(z + u, slices - 1) * slice_elems;
+#pragma unroll
+        for (int r = 0; r < kRegs; ++r)
+          v[u][r] = __hip_atomic_load(from + r * 256, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u)
+        if (z + u < slices) {
+#pragma unroll
+          for (int r = 0; r < kRegs; ++r) acc[r / 16 / TN][r / 16 % TN][r % 16] += v[u][r];
+        }
+    }
+  }
+
+  // Epilogue.  Accumulator register r of lane l holds row 8*(r/4)+4*(l/32)+r%4,
+  // column l%32 of its 32x32 block; a half-wave therefore stores 32 consecutive
+  // pixels of one output channel.  Like the K loop it addresses through buffer
+  // descriptors: one VGPR offset per lane (bit 31 set for a column past the last
+  // pixel, which drops its stores), the row as a scalar offset.  Per-channel
+  // factors and residual values are fetched eight rows at a time, all loads of
+  // a batch issued before the first use.
+  const bool has_scale = scale_ptr != nullptr;
+  const bool has_shift = shift_ptr != nullptr;
+  const bool has_res = e.residual != nullptr;
+  const __amdgpu_buffer_rsrc_t yres =
+      __builtin_amdgcn_make_buffer_rsrc(yout, 0, e.y_bytes, kBufferFlags);
+  const __amdgpu_buffer_rsrc_t rres = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(e.residual), 0, has_res ? e.y_bytes : 0, kBufferFlags);
+  // 0: none, 1: ReLU (max with 0), 2: leaky ReLU, 3: TanH / Sigmoid
+  const int act_mode = e.act == MC_ACT_NONE ? 0
+                       : e.act == MC_ACT_RELU ? (e.slope == 0.f ? 1 : 2)
+                                              : 3;
+  const unsigned cs4 = static_cast<unsigned>(e.y_cstride) * 4;
+#define MC_ROW(r) (8 * ((r) / 4) + ((r) % 4))
+#define MC_LOADF(res, voff, soff) \
+  __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(res, voff, soff, 0))
+#define MC_STORE_ROWS(EXPR)                                                                  \
+  _Pragma("unroll") for (int q = 0; q < 8; ++q) {                                            \
+    const float v = acc[i][j][half * 8 + q];                                                 \
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, (EXPR)), yres, y_voff,\
+                                          MC_ROW(half * 8 + q) * cs4, 0);                    \
+  }
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int p = nt * BN + wn0 + j * 32 + l32;
+    const int n = fast_div(p, e.div_hw_mul, e.div_hw_shift);
+    const int rem = p - n * e.HqWq;
+    int ybase;
+    const int qh = fast_div(rem, e.div_w_mul, e.div_w_shift);
+    const int qw = rem - qh * e.Wq;
+    ybase = n * e.y_nstride + (qh * e.out_sh + e.out_oh) * e.Wo + qw * e.out_sw + e.out_ow;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int mblock = mt * BM + wm0 + i * 32;  // wave-uniform
+      const int m0 = mblock + 4 * lhi;
+      if (mblock + 32 <= e.M) {
+        // All 32 rows are real channels.
+        const unsigned c0 = g * e.M + m0;
+        const unsigned y_voff =
+            p < e.P ? static_cast<unsigned>(ybase + c0 * e.y_cstride) * 4 : kNoElement;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          if (has_scale | has_shift) {
+            float sc[8], sh[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+              const int lrow = wm0 + i * 32 + 4 * lhi + MC_ROW(half * 8 + q);
+              const float2 f = *reinterpret_cast<const float2*>(factors + lrow * FPITCH);
+              sc[q] = f.x;
+              sh[q] = f.y;
+            }
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+              acc[i][j][half * 8 + q] = acc[i][j][half * 8 + q] * sc[q] + sh[q];
+          }
+          if (has_res) {
+            float rs[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) rs[q] = MC_LOADF(rres, y_voff, MC_ROW(half * 8 + q) * cs4);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) acc[i][j][half * 8 + q] += rs[q];
+          }
+          if (act_mode == 0) {
+            MC_STORE_ROWS(v)
+          } else if (act_mode == 1) {
+            MC_STORE_ROWS(fmaxf(v, 0.f))
+          } else if (act_mode == 2) {
+            MC_STORE_ROWS(v > 0.f ? v : v * e.slope)
+          } else {
+            MC_STORE_ROWS(apply_act(v, e.act, e.slope))
+          }
+        }
+      } else if (p < e.P) {
+        // Block straddles the last channel: row by row, skipping rows >= M.
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int m = m0 + MC_ROW(r);
+          if (m < e.M) {
+            const int c = g * e.M + m;
+            float v = acc[i][j][r];
+            if (has_scale) v *= a.scale[c];
+            if (has_shift) v += a.shift[c];
+            const int yo = ybase + c * e.y_cstride;
+            if (has_res) v += e.residual[yo];
+            yout[yo] = apply_act(v, e.act, e.slope);
+          }
+        }
+      }
+    }
+  }
+#undef MC_ROW
+#undef MC_LOADF
+#undef MC_STORE_ROWS
+}
+
 // OCC = wavefronts per SIMD the register allocation must leave room for.
 // MODE selects how the K loop finds and guards the elements it gathers:
 //   kModeMasks     tap table + one "outside the image" bit mask per tap row and
@@ -128,11 +326,6 @@ __device__ __forceinline__ float apply_act(float v, int act, float slope) {
 //                  rows a thread gathers per step share one tap and one
 //                  validity test;
 //   kModePointwise no table and no mask, see below;
-//   kModePointwiseQuad  the same for stride 1 on planes of a multiple of four pixels with
-//                  K a multiple of 16 (64-pixel tile only): a thread fetches four
-//                  consecutive pixels of one channel with one 16-byte load instead of
-//                  one pixel of four channels with four loads, and transposes them on
-//                  the way into LDS (four 4-byte stores).  Same products, same order.
 // Pointwise: every row k of the gather is channel k of the bottom blob
 // at the thread's own pixel (1x1 kernel, no padding), so the K loop needs no
 // tap table and no bounds handling at all.
@@ -221,28 +414,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
   const int pj = tid % BN;
   const int prow = tid / BN;  // wave-uniform because BN >= 64
   // byte offset of the pixel's origin from the descriptor base (never negative)
-  constexpr bool PW4 = MODE == kModePointwiseQuad;  // pointwise, stride 1: four pixels of a channel per load
-  constexpr bool PW = MODE == kModePointwise || PW4;
-  static_assert(!PW4 || (BN == 64 && KS == 1), "the pixel-quad gather is built for the 64-pixel tile");
+  constexpr bool PW = MODE == kModePointwise;
   unsigned xvoff = PW ? kNoElement : 0u;
   unsigned row_bad = 0xFFFFFFFFu, col_bad = 0xFFFFFFFFu;
   {
-    // PW4: thread = (K row tid % 16, pixel quad tid / 16); the plane is a multiple of four
-    // pixels, so a quad never straddles two images
-    const int p = PW4 ? nt * BN + 4 * (tid >> 4) : nt * BN + pj;
+    const int p = nt * BN + pj;
     // (the divisions are prepared for every column of the last tile, also those past the
     // last pixel: the pointwise modes compute first and pick afterwards, without a branch)
     const int n = fast_div(p, a.div_hw_mul, a.div_hw_shift);
     const int rem = p - n * a.HqWq;
-    // (the pixel-quad mode runs only where pixel `rem` of the iteration grid is element
-    // `rem` of the bottom plane and of the top plane: no row and column needed)
-    const int qh = PW4 ? 0 : fast_div(rem, a.div_w_mul, a.div_w_shift);
-    const int qw = PW4 ? 0 : rem - qh * a.Wq;
+    const int qh = fast_div(rem, a.div_w_mul, a.div_w_shift);
+    const int qw = rem - qh * a.Wq;
     const int hi0 = qh * a.q_sh + a.in_oh;
     const int wi0 = qw * a.q_sw + a.in_ow;
-    unsigned origin = static_cast<unsigned>(
-        ((n * a.x_nstride + g * a.x_gstride + (PW4 ? rem : hi0 * a.W + wi0)) << 2) + a.pix_shift);
-    if constexpr (PW4) origin += static_cast<unsigned>(tid & 15) * (static_cast<unsigned>(a.x_cstride) * 4u);
+    const unsigned origin = static_cast<unsigned>(
+        ((n * a.x_nstride + g * a.x_gstride + hi0 * a.W + wi0) << 2) + a.pix_shift);
     if constexpr (PW) xvoff = p < a.P ? origin : kNoElement;
     if (!PW && p < a.P) {
       xvoff = origin;
@@ -288,8 +474,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
   const unsigned wt_kt_bytes = static_cast<unsigned>(a.Mpad) * BK * 4;
   const unsigned wt_g_bytes = static_cast<unsigned>(g) * (a.Kpad / BK) * wt_kt_bytes;
   // (said to be uniform: the compiler otherwise merges this load with the one inside the
-  // divergent branch above into a vector register, and every pixel-quad load of the K
-  // loop, whose scalar offset is a multiple of it, gets wrapped in a loop over lanes)
+  // divergent branch above into a vector register, and every load of the K loop, whose
+  // scalar offset is a multiple of it, gets wrapped in a loop over lanes)
   const unsigned x_cbytes = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(a.x_cstride) * 4);
   const int kmax = a.K - 1;
 
@@ -319,12 +505,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
     _Pragma("unroll") for (int i = 0; i < B_Q; ++i) {                                        \
       const int krow =                                                                       \
           __builtin_amdgcn_readfirstlane(kt16 * BK + (i * ROWS_PER_PASS + prow) * 4);        \
-      if constexpr (PW4) {                                                                   \
-        /* K is a multiple of 16 here: no padding rows */                                    \
-        const u32x4 q4 = __builtin_amdgcn_raw_buffer_load_b128(                              \
-            xres, xvoff, static_cast<unsigned>(kt16 * BK) * x_cbytes, 0);                    \
-        breg[ks][i] = __builtin_bit_cast(float4, q4);                                        \
-      } else if constexpr (PW) {                                                             \
+      if constexpr (PW) {                                                                    \
         /* padding rows re-read the last channel; their filter rows are zero */              \
         breg[ks][i].x = MC_LOADF(xres, xvoff, static_cast<unsigned>(min(krow, kmax)) * x_cbytes);\
         breg[ks][i].y =                                                                          \
@@ -361,16 +542,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
         *reinterpret_cast<float4*>(&As[buf][ks][f / QUADS][(f % QUADS) * 4]) = areg[ks][i];  \
     }                                                                                        \
     _Pragma("unroll") for (int i = 0; i < B_Q; ++i) {                                        \
-      if constexpr (PW4) {                                                                   \
-        float* col = &Bs[buf][ks][4 * (tid >> 4)][tid & 15];                                 \
-        col[0] = breg[ks][i].x;                                                              \
-        col[LDK] = breg[ks][i].y;                                                            \
-        col[2 * LDK] = breg[ks][i].z;                                                        \
-        col[3 * LDK] = breg[ks][i].w;                                                        \
-      } else {                                                                               \
-        *reinterpret_cast<float4*>(&Bs[buf][ks][pj][(i * ROWS_PER_PASS + prow) * 4]) =       \
-            breg[ks][i];                                                                     \
-      }                                                                                      \
+      *reinterpret_cast<float4*>(&Bs[buf][ks][pj][(i * ROWS_PER_PASS + prow) * 4]) =         \
+          breg[ks][i];                                                                       \
     }                                                                                        \
   }
   // One MFMA K step multiplies k-pairs; which two physical k rows form a pair
@@ -500,189 +673,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 #undef MC_COMPUTE
 #undef MC_INTERLEAVE
 
-  // What the epilogue reads from the argument block is fetched here in one batch:
-  // fetched where it is first used, the fields cost the wavefront four or five
-  // scalar-memory round trips after the last MFMA, one after the other.  (Before the K
-  // loop they would not fit the scalar registers the loop needs.)
-  struct {
-    int* counters;
-    const float* residual;
-    unsigned y_bytes, div_hw_mul, div_hw_shift, div_w_mul, div_w_shift;
-    int y_cstride, y_nstride, Wo, out_sh, out_sw, out_oh, out_ow, M, P, HqWq, Wq, act;
-    float slope;
-  } e = {a.counters, a.residual, a.y_bytes, a.div_hw_mul, a.div_hw_shift, a.div_w_mul, a.div_w_shift,
-         a.y_cstride, a.y_nstride, a.Wo, a.out_sh, a.out_sw, a.out_oh, a.out_ow, a.M, a.P, a.HqWq, a.Wq,
-         a.act, a.slope};
-  asm volatile("" ::"s"(e.counters), "s"(e.residual), "s"(e.y_bytes), "s"(e.div_hw_mul), "s"(e.div_hw_shift),
-               "s"(e.div_w_mul), "s"(e.div_w_shift), "s"(e.y_cstride), "s"(e.y_nstride), "s"(e.Wo),
-               "s"(e.out_sh), "s"(e.out_sw), "s"(e.out_oh), "s"(e.out_ow), "s"(e.M), "s"(e.P), "s"(e.HqWq),
-               "s"(e.Wq), "s"(e.act), "s"(e.slope));
-
-  if (e.counters != nullptr) {
-    // K slices summed here: see IgemmArgs::partial.  The partial sums and the
-    // counter are accessed with device-scope atomic operations only (relaxed
-    // stores and loads that go past the per-XCD L2, which is not coherent with
-    // the other seven), so no cache write-back or invalidation is needed: a
-    // workgroup waits until its own stores have completed and then counts.
-    // What this rests on is particular to the parts it is built for: a store with
-    // device scope (sc1) is written through to the memory side, where all XCDs meet,
-    // and vmcnt counts it down only when that write has been acknowledged; an
-    // atomic on the counter issued after the wait is therefore ordered behind the
-    // partial sums at the one place every later device-scope load reads from.  The
-    // language's memory model promises none of this for relaxed accesses.
-#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx942__) && !defined(__gfx950__)
-#error "the in-launch sum of K slices relies on gfx942 / gfx950 device-scope write-through"
-#endif
-    const int tile_id = (sub_index * gridDim.y + g) * gridDim.x + blockIdx.x;
-    constexpr int kRegs = TM * TN * 16;  // accumulator registers per thread
-    float* mine = a.partial +
-                  (static_cast<size_t>(kslice) * a.partial_tiles + tile_id) * (kRegs * 256) + tid;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          __hip_atomic_store(mine + ((i * TN + j) * 16 + r) * 256, acc[i][j][r], __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's partial sums have arrived
-    __syncthreads();  // ... every thread's, and every wave is done with the tiles in LDS
-    int* arrived = reinterpret_cast<int*>(&As[0][0][0][0]);
-    if (tid == 0)
-      arrived[0] = __hip_atomic_fetch_add(&e.counters[tile_id], 1, __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (arrived[0] != batch.slices - 1) return;  // uniform over the workgroup
-    // the next launch on this stream starts from zero
-    if (tid == 0)
-      __hip_atomic_store(&e.counters[tile_id], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const float* part = a.partial + static_cast<size_t>(tile_id) * (kRegs * 256) + tid;
-    const size_t slice_elems = static_cast<size_t>(a.partial_tiles) * (kRegs * 256);
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          acc[i][j][r] = __hip_atomic_load(part + ((i * TN + j) * 16 + r) * 256, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-    for (int z = 1; z < batch.slices; ++z) {
-      part += slice_elems;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            acc[i][j][r] += __hip_atomic_load(part + ((i * TN + j) * 16 + r) * 256, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
-
-  // Epilogue.  Accumulator register r of lane l holds row 8*(r/4)+4*(l/32)+r%4,
-  // column l%32 of its 32x32 block; a half-wave therefore stores 32 consecutive
-  // pixels of one output channel.  Like the K loop it addresses through buffer
-  // descriptors: one VGPR offset per lane (bit 31 set for a column past the last
-  // pixel, which drops its stores), the row as a scalar offset.  Per-channel
-  // factors and residual values are fetched eight rows at a time, all loads of
-  // a batch issued before the first use.
-  const bool has_scale = scale_ptr != nullptr;
-  const bool has_shift = shift_ptr != nullptr;
-  const bool has_res = e.residual != nullptr;
-  const __amdgpu_buffer_rsrc_t yres =
-      __builtin_amdgcn_make_buffer_rsrc(yout, 0, e.y_bytes, kBufferFlags);
-  const __amdgpu_buffer_rsrc_t rres = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(e.residual), 0, has_res ? e.y_bytes : 0, kBufferFlags);
-  // 0: none, 1: ReLU (max with 0), 2: leaky ReLU, 3: TanH / Sigmoid
-  const int act_mode = e.act == MC_ACT_NONE ? 0
-                       : e.act == MC_ACT_RELU ? (e.slope == 0.f ? 1 : 2)
-                                              : 3;
-  const unsigned cs4 = static_cast<unsigned>(e.y_cstride) * 4;
-#define MC_ROW(r) (8 * ((r) / 4) + ((r) % 4))
-#define MC_LOADF(res, voff, soff) \
-  __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(res, voff, soff, 0))
-#define MC_STORE_ROWS(EXPR)                                                                  \
-  _Pragma("unroll") for (int q = 0; q < 8; ++q) {                                            \
-    const float v = acc[i][j][half * 8 + q];                                                 \
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, (EXPR)), yres, y_voff,\
-                                          MC_ROW(half * 8 + q) * cs4, 0);                    \
-  }
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int p = nt * BN + wn0 + j * 32 + l32;
-    const int n = fast_div(p, e.div_hw_mul, e.div_hw_shift);
-    const int rem = p - n * e.HqWq;
-    int ybase;
-    if constexpr (PW4) {
-      ybase = n * e.y_nstride + rem;
-    } else {
-      const int qh = fast_div(rem, e.div_w_mul, e.div_w_shift);
-      const int qw = rem - qh * e.Wq;
-      ybase = n * e.y_nstride + (qh * e.out_sh + e.out_oh) * e.Wo + qw * e.out_sw + e.out_ow;
-    }
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int mblock = mt * BM + wm0 + i * 32;  // wave-uniform
-      const int m0 = mblock + 4 * lhi;
-      if (mblock + 32 <= e.M) {
-        // All 32 rows are real channels.
-        const unsigned c0 = g * e.M + m0;
-        const unsigned y_voff =
-            p < e.P ? static_cast<unsigned>(ybase + c0 * e.y_cstride) * 4 : kNoElement;
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          if (has_scale | has_shift) {
-            float sc[8], sh[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-              const int lrow = wm0 + i * 32 + 4 * lhi + MC_ROW(half * 8 + q);
-              const float2 f = *reinterpret_cast<const float2*>(&As[0][0][lrow][BK]);
-              sc[q] = f.x;
-              sh[q] = f.y;
-            }
-#pragma unroll
-            for (int q = 0; q < 8; ++q)
-              acc[i][j][half * 8 + q] = acc[i][j][half * 8 + q] * sc[q] + sh[q];
-          }
-          if (has_res) {
-            float rs[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) rs[q] = MC_LOADF(rres, y_voff, MC_ROW(half * 8 + q) * cs4);
-#pragma unroll
-            for (int q = 0; q < 8; ++q) acc[i][j][half * 8 + q] += rs[q];
-          }
-          if (act_mode == 0) {
-            MC_STORE_ROWS(v)
-          } else if (act_mode == 1) {
-            MC_STORE_ROWS(fmaxf(v, 0.f))
-          } else if (act_mode == 2) {
-            MC_STORE_ROWS(v > 0.f ? v : v * e.slope)
-          } else {
-            MC_STORE_ROWS(apply_act(v, e.act, e.slope))
-          }
-        }
-      } else if (p < e.P) {
-        // Block straddles the last channel: row by row, skipping rows >= M.
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = m0 + MC_ROW(r);
-          if (m < e.M) {
-            const int c = g * e.M + m;
-            float v = acc[i][j][r];
-            if (has_scale) v *= a.scale[c];
-            if (has_shift) v += a.shift[c];
-            const int yo = ybase + c * e.y_cstride;
-            if (has_res) v += e.residual[yo];
-            yout[yo] = apply_act(v, e.act, e.slope);
-          }
-        }
-      }
-    }
-  }
-#undef MC_ROW
-#undef MC_LOADF
-#undef MC_STORE_ROWS
+  finish_tile<BM, BN, TM, TN, LDK * 4, OCC == 8 ? 2 : 1>(a, batch.slices, sub_index, kslice, g, mt, nt, wm0, wn0, acc,
+                                       reinterpret_cast<const char*>(&As[0][0][0][BK]),
+                                       reinterpret_cast<int*>(&As[0][0][0][0]), scale_ptr, shift_ptr, yout);
 }
+
+#include "igemm_split.h"
 
 // Split-K tail for a launch whose output channels belong to two blobs (two
 // sibling layers computed together): v = act((sum over slices, in slice order) *
@@ -850,8 +846,8 @@ struct TileConfig {
   int bm, bn;
   int ks;  // 16-row K tiles per stage
   const char* name;
-  void (*kernel[4])(const IgemmBatch);  // indexed by mode; [3] (pixel-quad pointwise) may be null
-  void (*one_sub[4])(const IgemmBatch);  // the same for launches of one sub-problem, or null
+  void (*kernel[3])(const IgemmBatch);   // indexed by mode
+  void (*one_sub[3])(const IgemmBatch);  // the same for launches of one sub-problem, or null
 };
 
 const TileConfig kConfigs[] = {
@@ -866,10 +862,9 @@ const TileConfig kConfigs[] = {
       igemm_kernel<64, 128, 2, 2, 5, kModePointwise, 1>}},
     {64, 64, 1, "igemm_f32_64x64",
      {igemm_kernel<64, 64, 2, 2, 8, kModeMasks, 1>, igemm_kernel<64, 64, 2, 2, 8, kModeOneMask, 1>,
-      igemm_kernel<64, 64, 2, 2, 8, kModePointwise, 1>, igemm_kernel<64, 64, 2, 2, 8, kModePointwiseQuad, 1>},
+      igemm_kernel<64, 64, 2, 2, 8, kModePointwise, 1>},
      {igemm_kernel<64, 64, 2, 2, 8, kModeMasks, 1, true>, igemm_kernel<64, 64, 2, 2, 8, kModeOneMask, 1, true>,
-      igemm_kernel<64, 64, 2, 2, 8, kModePointwise, 1, true>,
-      igemm_kernel<64, 64, 2, 2, 8, kModePointwiseQuad, 1, true>}},
+      igemm_kernel<64, 64, 2, 2, 8, kModePointwise, 1, true>}},
     {32, 128, 1, "igemm_f32_32x128",
      {igemm_kernel<32, 128, 1, 4, 4, kModeMasks, 1>, igemm_kernel<32, 128, 1, 4, 4, kModeOneMask, 1>,
       igemm_kernel<32, 128, 1, 4, 4, kModePointwise, 1>}},
@@ -904,7 +899,8 @@ struct SubProblem {
   int* tap_dev = nullptr;    // tap_dh followed by tap_dw
   int4* ktab_dev = nullptr;
   int* wk_off_dev = nullptr;
-  float* wt_dev = nullptr;
+  float* wt_dev = nullptr;           // fp32: plans of the fp32 kernel and of the per-pixel kernel
+  uint16_t* wt_split_dev = nullptr;  // bf16 terms: plans of the split kernel
 };
 
 }  // namespace
@@ -929,6 +925,11 @@ struct mcConvPlan {
   // 3x3 stride 1: the Winograd path, and who decides (-1 = by size, 0 = never, 1 = always)
   WinogradState* winograd = nullptr;
   int winograd_mode = -1;
+  // fp32 products from three bf16 terms per operand (igemm_split.h): Convolution.
+  // Deconvolution and InnerProduct keep the fp32 instruction: a
+  // generator's last layers reach sums of 1e6 and more in front of a tanh when its
+  // statistics are not normalised, where the last bit of a sum decides the sign of an output.
+  bool split = false;
   std::vector<SubProblem> subs;
 };
 
@@ -992,6 +993,50 @@ int pick_split(const mcConvPlan* plan, long blocks, int KT) {
   return std::max(s, 1);
 }
 
+// Tile and K slices of one launch: the pair with the smallest estimated time.  A CU works
+// through ceil(workgroups / 256) of them, each K tiles long plus a fixed part
+// (prologue, epilogue); slicing K spreads a launch of few tiles over the chip and
+// costs the partial sums' way to memory and back.  stage_us and fixed_us of a tile are its
+// measured throughput on full launches (kConfigs).
+struct LaunchChoice {
+  int config, slices;
+};
+LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const SubProblem*>& live, int num) {
+  LaunchChoice best = {3, 1};
+  double best_us = 1e30;
+  for (int c = 0; c < kNumSplitConfigs; ++c) {
+    const SplitConfig& cfg = kSplitConfigs[c];
+    if (plan->forced_config >= 0 ? c != plan->forced_config : cfg.stage_us == 0.f) continue;
+    if (plan->forced_config < 0 && cfg.bm == 32 && plan->M > 32) continue;
+    const long mt = ceil_div(plan->M, cfg.bm);
+    long blocks = 0, tile_stages = 0;
+    int min_kt = 1 << 30;
+      for (const SubProblem* s : live) {
+      const long b = mt * ceil_div((long)num * s->Hq * s->Wq, cfg.bn) * plan->geom.group;
+      blocks += b;
+      tile_stages += b * (s->Kpad / BK);
+      if (s->Kpad > 0) min_kt = std::min(min_kt, s->Kpad / (BK * cfg.ks));
+    }
+      if (min_kt == (1 << 30)) min_kt = 1;
+    const double stages = blocks > 0 ? static_cast<double>(tile_stages) / blocks : 0.;  // of a tile, on average
+    int first = 1, last = std::max(1, std::min(24, min_kt * cfg.ks / 4));
+    if (plan->forced_split >= 1) first = last = std::min(plan->forced_split, std::max(min_kt, 1));
+    for (int s = first; s <= last; ++s) {
+      const double rounds = ceil_div(blocks * s, kNumCu);
+      // few wavefronts to hide the gather's latency (and that of the tap table, if any)
+      const double alone = plan->subs[0].pointwise ? (rounds < 2 ? 1.2 : rounds < 3 ? 1.1 : 1.)
+                                                   : (rounds < 2 ? 2. : rounds < 3 ? 1.4 : rounds < 4 ? 1.15 : 1.);
+      double us = rounds * (stages / s * cfg.stage_us * alone + cfg.fixed_us);
+      if (s > 1) us += 1.2 + 0.26 * s + 2e-6 * blocks * s * cfg.bm * cfg.bn;
+      if (us < best_us) {
+        best_us = us;
+        best = {c, s};
+      }
+    }
+  }
+  return best;
+}
+
 int free_sub(SubProblem& s) {
   if (s.ktab_dev) (void)hipFree(s.ktab_dev);
   if (s.tap_dev) (void)hipFree(s.tap_dev);
@@ -1001,6 +1046,8 @@ int free_sub(SubProblem& s) {
   s.ktab_dev = nullptr;
   s.wk_off_dev = nullptr;
   s.wt_dev = nullptr;
+  if (s.wt_split_dev) (void)hipFree(s.wt_split_dev);
+  s.wt_split_dev = nullptr;
   return 0;
 }
 
@@ -1009,9 +1056,8 @@ inline int floordiv(int a, int b) { return (a >= 0) ? a / b : -((-a + b - 1) / b
 
 }  // namespace
 
-extern "C" {
-
-int mcConvPlanCreate(const mcConvGeom* gp, mcConvPlan** out) {
+namespace {
+int create_plan(const mcConvGeom* gp, bool inner_product, mcConvPlan** out) {
   MC_REQUIRE(gp && out, "mcConvPlanCreate: null argument");
   const mcConvGeom& g = *gp;
   MC_REQUIRE(g.channels_in > 0 && g.channels_out > 0 && g.height_in > 0 && g.width_in > 0,
@@ -1056,6 +1102,7 @@ int mcConvPlanCreate(const mcConvGeom* gp, mcConvPlan** out) {
     return 0;
   }
   plan->Mpad = ceil_div(plan->M, 128) * 128;
+  plan->split = !g.transposed && !inner_product;
   const int HW = g.height_in * g.width_in;
   const int khkw = g.kernel_h * g.kernel_w;
 
@@ -1172,7 +1219,9 @@ int mcConvPlanCreate(const mcConvGeom* gp, mcConvPlan** out) {
       e = hipMalloc(&s.ktab_dev, sizeof(int4) * s.Kpad);
       if (e == hipSuccess) e = hipMalloc(&s.wk_off_dev, sizeof(int) * s.K);
       if (e == hipSuccess) e = hipMalloc(&s.tap_dev, sizeof(int) * taps.size());
-      if (e == hipSuccess) e = hipMalloc(&s.wt_dev, wt_bytes);
+      if (e == hipSuccess && (!plan->split || plan->M <= kThinM)) e = hipMalloc(&s.wt_dev, wt_bytes);
+      if (e == hipSuccess && plan->split)
+        e = hipMalloc(&s.wt_split_dev, wt_bytes / sizeof(float) * 3 * sizeof(uint16_t));
       if (e == hipSuccess)
         e = hipMemcpy(s.ktab_dev, s.ktab.data(), sizeof(int4) * s.Kpad, hipMemcpyHostToDevice);
       if (e == hipSuccess)
@@ -1193,10 +1242,16 @@ int mcConvPlanCreate(const mcConvGeom* gp, mcConvPlan** out) {
   return 0;
 }
 
+}  // namespace
+
+extern "C" {
+
+int mcConvPlanCreate(const mcConvGeom* gp, mcConvPlan** out) { return create_plan(gp, false, out); }
+
 int mcInnerProductPlanCreate(int K, int N, int transpose, mcConvPlan** out) {
   MC_REQUIRE(K > 0 && N > 0 && out, "mcInnerProductPlanCreate: bad argument");
   mcConvGeom g = {K, 1, 1, N, 1, 1, 1, 1, 0, 0, 1, 1, 1, 0};
-  if (mcConvPlanCreate(&g, out)) return -1;
+  if (create_plan(&g, true, out)) return -1;
   if (transpose) {
     // weights are K x N: element (k, m) sits at k*N + m
     mcConvPlan* plan = *out;
@@ -1243,10 +1298,18 @@ int mcConvPlanSetWeights(mcConvPlan* plan, const float* weights, void* stream) {
   for (auto& s : plan->subs) {
     if (s.Kpad == 0) continue;
     const long total = (long)plan->geom.group * s.Kpad * plan->Mpad;
-    pack_weights_kernel<<<ew_blocks(total, 256), 256, 0, st>>>(
-        weights, s.wt_dev, s.wk_off_dev, plan->geom.group, s.K, s.Kpad, plan->M, plan->Mpad,
-        plan->wm_stride, plan->wg_stride);
-    MC_LAUNCH_CHECK();
+    if (s.wt_dev) {
+      pack_weights_kernel<<<ew_blocks(total, 256), 256, 0, st>>>(
+          weights, s.wt_dev, s.wk_off_dev, plan->geom.group, s.K, s.Kpad, plan->M, plan->Mpad,
+          plan->wm_stride, plan->wg_stride);
+      MC_LAUNCH_CHECK();
+    }
+    if (s.wt_split_dev) {
+      pack_split_kernel<<<ew_blocks(total, 256), 256, 0, st>>>(
+          weights, s.wt_split_dev, s.wk_off_dev, plan->geom.group, s.K, s.Kpad, plan->M, plan->Mpad,
+          plan->wm_stride, plan->wg_stride);
+      MC_LAUNCH_CHECK();
+    }
   }
   if (plan->winograd && winograd_set_weights(plan->winograd, weights, st)) return -1;
   return 0;
@@ -1349,24 +1412,21 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
     max_pixels = std::max(max_pixels, pixels);
   }
   if (live.empty()) return 0;
-  const TileConfig& cfg = kConfigs[pick_config(plan, max_pixels)];
-  const int MT = ceil_div(plan->M, cfg.bm);
+  const LaunchChoice choice =
+      plan->split ? pick_split_launch(plan, live, num) : LaunchChoice{pick_config(plan, max_pixels), 0};
+  const int bm = plan->split ? kSplitConfigs[choice.config].bm : kConfigs[choice.config].bm;
+  const int bn = plan->split ? kSplitConfigs[choice.config].bn : kConfigs[choice.config].bn;
+  const int stage_kt = plan->split ? kSplitConfigs[choice.config].ks : kConfigs[choice.config].ks;
+  const int MT = ceil_div(plan->M, bm);
   long total_blocks = 0;
   int min_kt = 1 << 30;
   bool pointwise = !plan->force_general, one_mask = !plan->force_general;
-  bool quad_ok = true;  // stride-1 pointwise on planes of a multiple of four pixels, K a multiple of 16
   double flops = 0.;
   for (const SubProblem* s : live) {
     const long pixels = (long)num * s->Hq * s->Wq;
-    total_blocks += (long)MT * ceil_div(pixels, cfg.bn) * g.group;
-    if (s->Kpad > 0) min_kt = std::min(min_kt, s->Kpad / (BK * cfg.ks));
+    total_blocks += (long)MT * ceil_div(pixels, bn) * g.group;
+    if (s->Kpad > 0) min_kt = std::min(min_kt, s->Kpad / (BK * stage_kt));
     pointwise = pointwise && s->pointwise;
-    quad_ok = quad_ok && s->q_sh == 1 && s->q_sw == 1 && s->Hq == g.height_in && s->Wq == g.width_in &&
-              (s->Hq * s->Wq) % 4 == 0 && s->K % 16 == 0 && s->in_oh == 0 && s->in_ow == 0 &&
-              // ... and pixel p of an image is element p of its top plane as well (the kernel
-              // then needs no row / column of a pixel on either side)
-              s->out_sh == 1 && s->out_sw == 1 && s->out_oh == 0 && s->out_ow == 0 && s->Hq == plan->Ho &&
-              s->Wq == plan->Wo;
     one_mask = one_mask && s->one_mask;
     flops += 2.0 * pixels * plan->M * g.group * s->K;
   }
@@ -1377,7 +1437,7 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
   // side by side
   // Two tops are told apart by the pass that sums the slices, so such a launch
   // has at least two of them (a slice past the last K tile adds zeros).
-  int slices = thin ? 1 : pick_split(plan, total_blocks, min_kt);
+  int slices = thin ? 1 : plan->split ? choice.slices : pick_split(plan, total_blocks, min_kt);
   if (top_second && slices == 1) slices = 2;
   const long slice_stride = (out_count + 3) / 4 * 4;
   float* ws = nullptr;
@@ -1392,11 +1452,11 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
       long most = 0;
       for (size_t i = 0; i < nsub; ++i)
         most = std::max<long>(most, (long)MT * ceil_div((long)num * live[first + i]->Hq * live[first + i]->Wq,
-                                                         cfg.bn));
+                                                         bn));
       partial_tiles = std::max<long>(partial_tiles, most * g.group * (long)nsub);
     }
     MC_REQUIRE(partial_tiles < (1L << 31), "mcConvForward: grid too large");
-    if (stream_workspace(st, sizeof(float) * partial_tiles * cfg.bm * cfg.bn * slices, &ws)) return -1;
+    if (stream_workspace(st, sizeof(float) * partial_tiles * bm * bn * slices, &ws)) return -1;
     if (stream_counters(st, static_cast<size_t>(partial_tiles), &counters)) return -1;
   } else if (slices > 1) {
     if (stream_workspace(st, sizeof(float) * slice_stride * slices, &ws)) return -1;
@@ -1408,7 +1468,8 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
     MC_HIP(hipEventCreate(&tl.start));
     MC_HIP(hipEventCreate(&tl.stop));
     tl.flops = tl.issued = flops;
-    tl.name = thin ? "thin_f32" : cfg.name;
+    tl.name = thin ? "thin_f32"
+                   : plan->split ? kSplitConfigs[choice.config].name : kConfigs[choice.config].name;
     MC_HIP(hipEventRecord(tl.start, st));
   }
   for (size_t first = 0; first < live.size(); first += kMaxSubs) {
@@ -1422,6 +1483,7 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
       const long pixels = (long)num * s.Hq * s.Wq;
       IgemmArgs& a = batch.sub[i];
       a.wt = s.wt_dev;
+      a.wt_split = s.wt_split_dev;
       a.y = top;
       a.ktab = s.ktab_dev;
       a.tap_dh = s.tap_dev;
@@ -1469,7 +1531,7 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
       a.out_oh = s.out_oh;
       a.out_ow = s.out_ow;
       a.MT = MT;
-      a.NT = ceil_div(pixels, cfg.bn);
+      a.NT = ceil_div(pixels, bn);
       make_fast_div(a.MT, (unsigned long long)a.MT * a.NT + 1, &a.div_mt_mul, &a.div_mt_shift);
       a.act = ep ? ep->activation : MC_ACT_NONE;
       a.slope = ep ? ep->negative_slope : 0.f;
@@ -1478,7 +1540,7 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
       max_blocks = std::max(max_blocks, blocks);
       // every slice gets the same number of K tiles; slices past the last tile
       // of a short sub-problem write zeros
-      a.kt_per_split = ceil_div(std::max(s.Kpad / (BK * cfg.ks), 1), slices);
+      a.kt_per_split = ceil_div(std::max(s.Kpad / (BK * stage_kt), 1), slices);
       a.split_stride = 0;
       a.partial = nullptr;
       a.counters = nullptr;
@@ -1503,18 +1565,21 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
       dim3 grid(static_cast<unsigned>(max_blocks), g.group, nsub * slices);
       // A launch with less than one round of workgroups asks for enough LDS that
       // at most ceil(workgroups / CUs) of them fit a CU: the dispatcher then cannot
-      // fill some CUs to eight and leave others short (1-3 % on such launches).
+      // fill some CUs to the brim and leave others short (1-3 % on such launches).
       unsigned extra_lds = 0;
       const long wgs = max_blocks * g.group * nsub * slices;
-      if (wgs < 8L * kNumCu) {
-        const int limit = std::max<long>(3, ceil_div(wgs, static_cast<long>(kNumCu)));
-        const long stat = 2L * cfg.ks * (cfg.bm + cfg.bn) * LDK * 4;
+      const int per_cu = plan->split ? kSplitConfigs[choice.config].occ : 8;
+      if (wgs < static_cast<long>(per_cu) * kNumCu) {
+        const int limit = std::max<long>(plan->split ? 1 : 3, ceil_div(wgs, static_cast<long>(kNumCu)));
+        const long stat = plan->split ? 2L * stage_kt * (bm + bn) * 6 * BK + 8 * bm
+                                      : 2L * stage_kt * (bm + bn) * LDK * 4;
         const long want = (160L * 1024 / limit) / 1024 * 1024;
-        if (limit < 8 && want > stat) extra_lds = static_cast<unsigned>(want - stat);
+        if (limit < per_cu && want > stat) extra_lds = static_cast<unsigned>(want - stat);
       }
-      int mode = pointwise ? kModePointwise : (one_mask ? kModeOneMask : kModeMasks);
-      if (pointwise && quad_ok && cfg.kernel[kModePointwiseQuad]) mode = kModePointwiseQuad;
-      auto kernel = (nsub == 1 && cfg.one_sub[mode]) ? cfg.one_sub[mode] : cfg.kernel[mode];
+      const int mode = pointwise ? kModePointwise : (one_mask ? kModeOneMask : kModeMasks);
+      auto kernel = plan->split ? kSplitConfigs[choice.config].kernel[mode] : kConfigs[choice.config].kernel[mode];
+      if (nsub == 1 && !plan->split && kConfigs[choice.config].one_sub[mode])
+        kernel = kConfigs[choice.config].one_sub[mode];
       kernel<<<grid, 256, extra_lds, st>>>(batch);
     }
     MC_LAUNCH_CHECK();
@@ -1666,6 +1731,7 @@ const char* mcConvPlanKernelName(const mcConvPlan* plan, int num) {
   if (!plan || plan->subs.empty()) return "";
   if (takes_winograd(plan, num)) return "winograd_f32";
   if (use_thin(plan, num)) return "thin_f32";
+  if (plan->split) return kSplitConfigs[pick_split_launch(plan, {&plan->subs[0]}, num).config].name;
   const auto& s = plan->subs[0];
   return kConfigs[pick_config(plan, (long)num * s.Hq * s.Wq)].name;
 }

@@ -1,0 +1,91 @@
+"""Convolution on the bf16 matrix pipe with three terms per operand: the same fp32 result.
+
+Against a float64 convolution.  Any order of fp32 additions of the K products stays within
+K * 2^-24 * sum |x w| per element; the terms left out of the split are below 2^-26 of a
+product, so the bound holds with one more unit per product, which is far more than either needs.
+The norm of the error is held to half of sqrt(K) * 2^-24 of the result's for operands of
+random sign (fp32 products, one at a time, give 0.6 to 0.8 of it).
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def K(gpu_mode):
+    from minicaffe import kernels
+    return kernels
+
+
+def conv64(x, w, s, p):
+    return torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), stride=s, padding=p).numpy()
+
+
+def run(K, x, w, s, p, config, slices):
+    n, cin, h, wd = x.shape
+    plan = K.ConvPlan(K.conv_geom(cin, h, wd, w.shape[0], w.shape[2], s, p))
+    plan.force_config(config)
+    plan.force_split(slices)
+    xd, wt = torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda()
+    ho, wo = plan.output_shape()
+    y = torch.full((n, w.shape[0], ho, wo), float("nan"), device="cuda")
+    plan.set_weights(wt.data_ptr())
+    plan.forward(n, xd.data_ptr(), y.data_ptr())
+    torch.cuda.synchronize()
+    return y.cpu().numpy()
+
+
+@pytest.mark.parametrize("config", [0, 1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("case", [
+    # cin, size, cout, kernel, stride, pad, batch, slices: one K tile to many, odd and even numbers of
+    # stages, rows and pixels on both sides of a tile's edge, all three ways to gather
+    (1, 5, 3, 1, 1, 0, 1, 1), (16, 8, 32, 1, 1, 0, 1, 1), (17, 8, 33, 1, 1, 0, 2, 1), (33, 9, 65, 1, 2, 0, 3, 1),
+    (96, 16, 127, 1, 1, 0, 1, 1), (160, 11, 129, 1, 1, 0, 3, 3), (4, 16, 64, 3, 1, 1, 1, 1), (12, 13, 130, 3, 2, 1, 2, 2),
+    (3, 23, 24, 7, 2, 3, 2, 1), (5, 17, 40, 3, 1, 0, 3, 1)])
+def test_error_against_float64(K, case, config):
+    cin, size, cout, k, s, p, n, slices = case
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((n, cin, size, size)).astype(np.float32)
+    w = rng.standard_normal((cout, cin, k, k)).astype(np.float32)
+    want = conv64(x, w, s, p)
+    err = np.abs(run(K, x, w, s, p, config, slices) - want)
+    kk = cin * k * k
+    assert np.all(err <= (kk + 1) * 2.0 ** -24 * conv64(np.abs(x), np.abs(w), s, p) + 1e-30)
+    assert np.linalg.norm(err) <= 0.5 * max(2.0, np.sqrt(kk)) * 2.0 ** -24 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("config", [0, 1, 2, 4, 7])
+@pytest.mark.parametrize("geom", [(32, 1, 0), (8, 3, 1), (3, 5, 2)])
+def test_values_the_split_cannot_hold(K, config, geom):
+    """Infinities, NaN and magnitudes that round past bf16's largest value, in the bottom and in
+    the filters: the same special values as an fp32 convolution, finite ones where it is finite."""
+    cin, k, p = geom
+    rng = np.random.default_rng(6)
+    x = rng.standard_normal((3, cin, 12, 12)).astype(np.float32)
+    w = (0.1 * rng.standard_normal((70, cin, k, k))).astype(np.float32)
+    for i, v in enumerate((np.inf, -np.inf, np.nan, 3.4e38, -3.4e38, 1e-30)):
+        x[i % 3, (5 * i) % cin, (3 * i) % 12, (7 * i + 2) % 12] = v
+    big = x.copy()
+    w[11, 1, 0, 0], w[40, 0, k - 1, 0], w[69, cin - 1, 0, k - 1] = np.inf, np.nan, -np.inf
+    with np.errstate(all="ignore"):
+        # (padded by hand: the zeros of the padding are multiplied like any others, as im2col does)
+        xp = torch.nn.functional.pad(torch.from_numpy(x), (p, p, p, p))
+        want = torch.nn.functional.conv2d(xp, torch.from_numpy(w)).numpy()
+        got = run(K, x, w, 1, p, config, 1)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.where(np.isinf(got), np.sign(got), 0), np.where(np.isinf(want), np.sign(want), 0))
+    ok = np.isfinite(want)
+    assert ok.any() and not ok.all()
+    scale = np.maximum(np.abs(want[ok]), 1.0)
+    assert np.all(np.abs(got[ok].astype(np.float64) - want[ok]) <= 2 * cin * k * k * 2.0 ** -24 * 10 * scale)
+
+
+def test_filters_above_the_largest_bf16(K):
+    """A filter value that rounding to bf16 would carry to infinity is kept."""
+    x = np.full((1, 32, 4, 4), 0.01, np.float32)
+    w = np.zeros((64, 32, 1, 1), np.float32)
+    w[:, 3] = np.float32(3.4e38)
+    want = conv64(x, w, 1, 0)
+    assert np.allclose(run(K, x, w, 1, 0, 3, 1), want, rtol=3 * 2.0 ** -24, atol=0)
