@@ -68,6 +68,10 @@ struct IgemmArgs {
   unsigned div_hw_mul, div_hw_shift;  // p / HqWq  as multiply-high and shift (shift 32: divisor 1)
   unsigned div_w_mul, div_w_shift;    // rem / Wq
   unsigned div_mt_mul, div_mt_shift;  // logical tile / MT
+  // taps of a Convolution without the table: row / taps, tap / columns (times 2^-16), and the
+  // bytes between neighbouring taps
+  unsigned div_taps_mul, div_taps_shift;
+  int div_kw_mul, tap_h4, tap_w4;
   unsigned y_bytes, c_bytes;          // top blob and per-channel vector extents (descriptors)
   int H, W;           // bottom height / width
   int q_sh, q_sw;     // bottom origin of pixel (qh,qw): qh*q_sh + in_oh
@@ -1510,6 +1514,12 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
       // columns up to the end of the last pixel tile are divided (and then ignored)
       make_fast_div(a.HqWq, pixels + 512, &a.div_hw_mul, &a.div_hw_shift);
       make_fast_div(a.Wq, (unsigned long long)a.HqWq + 1, &a.div_w_mul, &a.div_w_shift);
+      if (s.one_mask) {
+        make_fast_div(a.n_dh * a.n_dw, (unsigned long long)s.Kpad / 4 + 1, &a.div_taps_mul, &a.div_taps_shift);
+        a.div_kw_mul = 65536 / a.n_dw + 1;  // exact for the at most 31 taps
+        a.tap_h4 = g.dilation_h * g.width_in * 4;
+        a.tap_w4 = g.dilation_w * 4;
+      }
       a.y_bytes = static_cast<unsigned>(out_count * 4);
       a.c_bytes = static_cast<unsigned>(g.channels_out) * 4;
       a.H = g.height_in;

@@ -176,6 +176,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
       reinterpret_cast<const char*>(a.wt_split) + static_cast<size_t>(g) * (a.Kpad / BK) * wt_kt_bytes;
   const unsigned x_cbytes = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(a.x_cstride) * 4);
   const int kmax = a.K - 1;
+  const int n_taps = a.n_dh * a.n_dw, quads = a.K / 4;  // (kModeOneMask: K is a multiple of 4)
+  int quad_tap[(BE + 3) / 4];
+  unsigned quad_off[(BE + 3) / 4];
 
   // two sets: tile t waits in set t % 2
   u32x4 areg[2][KS][A_VEC];
@@ -205,12 +208,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
       /* padding rows re-read the last channel; their filter rows are zero */                \
       breg[set][ks][e] = MC_LOADF(xres, xvoff, static_cast<unsigned>(min(krow + (e), kmax)) * x_cbytes); \
     } else if constexpr (MODE == kModeOneMask) {                                             \
-      /* four rows from a multiple of four: four channels at one tap */                      \
-      const unsigned pb = __builtin_amdgcn_ubfe(row_bad, a.ktab[krow + (e) / 4 * 4].w, 1);   \
-      breg[set][ks][e] = MC_LOADF(xres, (pb << 31) | xvoff, a.ktab[krow + (e)].x);           \
+      const unsigned pb = __builtin_amdgcn_ubfe(row_bad, quad_tap[(e) / 4], 1);              \
+      breg[set][ks][e] = MC_LOADF(xres, (pb << 31) | xvoff, quad_off[(e) / 4] + (e) % 4 * x_cbytes); \
     } else {                                                                                 \
       const int4 tap = a.ktab[krow + (e)];                                                   \
       MC_GATHER1(breg[set][ks][e], tap);                                                     \
+    }                                                                                        \
+  }
+  // One mask: rows 4 q .. 4 q + 3 are four channels (block q / taps) at tap q % taps.
+  // Computed on the scalar unit: a table would be fetched through the scalar cache, whose
+  // answers arrive in no order among the LDS reads, and the first product of every stage would
+  // wait for it.  Padding rows get tap 31, which is outside the image for every pixel.
+#define MC_QUADS(kt16)                                                                       \
+  if constexpr (MODE == kModeOneMask) {                                                      \
+    _Pragma("unroll") for (int q = 0; q < BE / 4; ++q) {                                     \
+      const int row = __builtin_amdgcn_readfirstlane((kt16)*BK + prow * BE) / 4 + q;         \
+      const int block = fast_div(row, a.div_taps_mul, a.div_taps_shift);                     \
+      const int tap = row - block * n_taps;                                                  \
+      const int ti = (tap * a.div_kw_mul) >> 16;                                             \
+      const unsigned off = static_cast<unsigned>(block) * 4u * x_cbytes +                    \
+                           static_cast<unsigned>(ti * a.tap_h4 + (tap - ti * a.n_dw) * a.tap_w4); \
+      quad_tap[q] = row < quads ? tap : 31;                                                  \
+      quad_off[q] = row < quads ? off : 0u;                                                  \
     }                                                                                        \
   }
 #define MC_STORE_A(set, ks, i)                                                               \
@@ -232,6 +251,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 #define MC_LOAD_TILES(set, kt)                                                               \
   _Pragma("unroll") for (int ks = 0; ks < KS; ++ks) {                                        \
     _Pragma("unroll") for (int i = 0; i < A_VEC; ++i) MC_LOAD_A(set, ks, (kt)*KS + ks, i)    \
+    MC_QUADS((kt)*KS + ks)                                                                   \
     _Pragma("unroll") for (int e = 0; e < BE; ++e) MC_LOAD_B(set, ks, (kt)*KS + ks, e)       \
   }
 #define MC_STORE_TILES(set)                                                                  \
@@ -278,6 +298,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
         accs[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(                                \
             av[s / P == 2 || s / P == 3 ? 1 : (s / P == 5 ? 2 : 0)][i],                      \
             bv[s / P == 1 || s / P == 3 ? 1 : (s / P == 4 ? 2 : 0)][j], accs[i][j], 0, 0, 0);\
+      if (load && s == 0) {                                                                  \
+        MC_QUADS(kt16)                                                                       \
+      }                                                                                      \
       if (P > 1 && s == 0) MC_READ_B(buf, ks, 1)                                             \
       if (P > 1 && s == 1) MC_READ_A(buf, ks, 1)                                             \
       if (s == P) MC_READ_B(buf, ks, 2)                                                      \
@@ -379,6 +402,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 #undef MC_GATHER1
 #undef MC_LOAD_A
 #undef MC_LOAD_B
+#undef MC_QUADS
 #undef MC_STORE_A
 #undef MC_SPLIT_B
 #undef MC_STORE_B
