@@ -51,6 +51,16 @@ real_t* CaffeBlobData(BlobHandle blob) {
   }
 }
 
+int CaffeBlobSetData(BlobHandle blob, const real_t* data, int count) {
+  API_BEGIN();
+  CHECK(blob != nullptr && data != nullptr) << "CaffeBlobSetData: null argument";
+  caffe::Blob* b = static_cast<caffe::Blob*>(blob);
+  CHECK_EQ(count, b->count()) << "CaffeBlobSetData: the blob has another number of elements";
+  CHECK(b->data()) << "blob '" << b->name() << "' has no memory";
+  b->data()->Assign(data, sizeof(real_t) * static_cast<size_t>(count));
+  API_END();
+}
+
 int CaffeBlobReshape(BlobHandle blob, int shape_size, int* shape) {
   API_BEGIN();
   CHECK(blob != nullptr && shape_size >= 0 && (shape != nullptr || shape_size == 0))

@@ -96,6 +96,8 @@ class SyncedMemory {
   void* mutable_cpu_data();
   const void* gpu_data();
   void* mutable_gpu_data();
+  // Fills the first `bytes` bytes from `src` (which may be the host copy itself).
+  void Assign(const void* src, size_t bytes);
   SyncedHead head() const { return head_; }
   size_t size() const { return size_; }
   // Bumped by every mutable_* access: cheap "did the contents possibly change".

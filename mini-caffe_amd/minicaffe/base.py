@@ -41,6 +41,7 @@ def _declare_c_api(lib):
     for fn in ("CaffeBlobNum", "CaffeBlobChannels", "CaffeBlobHeight", "CaffeBlobWidth",
                "CaffeBlobCount", "CaffeBlobData"):
         getattr(lib, fn).argtypes = [BlobHandle]
+    lib.CaffeBlobSetData.argtypes = [BlobHandle, ctypes.c_void_p, ctypes.c_int]
     lib.CaffeBlobReshape.argtypes = [BlobHandle, ctypes.c_int, _int_p]
     lib.CaffeBlobShape.argtypes = [BlobHandle, _int_p, ctypes.POINTER(_int_p)]
     lib.CaffeNetCreate.argtypes = [ctypes.c_char_p, ctypes.c_char_p, ctypes.POINTER(NetHandle)]

@@ -2,6 +2,8 @@
 import ctypes
 from collections import defaultdict
 
+import numpy as np
+
 from .base import LIB, BlobHandle, NetHandle, c_str, check_call, py_str
 from .blob import Blob
 
@@ -73,5 +75,8 @@ class Net(object):
         for k, v in kwargs.items():
             blob = self.get_blob(k)
             blob.reshape(*v.shape)
-            blob.data[...] = v
+            if v.dtype == np.float32 and v.flags.c_contiguous and 0 < v.size == blob.count:
+                check_call(LIB.CaffeBlobSetData(blob.handle, v.ctypes.data, v.size))
+            else:
+                blob.data[...] = v
         check_call(LIB.CaffeNetForward(self.handle))
