@@ -523,7 +523,7 @@ struct SplitConfig {
     igemm_split_kernel<BM, BN, WM, WN, OCC, kModeOneMask, KS>,                \
     igemm_split_kernel<BM, BN, WM, WN, OCC, kModePointwise, KS>}}
 const SplitConfig kSplitConfigs[] = {
-    MC_CONFIG(128, 128, 2, 2, 2, 1, 0.68f, 3.3f, "igemm_f32_128x128"),
+    MC_CONFIG(128, 128, 2, 2, 2, 1, 0.56f, 3.3f, "igemm_f32_128x128"),
     MC_CONFIG(128, 64, 2, 2, 3, 1, 0.363f, 0.9f, "igemm_f32_128x64"),
     MC_CONFIG(64, 128, 2, 2, 3, 1, 0.377f, 1.2f, "igemm_f32_64x128"),
     MC_CONFIG(64, 64, 2, 2, 4, 1, 0.f, 0.f, "igemm_f32_64x64"),
