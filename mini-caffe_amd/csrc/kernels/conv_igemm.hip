@@ -1001,7 +1001,7 @@ int pick_split(const mcConvPlan* plan, long blocks, int KT) {
 // through ceil(workgroups / 256) of them, each K tiles long plus a fixed part
 // (prologue, epilogue); slicing K spreads a launch of few tiles over the chip and
 // costs the partial sums' way to memory and back.  stage_us and fixed_us of a tile are its
-// measured throughput on full launches (kConfigs).
+// measured throughput on full launches (kSplitConfigs).
 struct LaunchChoice {
   int config, slices;
 };

@@ -36,6 +36,11 @@ __device__ __forceinline__ float bf16_value(unsigned bits) { return __builtin_bi
 // bf16 products overlap with it: six VALU instructions per product cost nothing measurable
 // with four wavefronts per SIMD.
 //
+// What bounds it: the matrix pipe at the clock the chip holds under this load (about 1.7 GHz):
+// 1024 -> 1024 1x1 over 16 384 pixels 171 us, 201 TFLOP/s, 68 % of the cycles (fp32 products: 261
+// us); small K on large maps: HBM (64 -> 256 1x1 on 64 x 56x56: 77 -> 61 us, 4.2 TB/s); single
+// images: the latency of a slice's loads (512 -> 512 3x3 on one 7x7 map: 21.8 -> 16.4 us).
+//
 // Values the split cannot hold (infinities, NaN, magnitudes that round past bf16's
 // largest) leave an accumulator non-finite.  A wavefront that finds one after the K loop
 // forms its block again with fp32 products straight from memory (below).

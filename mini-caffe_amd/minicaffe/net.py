@@ -75,7 +75,8 @@ class Net(object):
         for k, v in kwargs.items():
             blob = self.get_blob(k)
             blob.reshape(*v.shape)
-            if v.dtype == np.float32 and v.flags.c_contiguous and 0 < v.size == blob.count:
+            if (isinstance(v, np.ndarray) and v.dtype == np.float32 and v.flags.c_contiguous and
+                    0 < v.size == blob.count):
                 check_call(LIB.CaffeBlobSetData(blob.handle, v.ctypes.data, v.size))
             else:
                 blob.data[...] = v
