@@ -531,10 +531,12 @@ const SplitConfig kSplitConfigs[] = {
     MC_CONFIG(128, 128, 2, 2, 2, 1, 0.56f, 3.3f, "igemm_f32_128x128"),
     MC_CONFIG(128, 64, 2, 2, 3, 1, 0.363f, 0.9f, "igemm_f32_128x64"),
     MC_CONFIG(64, 128, 2, 2, 3, 1, 0.377f, 1.2f, "igemm_f32_64x128"),
-    MC_CONFIG(64, 64, 2, 2, 4, 1, 0.f, 0.f, "igemm_f32_64x64"),
+    // (3, 5 and 6, taken on request only, are other places' tiles: each instance is many
+    // seconds of compilation, and none of their own shapes was the best of any layer measured)
+    MC_CONFIG(64, 64, 2, 2, 3, 2, 0.f, 0.f, "igemm_f32_64x64x32"),
     MC_CONFIG(32, 128, 1, 4, 4, 1, 0.215f, 0.6f, "igemm_f32_32x128"),
-    MC_CONFIG(32, 256, 1, 4, 2, 1, 0.f, 0.f, "igemm_f32_32x256"),
-    MC_CONFIG(64, 256, 1, 4, 2, 1, 0.f, 0.f, "igemm_f32_64x256"),
+    MC_CONFIG(32, 128, 1, 4, 4, 1, 0.f, 0.f, "igemm_f32_32x128"),
+    MC_CONFIG(64, 128, 2, 2, 3, 1, 0.f, 0.f, "igemm_f32_64x128"),
     MC_CONFIG(64, 64, 2, 2, 3, 2, 0.21f, 0.8f, "igemm_f32_64x64x32"),
 };
 #undef MC_CONFIG
