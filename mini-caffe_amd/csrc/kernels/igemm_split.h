@@ -2,11 +2,21 @@
 // (inside its namespace), which defines the argument block, the gather modes and the
 // common end of a tile.
 
-// x = h + m + l in bf16 (round to nearest even at every step): 8 + 8 + 8 significand
-// bits, so the three terms hold every bit of a float whose magnitude neither reaches
-// bf16's largest value nor comes near the smallest normal float.  Two values at a time:
-// each returned word holds the terms of a (low half) and b (high half).
+// Both operands are multiplied by 2^24 before they are split, the sums by 2^-48 after the K
+// loop.  bf16 has float's exponents, so the third term of a value, 2^-17 of it and less, would
+// fall below bf16's smallest normal number for values under 2^-109 and be lost; times
+// 2^24 every float, down to the smallest subnormal, keeps all its bits in normal
+// bf16 numbers.  The price is at the other end: operands from 2^103 and sums from 2^80 on are not
+// finite in the accumulators and take the fp32 products below.
+constexpr float kSplitScale = 0x1p24f;
+constexpr float kSplitUnscale = 0x1p-48f;
+
+// x * 2^24 = h + m + l in bf16 (round to nearest even at every step): 8 + 8 + 8 significand
+// bits hold every bit of a float.  Two values at a time: each returned word holds the
+// terms of a (low half) and b (high half).
 __device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsigned& m, unsigned& l) {
+  a *= kSplitScale;
+  b *= kSplitScale;
   const bf16x2 hv = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
   h = __builtin_bit_cast(unsigned, hv);
   a -= __builtin_bit_cast(float, h << 16);
@@ -20,6 +30,16 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsign
 }
 
 __device__ __forceinline__ float bf16_value(unsigned bits) { return __builtin_bit_cast(float, bits << 16); }
+
+// First term of a filter value whose terms cannot hold it: a NaN, which sends every sum it
+// enters to the fp32 products.  The other two terms are the upper and the lower half of the value.
+constexpr unsigned kNotSplit = 0x7FFFu;
+
+// The filter value of packed terms, exactly.
+__device__ __forceinline__ float filter_value(unsigned h, unsigned m, unsigned l) {
+  if (h == kNotSplit) return __builtin_bit_cast(float, m << 16 | l);
+  return ((bf16_value(h) + bf16_value(m)) + bf16_value(l)) * (1.f / kSplitScale);
+}
 
 // The products run on the bf16 matrix pipe, which multiplies sixteen times as many values per
 // cycle as the fp32 one, without giving up fp32 accuracy: both operands are split
@@ -41,8 +61,8 @@ __device__ __forceinline__ float bf16_value(unsigned bits) { return __builtin_bi
 // us); small K on large maps: HBM (64 -> 256 1x1 on 64 x 56x56: 77 -> 61 us, 4.2 TB/s); single
 // images: the latency of a slice's loads (512 -> 512 3x3 on one 7x7 map: 21.8 -> 16.4 us).
 //
-// Values the split cannot hold (infinities, NaN, magnitudes that round past bf16's
-// largest) leave an accumulator non-finite.  A wavefront that finds one after the K loop
+// Values the split cannot hold (infinities, NaN, magnitudes of 2^103 and above) and sums of
+// 2^80 and above leave an accumulator non-finite.  A wavefront that finds one after the K loop
 // forms its block again with fp32 products straight from memory (below).
 //
 // OCC = wavefronts per SIMD the register allocation must leave room for.
@@ -424,15 +444,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        acc[i][j][r] += accs[i][j][r];
+        acc[i][j][r] = (acc[i][j][r] + accs[i][j][r]) * kSplitUnscale;
         probe = __builtin_fmaf(acc[i][j][r], 0.f, probe);
       }
   if (__any(probe != 0.f)) {
-    // Rare: an operand is infinite, NaN or above bf16's largest value, or a sum
-    // overflows.  The wavefront forms its blocks again from fp32 values: its lanes read
-    // their filter rows (h + m + l is the filter value) and the bottom straight from
-    // memory, eight K rows each, and multiply with the fp32 instruction.  No LDS and no
-    // barrier: the other wavefronts do not take part.
+    // Rare: an operand is infinite, NaN or of 2^103 and above, or a sum is of 2^80 and
+    // above.  The wavefront forms its blocks again from fp32 values: its lanes read
+    // their filter rows and the bottom straight from memory, eight K rows each, and
+    // multiply with the fp32 instruction.  No LDS and no barrier: the other wavefronts
+    // do not take part.
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       unsigned voff, rbad, cbad;
@@ -460,7 +480,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
                                        : ((rbad >> tap.y) | (cbad >> tap.z)) & 1u;
               off = bad ? kNoElement : voff + static_cast<unsigned>(tap.x);
             }
-            const float wv = bf16_value(w[e]) + bf16_value(w[plane + e]) + bf16_value(w[2 * plane + e]);
+            const float wv = filter_value(w[e], w[plane + e], w[2 * plane + e]);
             sum = __builtin_amdgcn_mfma_f32_32x32x2f32(wv, MC_LOADF(xres, off, 0), sum, 0, 0, 0);
           }
         }
@@ -477,9 +497,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 
 // Packed filter wt[g][kt][plane][kl / 8][m][kl % 8] = the bf16 terms of
 // w[g*wg_stride + wk_off[k] + m*wm_stride] with k = kt*16 + kl, zero where k >= K or
-// m >= M.  The terms always add up to the weight: where it is not finite the
-// first term is the weight and the others are zero, and where rounding to bf16 would
-// overflow the first term is cut off instead.
+// m >= M.  filter_value() of the terms is the weight, for every weight.
 __global__ void pack_split_kernel(const float* __restrict__ w, uint16_t* __restrict__ wt,
                                   const int* __restrict__ wk_off, int G, int K, int Kpad, int M, int Mpad, int wm_stride, int wg_stride) {
   const long total = (long)G * Kpad * Mpad;
@@ -496,18 +514,16 @@ __global__ void pack_split_kernel(const float* __restrict__ w, uint16_t* __restr
     float v = 0.f;
     if (k < K && m < M) v = w[(long)g * wg_stride + wk_off[k] + (long)m * wm_stride];
     const unsigned bits = __builtin_bit_cast(unsigned, v);
-    const bool special = (bits & 0x7F800000u) == 0x7F800000u;
-    float h = static_cast<float>(static_cast<__bf16>(v));
-    if (!special && __builtin_isinf(h)) h = __builtin_bit_cast(float, bits & 0xFFFF0000u);
-    const float r = special ? 0.f : v - h;
-    const float mid = static_cast<float>(static_cast<__bf16>(r));
-    const float low = r - mid;
+    v *= kSplitScale;
+    const float h = static_cast<float>(static_cast<__bf16>(v));
+    const float mid = static_cast<float>(static_cast<__bf16>(v - h));
+    const float low = static_cast<float>(static_cast<__bf16>(v - h - mid));
+    const bool fits = __builtin_isfinite(h);
     uint16_t* out = wt + (((static_cast<size_t>(g) * KT + kt) * 6 + kl / 8) * Mpad + m) * 8 + kl % 8;
     const size_t plane = static_cast<size_t>(Mpad) * 16;
-    out[0] = static_cast<uint16_t>(__builtin_bit_cast(unsigned, h) >> 16);
-    out[plane] = static_cast<uint16_t>(__builtin_bit_cast(unsigned, mid) >> 16);
-    out[2 * plane] =
-        static_cast<uint16_t>(__builtin_bit_cast(unsigned, static_cast<float>(static_cast<__bf16>(low))) >> 16);
+    out[0] = static_cast<uint16_t>(fits ? __builtin_bit_cast(unsigned, h) >> 16 : kNotSplit);
+    out[plane] = static_cast<uint16_t>(fits ? __builtin_bit_cast(unsigned, mid) >> 16 : bits >> 16);
+    out[2 * plane] = static_cast<uint16_t>(fits ? __builtin_bit_cast(unsigned, low) >> 16 : bits & 0xFFFFu);
   }
 }
 

@@ -89,3 +89,20 @@ def test_filters_above_the_largest_bf16(K):
     w[:, 3] = np.float32(3.4e38)
     want = conv64(x, w, 1, 0)
     assert np.allclose(run(K, x, w, 1, 0, 3, 1), want, rtol=3 * 2.0 ** -24, atol=0)
+
+
+@pytest.mark.parametrize("config", [0, 1, 2, 4, 7])
+@pytest.mark.parametrize("sx,sw", [
+    (1e-36, 1.0), (1.0, 1e-36), (1e-37, 10.0), (1e-40, 1e10), (1e10, 1e-40), (1e-18, 1e-18), (1e-42, 1e20), (1e20, 1e-42),
+    (1e30, 1e-30), (1e36, 1e-30), (1e-36, 1e36), (1e20, 1e10), (1e12, 1e12), (1e25, 1.0)])
+@pytest.mark.parametrize("geom", [(1, 1, 0), (37, 1, 0), (12, 3, 1)])
+def test_all_magnitudes_keep_their_bits(K, geom, sx, sw, config):
+    """Operands from subnormal numbers to 1e36: no term of a split may leave bf16's range.  The bound of
+    fp32 products, K * 2^-24 * sum |x w|, and one unit of the smallest float per product."""
+    cin, k, p = geom
+    rng = np.random.default_rng(8)
+    x = (sx * rng.uniform(0.5, 1, (2, cin, 9, 9)) * rng.choice([-1, 1], (2, cin, 9, 9))).astype(np.float32)
+    w = (sw * rng.uniform(0.5, 1, (40, cin, k, k)) * rng.choice([-1, 1], (40, cin, k, k))).astype(np.float32)
+    kk = cin * k * k
+    err = np.abs(run(K, x, w, 1, p, config, 1) - conv64(x, w, 1, p))
+    assert np.all(err <= (kk + 1) * (2.0 ** -24 * conv64(np.abs(x), np.abs(w), 1, p) + 2.0 ** -149))
