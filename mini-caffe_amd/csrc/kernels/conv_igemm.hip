@@ -41,7 +41,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-constexpr int kModeMasks = 0, kModeOneMask = 1, kModePointwise = 2;
+constexpr int kModeMasks = 0, kModeOneMask = 1, kModePointwise = 2, kModePointwiseQuad = 3;
 // Buffer descriptor word 3 for raw dword access on gfx9-family CDNA parts
 // (32-bit data format, no swizzle, offsets checked against num_records).
 constexpr int kBufferFlags = 0x00020000;
@@ -51,8 +51,10 @@ constexpr unsigned kNoElement = 0x80000000u;
 
 struct IgemmArgs {
   const float* __restrict__ x;
-  const float* __restrict__ wt;           // packed filter, fp32 (pack_weights_kernel), or null
-  const uint16_t* __restrict__ wt_split;  // packed filter, three bf16 planes, or null
+  union {  // packed filter
+    const float* __restrict__ wt;           // fp32 (pack_weights_kernel)
+    const uint16_t* __restrict__ wt_split;  // the split kernel's, three bf16 planes (pack_split_kernel)
+  };
   float* __restrict__ y;
   const int4* __restrict__ ktab;  // [Kpad] {byte offset, row-tap index, column-tap index, 0}
   const int* __restrict__ tap_dh;  // bottom row offset of row-tap index b
@@ -68,10 +70,6 @@ struct IgemmArgs {
   unsigned div_hw_mul, div_hw_shift;  // p / HqWq  as multiply-high and shift (shift 32: divisor 1)
   unsigned div_w_mul, div_w_shift;    // rem / Wq
   unsigned div_mt_mul, div_mt_shift;  // logical tile / MT
-  // taps of a Convolution without the table: row / taps, tap / columns (times 2^-16), and the
-  // bytes between neighbouring taps
-  unsigned div_taps_mul, div_taps_shift;
-  int div_kw_mul, tap_h4, tap_w4;
   unsigned y_bytes, c_bytes;          // top blob and per-channel vector extents (descriptors)
   int H, W;           // bottom height / width
   int q_sh, q_sw;     // bottom origin of pixel (qh,qw): qh*q_sh + in_oh
@@ -104,8 +102,13 @@ struct IgemmArgs {
 // in one launch: blockIdx.z = sub-problem * slices + K slice.
 constexpr int kMaxSubs = 4;
 struct IgemmBatch {
-  IgemmArgs sub[kMaxSubs];
+  // (first: every cache line of the arguments that a launch touches is a trip to memory)
   int slices;
+  // The split kernel's taps, which go without the table: row / taps, tap / columns (times
+  // 2^-16), and the bytes between neighbouring taps.
+  int div_kw_mul, tap_h4, tap_w4;
+  unsigned div_taps_mul, div_taps_shift;
+  IgemmArgs sub[kMaxSubs];
 };
 
 __device__ __forceinline__ float f4at(const float4& v, int e) {
@@ -125,200 +128,6 @@ __device__ __forceinline__ float apply_act(float v, int act, float slope) {
   }
 }
 
-// What follows the K loop: the sum over K slices inside the launch, then the layer's
-// epilogue and the store.  `factors`: (scale, shift) of tile row r at factors + r * FPITCH
-// bytes, in LDS; `arrived`: one int of LDS that no wavefront needs any more after a barrier.
-template <int BM, int BN, int TM, int TN, int FPITCH, int AHEAD>
-__device__ __forceinline__ void finish_tile(const IgemmArgs& a, int slices, int sub_index, int kslice, int g,
-                                            int mt, int nt, int wm0, int wn0, acc16 (&acc)[TM][TN],
-                                            const char* factors, int* arrived, const float* scale_ptr,
-                                            const float* shift_ptr, float* __restrict__ yout) {
-  const int tid = threadIdx.x;
-  const int l32 = tid & 31, lhi = (tid & 63) >> 5;
-  // What the epilogue reads from the argument block is fetched here in one batch:
-  // fetched where it is first used, the fields cost the wavefront four or five
-  // scalar-memory round trips after the last MFMA, one after the other.  (Before the K
-  // loop they would not fit the scalar registers the loop needs.)
-  struct {
-    int* counters;
-    const float* residual;
-    unsigned y_bytes, div_hw_mul, div_hw_shift, div_w_mul, div_w_shift;
-    int y_cstride, y_nstride, Wo, out_sh, out_sw, out_oh, out_ow, M, P, HqWq, Wq, act;
-    float slope;
-  } e = {a.counters, a.residual, a.y_bytes, a.div_hw_mul, a.div_hw_shift, a.div_w_mul, a.div_w_shift,
-         a.y_cstride, a.y_nstride, a.Wo, a.out_sh, a.out_sw, a.out_oh, a.out_ow, a.M, a.P, a.HqWq, a.Wq,
-         a.act, a.slope};
-  asm volatile("" ::"s"(e.counters), "s"(e.residual), "s"(e.y_bytes), "s"(e.div_hw_mul), "s"(e.div_hw_shift),
-               "s"(e.div_w_mul), "s"(e.div_w_shift), "s"(e.y_cstride), "s"(e.y_nstride), "s"(e.Wo),
-               "s"(e.out_sh), "s"(e.out_sw), "s"(e.out_oh), "s"(e.out_ow), "s"(e.M), "s"(e.P), "s"(e.HqWq),
-               "s"(e.Wq), "s"(e.act), "s"(e.slope));
-
-  if (e.counters != nullptr) {
-    // K slices summed here: see IgemmArgs::partial.  The partial sums and the
-    // counter are accessed with device-scope atomic operations only (relaxed
-    // stores and loads that go past the per-XCD L2, which is not coherent with
-    // the other seven), so no cache write-back or invalidation is needed: a
-    // workgroup waits until its own stores have completed and then counts.
-    // What this rests on is particular to the parts it is built for: a store with
-    // device scope (sc1) is written through to the memory side, where all XCDs meet,
-    // and vmcnt counts it down only when that write has been acknowledged; an
-    // atomic on the counter issued after the wait is therefore ordered behind the
-    // partial sums at the one place every later device-scope load reads from.  The
-    // language's memory model promises none of this for relaxed accesses.
-#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx942__) && !defined(__gfx950__)
-#error "the in-launch sum of K slices relies on gfx942 / gfx950 device-scope write-through"
-#endif
-    const int tile_id = (sub_index * gridDim.y + g) * gridDim.x + blockIdx.x;
-    constexpr int kRegs = TM * TN * 16;  // accumulator registers per thread
-    float* mine = a.partial +
-                  (static_cast<size_t>(kslice) * a.partial_tiles + tile_id) * (kRegs * 256) + tid;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          __hip_atomic_store(mine + ((i * TN + j) * 16 + r) * 256, acc[i][j][r], __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's partial sums have arrived
-    __syncthreads();  // ... every thread's, and every wave is done with the tiles in LDS
-    if (tid == 0)
-      arrived[0] = __hip_atomic_fetch_add(&e.counters[tile_id], 1, __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (arrived[0] != slices - 1) return;  // uniform over the workgroup
-    // the next launch on this stream starts from zero
-    if (tid == 0)
-      __hip_atomic_store(&e.counters[tile_id], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // Slices are added in slice order, the loads of AHEAD of them together (as many as the
-    // registers hold): one at a time each costs a round trip to memory (2048 -> 512 1x1
-    // on one 7x7 map, eight slices: 12.9 us, four at a time 11.8).
-    const float* part = a.partial + static_cast<size_t>(tile_id) * (kRegs * 256) + tid;
-    const size_t slice_elems = static_cast<size_t>(a.partial_tiles) * (kRegs * 256);
-#pragma unroll
-    for (int r = 0; r < kRegs; ++r)
-      acc[r / 16 / TN][r / 16 % TN][r % 16] =
-          __hip_atomic_load(part + r * 256, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int z = 1; z < slices; z += AHEAD) {
-      float v[AHEAD][kRegs];
-#pragma unroll
-      for (int u = 0; u < AHEAD; ++u) {
-        // (a slice past the last one is read as the last one and not added)
-        const float* from = part + min(z + u, slices - 1) * slice_elems;
-#pragma unroll
-        for (int r = 0; r < kRegs; ++r)
-          v[u][r] = __hip_atomic_load(from + r * 256, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-#pragma unroll
-      for (int u = 0; u < AHEAD; ++u)
-        if (z + u < slices) {
-#pragma unroll
-          for (int r = 0; r < kRegs; ++r) acc[r / 16 / TN][r / 16 % TN][r % 16] += v[u][r];
-        }
-    }
-  }
-
-  // Epilogue.  Accumulator register r of lane l holds row 8*(r/4)+4*(l/32)+r%4,
-  // column l%32 of its 32x32 block; a half-wave therefore stores 32 consecutive
-  // pixels of one output channel.  Like the K loop it addresses through buffer
-  // descriptors: one VGPR offset per lane (bit 31 set for a column past the last
-  // pixel, which drops its stores), the row as a scalar offset.  Per-channel
-  // factors and residual values are fetched eight rows at a time, all loads of
-  // a batch issued before the first use.
-  const bool has_scale = scale_ptr != nullptr;
-  const bool has_shift = shift_ptr != nullptr;
-  const bool has_res = e.residual != nullptr;
-  const __amdgpu_buffer_rsrc_t yres =
-      __builtin_amdgcn_make_buffer_rsrc(yout, 0, e.y_bytes, kBufferFlags);
-  const __amdgpu_buffer_rsrc_t rres = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(e.residual), 0, has_res ? e.y_bytes : 0, kBufferFlags);
-  // 0: none, 1: ReLU (max with 0), 2: leaky ReLU, 3: TanH / Sigmoid
-  const int act_mode = e.act == MC_ACT_NONE ? 0
-                       : e.act == MC_ACT_RELU ? (e.slope == 0.f ? 1 : 2)
-                                              : 3;
-  const unsigned cs4 = static_cast<unsigned>(e.y_cstride) * 4;
-#define MC_ROW(r) (8 * ((r) / 4) + ((r) % 4))
-#define MC_LOADF(res, voff, soff) \
-  __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(res, voff, soff, 0))
-#define MC_STORE_ROWS(EXPR)                                                                  \
-  _Pragma("unroll") for (int q = 0; q < 8; ++q) {                                            \
-    const float v = acc[i][j][half * 8 + q];                                                 \
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, (EXPR)), yres, y_voff,\
-                                          MC_ROW(half * 8 + q) * cs4, 0);                    \
-  }
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int p = nt * BN + wn0 + j * 32 + l32;
-    const int n = fast_div(p, e.div_hw_mul, e.div_hw_shift);
-    const int rem = p - n * e.HqWq;
-    int ybase;
-    const int qh = fast_div(rem, e.div_w_mul, e.div_w_shift);
-    const int qw = rem - qh * e.Wq;
-    ybase = n * e.y_nstride + (qh * e.out_sh + e.out_oh) * e.Wo + qw * e.out_sw + e.out_ow;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int mblock = mt * BM + wm0 + i * 32;  // wave-uniform
-      const int m0 = mblock + 4 * lhi;
-      if (mblock + 32 <= e.M) {
-        // All 32 rows are real channels.
-        const unsigned c0 = g * e.M + m0;
-        const unsigned y_voff =
-            p < e.P ? static_cast<unsigned>(ybase + c0 * e.y_cstride) * 4 : kNoElement;
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          if (has_scale | has_shift) {
-            float sc[8], sh[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-              const int lrow = wm0 + i * 32 + 4 * lhi + MC_ROW(half * 8 + q);
-              const float2 f = *reinterpret_cast<const float2*>(factors + lrow * FPITCH);
-              sc[q] = f.x;
-              sh[q] = f.y;
-            }
-#pragma unroll
-            for (int q = 0; q < 8; ++q)
-              acc[i][j][half * 8 + q] = acc[i][j][half * 8 + q] * sc[q] + sh[q];
-          }
-          if (has_res) {
-            float rs[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) rs[q] = MC_LOADF(rres, y_voff, MC_ROW(half * 8 + q) * cs4);
-#pragma unroll
-            for (int q = 0; q < 8; ++q) acc[i][j][half * 8 + q] += rs[q];
-          }
-          if (act_mode == 0) {
-            MC_STORE_ROWS(v)
-          } else if (act_mode == 1) {
-            MC_STORE_ROWS(fmaxf(v, 0.f))
-          } else if (act_mode == 2) {
-            MC_STORE_ROWS(v > 0.f ? v : v * e.slope)
-          } else {
-            MC_STORE_ROWS(apply_act(v, e.act, e.slope))
-          }
-        }
-      } else if (p < e.P) {
-        // Block straddles the last channel: row by row, skipping rows >= M.
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = m0 + MC_ROW(r);
-          if (m < e.M) {
-            const int c = g * e.M + m;
-            float v = acc[i][j][r];
-            if (has_scale) v *= a.scale[c];
-            if (has_shift) v += a.shift[c];
-            const int yo = ybase + c * e.y_cstride;
-            if (has_res) v += e.residual[yo];
-            yout[yo] = apply_act(v, e.act, e.slope);
-          }
-        }
-      }
-    }
-  }
-#undef MC_ROW
-#undef MC_LOADF
-#undef MC_STORE_ROWS
-}
-
 // OCC = wavefronts per SIMD the register allocation must leave room for.
 // MODE selects how the K loop finds and guards the elements it gathers:
 //   kModeMasks     tap table + one "outside the image" bit mask per tap row and
@@ -330,6 +139,11 @@ __device__ __forceinline__ void finish_tile(const IgemmArgs& a, int slices, int 
 //                  rows a thread gathers per step share one tap and one
 //                  validity test;
 //   kModePointwise no table and no mask, see below;
+//   kModePointwiseQuad  the same for stride 1 on planes of a multiple of four pixels with
+//                  K a multiple of 16 (64-pixel tile only): a thread fetches four
+//                  consecutive pixels of one channel with one 16-byte load instead of
+//                  one pixel of four channels with four loads, and transposes them on
+//                  the way into LDS (four 4-byte stores).  Same products, same order.
 // Pointwise: every row k of the gather is channel k of the bottom blob
 // at the thread's own pixel (1x1 kernel, no padding), so the K loop needs no
 // tap table and no bounds handling at all.
@@ -418,21 +232,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
   const int pj = tid % BN;
   const int prow = tid / BN;  // wave-uniform because BN >= 64
   // byte offset of the pixel's origin from the descriptor base (never negative)
-  constexpr bool PW = MODE == kModePointwise;
+  constexpr bool PW4 = MODE == kModePointwiseQuad;  // pointwise, stride 1: four pixels of a channel per load
+  constexpr bool PW = MODE == kModePointwise || PW4;
+  static_assert(!PW4 || (BN == 64 && KS == 1), "the pixel-quad gather is built for the 64-pixel tile");
   unsigned xvoff = PW ? kNoElement : 0u;
   unsigned row_bad = 0xFFFFFFFFu, col_bad = 0xFFFFFFFFu;
   {
-    const int p = nt * BN + pj;
+    // PW4: thread = (K row tid % 16, pixel quad tid / 16); the plane is a multiple of four
+    // pixels, so a quad never straddles two images
+    const int p = PW4 ? nt * BN + 4 * (tid >> 4) : nt * BN + pj;
     // (the divisions are prepared for every column of the last tile, also those past the
     // last pixel: the pointwise modes compute first and pick afterwards, without a branch)
     const int n = fast_div(p, a.div_hw_mul, a.div_hw_shift);
     const int rem = p - n * a.HqWq;
-    const int qh = fast_div(rem, a.div_w_mul, a.div_w_shift);
-    const int qw = rem - qh * a.Wq;
+    // (the pixel-quad mode runs only where pixel `rem` of the iteration grid is element
+    // `rem` of the bottom plane and of the top plane: no row and column needed)
+    const int qh = PW4 ? 0 : fast_div(rem, a.div_w_mul, a.div_w_shift);
+    const int qw = PW4 ? 0 : rem - qh * a.Wq;
     const int hi0 = qh * a.q_sh + a.in_oh;
     const int wi0 = qw * a.q_sw + a.in_ow;
-    const unsigned origin = static_cast<unsigned>(
-        ((n * a.x_nstride + g * a.x_gstride + hi0 * a.W + wi0) << 2) + a.pix_shift);
+    unsigned origin = static_cast<unsigned>(
+        ((n * a.x_nstride + g * a.x_gstride + (PW4 ? rem : hi0 * a.W + wi0)) << 2) + a.pix_shift);
+    if constexpr (PW4) origin += static_cast<unsigned>(tid & 15) * (static_cast<unsigned>(a.x_cstride) * 4u);
     if constexpr (PW) xvoff = p < a.P ? origin : kNoElement;
     if (!PW && p < a.P) {
       xvoff = origin;
@@ -478,8 +299,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
   const unsigned wt_kt_bytes = static_cast<unsigned>(a.Mpad) * BK * 4;
   const unsigned wt_g_bytes = static_cast<unsigned>(g) * (a.Kpad / BK) * wt_kt_bytes;
   // (said to be uniform: the compiler otherwise merges this load with the one inside the
-  // divergent branch above into a vector register, and every load of the K loop, whose
-  // scalar offset is a multiple of it, gets wrapped in a loop over lanes)
+  // divergent branch above into a vector register, and every pixel-quad load of the K
+  // loop, whose scalar offset is a multiple of it, gets wrapped in a loop over lanes)
   const unsigned x_cbytes = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(a.x_cstride) * 4);
   const int kmax = a.K - 1;
 
@@ -509,7 +330,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
     _Pragma("unroll") for (int i = 0; i < B_Q; ++i) {                                        \
       const int krow =                                                                       \
           __builtin_amdgcn_readfirstlane(kt16 * BK + (i * ROWS_PER_PASS + prow) * 4);        \
-      if constexpr (PW) {                                                                    \
+      if constexpr (PW4) {                                                                   \
+        /* K is a multiple of 16 here: no padding rows */                                    \
+        const u32x4 q4 = __builtin_amdgcn_raw_buffer_load_b128(                              \
+            xres, xvoff, static_cast<unsigned>(kt16 * BK) * x_cbytes, 0);                    \
+        breg[ks][i] = __builtin_bit_cast(float4, q4);                                        \
+      } else if constexpr (PW) {                                                             \
         /* padding rows re-read the last channel; their filter rows are zero */              \
         breg[ks][i].x = MC_LOADF(xres, xvoff, static_cast<unsigned>(min(krow, kmax)) * x_cbytes);\
         breg[ks][i].y =                                                                          \
@@ -546,8 +372,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
         *reinterpret_cast<float4*>(&As[buf][ks][f / QUADS][(f % QUADS) * 4]) = areg[ks][i];  \
     }                                                                                        \
     _Pragma("unroll") for (int i = 0; i < B_Q; ++i) {                                        \
-      *reinterpret_cast<float4*>(&Bs[buf][ks][pj][(i * ROWS_PER_PASS + prow) * 4]) =         \
-          breg[ks][i];                                                                       \
+      if constexpr (PW4) {                                                                   \
+        float* col = &Bs[buf][ks][4 * (tid >> 4)][tid & 15];                                 \
+        col[0] = breg[ks][i].x;                                                              \
+        col[LDK] = breg[ks][i].y;                                                            \
+        col[2 * LDK] = breg[ks][i].z;                                                        \
+        col[3 * LDK] = breg[ks][i].w;                                                        \
+      } else {                                                                               \
+        *reinterpret_cast<float4*>(&Bs[buf][ks][pj][(i * ROWS_PER_PASS + prow) * 4]) =       \
+            breg[ks][i];                                                                     \
+      }                                                                                      \
     }                                                                                        \
   }
   // One MFMA K step multiplies k-pairs; which two physical k rows form a pair
@@ -677,9 +511,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 #undef MC_COMPUTE
 #undef MC_INTERLEAVE
 
-  finish_tile<BM, BN, TM, TN, LDK * 4, OCC == 8 ? 2 : 1>(a, batch.slices, sub_index, kslice, g, mt, nt, wm0, wn0, acc,
-                                       reinterpret_cast<const char*>(&As[0][0][0][BK]),
-                                       reinterpret_cast<int*>(&As[0][0][0][0]), scale_ptr, shift_ptr, yout);
+#define MC_FACTORS(row) (&As[0][0][row][BK])
+#define MC_ARRIVED (reinterpret_cast<int*>(&As[0][0][0][0]))
+#define MC_SLICES batch.slices
+#define MC_AHEAD 1
+#define MC_PLAIN PW4
+#include "igemm_finish.h"
 }
 
 #include "igemm_split.h"
@@ -850,8 +687,8 @@ struct TileConfig {
   int bm, bn;
   int ks;  // 16-row K tiles per stage
   const char* name;
-  void (*kernel[3])(const IgemmBatch);   // indexed by mode
-  void (*one_sub[3])(const IgemmBatch);  // the same for launches of one sub-problem, or null
+  void (*kernel[4])(const IgemmBatch);   // indexed by mode; [3] (pixel-quad pointwise) may be null
+  void (*one_sub[4])(const IgemmBatch);  // the same for launches of one sub-problem, or null
 };
 
 const TileConfig kConfigs[] = {
@@ -866,9 +703,10 @@ const TileConfig kConfigs[] = {
       igemm_kernel<64, 128, 2, 2, 5, kModePointwise, 1>}},
     {64, 64, 1, "igemm_f32_64x64",
      {igemm_kernel<64, 64, 2, 2, 8, kModeMasks, 1>, igemm_kernel<64, 64, 2, 2, 8, kModeOneMask, 1>,
-      igemm_kernel<64, 64, 2, 2, 8, kModePointwise, 1>},
+      igemm_kernel<64, 64, 2, 2, 8, kModePointwise, 1>, igemm_kernel<64, 64, 2, 2, 8, kModePointwiseQuad, 1>},
      {igemm_kernel<64, 64, 2, 2, 8, kModeMasks, 1, true>, igemm_kernel<64, 64, 2, 2, 8, kModeOneMask, 1, true>,
-      igemm_kernel<64, 64, 2, 2, 8, kModePointwise, 1, true>}},
+      igemm_kernel<64, 64, 2, 2, 8, kModePointwise, 1, true>,
+      igemm_kernel<64, 64, 2, 2, 8, kModePointwiseQuad, 1, true>}},
     {32, 128, 1, "igemm_f32_32x128",
      {igemm_kernel<32, 128, 1, 4, 4, kModeMasks, 1>, igemm_kernel<32, 128, 1, 4, 4, kModeOneMask, 1>,
       igemm_kernel<32, 128, 1, 4, 4, kModePointwise, 1>}},
@@ -1015,13 +853,13 @@ LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const S
     const long mt = ceil_div(plan->M, cfg.bm);
     long blocks = 0, tile_stages = 0;
     int min_kt = 1 << 30;
-      for (const SubProblem* s : live) {
+    for (const SubProblem* s : live) {
       const long b = mt * ceil_div((long)num * s->Hq * s->Wq, cfg.bn) * plan->geom.group;
       blocks += b;
       tile_stages += b * (s->Kpad / BK);
       if (s->Kpad > 0) min_kt = std::min(min_kt, s->Kpad / (BK * cfg.ks));
     }
-      if (min_kt == (1 << 30)) min_kt = 1;
+    if (min_kt == (1 << 30)) min_kt = 1;
     const double stages = blocks > 0 ? static_cast<double>(tile_stages) / blocks : 0.;  // of a tile, on average
     int first = 1, last = std::max(1, std::min(24, min_kt * cfg.ks / 4));
     if (plan->forced_split >= 1) first = last = std::min(plan->forced_split, std::max(min_kt, 1));
@@ -1425,12 +1263,19 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
   long total_blocks = 0;
   int min_kt = 1 << 30;
   bool pointwise = !plan->force_general, one_mask = !plan->force_general;
+  bool quad_ok = true;  // stride-1 pointwise on planes of a multiple of four pixels, K a multiple of 16
   double flops = 0.;
   for (const SubProblem* s : live) {
     const long pixels = (long)num * s->Hq * s->Wq;
     total_blocks += (long)MT * ceil_div(pixels, bn) * g.group;
     if (s->Kpad > 0) min_kt = std::min(min_kt, s->Kpad / (BK * stage_kt));
     pointwise = pointwise && s->pointwise;
+    quad_ok = quad_ok && s->q_sh == 1 && s->q_sw == 1 && s->Hq == g.height_in && s->Wq == g.width_in &&
+              (s->Hq * s->Wq) % 4 == 0 && s->K % 16 == 0 && s->in_oh == 0 && s->in_ow == 0 &&
+              // ... and pixel p of an image is element p of its top plane as well (the kernel
+              // then needs no row / column of a pixel on either side)
+              s->out_sh == 1 && s->out_sw == 1 && s->out_oh == 0 && s->out_ow == 0 && s->Hq == plan->Ho &&
+              s->Wq == plan->Wo;
     one_mask = one_mask && s->one_mask;
     flops += 2.0 * pixels * plan->M * g.group * s->K;
   }
@@ -1486,8 +1331,11 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
       const SubProblem& s = *live[first + i];
       const long pixels = (long)num * s.Hq * s.Wq;
       IgemmArgs& a = batch.sub[i];
-      a.wt = s.wt_dev;
-      a.wt_split = s.wt_split_dev;
+      if (plan->split && !thin) {
+        a.wt_split = s.wt_split_dev;
+      } else {
+        a.wt = s.wt_dev;
+      }
       a.y = top;
       a.ktab = s.ktab_dev;
       a.tap_dh = s.tap_dev;
@@ -1514,11 +1362,12 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
       // columns up to the end of the last pixel tile are divided (and then ignored)
       make_fast_div(a.HqWq, pixels + 512, &a.div_hw_mul, &a.div_hw_shift);
       make_fast_div(a.Wq, (unsigned long long)a.HqWq + 1, &a.div_w_mul, &a.div_w_shift);
-      if (s.one_mask) {
-        make_fast_div(a.n_dh * a.n_dw, (unsigned long long)s.Kpad / 4 + 1, &a.div_taps_mul, &a.div_taps_shift);
-        a.div_kw_mul = 65536 / a.n_dw + 1;  // exact for the at most 31 taps
-        a.tap_h4 = g.dilation_h * g.width_in * 4;
-        a.tap_w4 = g.dilation_w * 4;
+      if (plan->split && s.one_mask) {
+        make_fast_div(a.n_dh * a.n_dw, (unsigned long long)s.Kpad / 4 + 1, &batch.div_taps_mul,
+                      &batch.div_taps_shift);
+        batch.div_kw_mul = 65536 / a.n_dw + 1;  // exact for the at most 31 taps
+        batch.tap_h4 = g.dilation_h * g.width_in * 4;
+        batch.tap_w4 = g.dilation_w * 4;
       }
       a.y_bytes = static_cast<unsigned>(out_count * 4);
       a.c_bytes = static_cast<unsigned>(g.channels_out) * 4;
@@ -1586,7 +1435,9 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
         const long want = (160L * 1024 / limit) / 1024 * 1024;
         if (limit < per_cu && want > stat) extra_lds = static_cast<unsigned>(want - stat);
       }
-      const int mode = pointwise ? kModePointwise : (one_mask ? kModeOneMask : kModeMasks);
+      int mode = pointwise ? kModePointwise : (one_mask ? kModeOneMask : kModeMasks);
+      if (pointwise && quad_ok && !plan->split && kConfigs[choice.config].kernel[kModePointwiseQuad])
+        mode = kModePointwiseQuad;
       auto kernel = plan->split ? kSplitConfigs[choice.config].kernel[mode] : kConfigs[choice.config].kernel[mode];
       if (nsub == 1 && !plan->split && kConfigs[choice.config].one_sub[mode])
         kernel = kConfigs[choice.config].one_sub[mode];

@@ -37,8 +37,26 @@ constexpr unsigned kNotSplit = 0x7FFFu;
 
 // The filter value of packed terms, exactly.
 __device__ __forceinline__ float filter_value(unsigned h, unsigned m, unsigned l) {
-  if (h == kNotSplit) return __builtin_bit_cast(float, m << 16 | l);
-  return ((bf16_value(h) + bf16_value(m)) + bf16_value(l)) * (1.f / kSplitScale);
+  const float sum = ((bf16_value(h) + bf16_value(m)) + bf16_value(l)) * (1.f / kSplitScale);
+  return h == kNotSplit ? __builtin_bit_cast(float, m << 16 | l) : sum;
+}
+
+// The end of a tile.  `arrived`: an int of LDS that no wavefront needs any more after a barrier.
+template <int BM, int BN, int TM, int TN>
+__device__ __forceinline__ void finish_split_tile(const IgemmArgs& a, int slices, int kslice, int g, int mt,
+                                                  int nt, int wm0, int wn0, acc16 (&acc)[TM][TN],
+                                                  const float2* factors, int* arrived_lds,
+                                                  const float* scale_ptr, const float* shift_ptr,
+                                                  float* __restrict__ yout) {
+  const int tid = threadIdx.x;
+  const int l32 = tid & 31, lhi = (tid & 63) >> 5;
+  constexpr int sub_index = 0;  // a Convolution is one sub-problem
+#define MC_FACTORS(row) (factors + (row))
+#define MC_ARRIVED arrived_lds
+#define MC_SLICES slices
+#define MC_AHEAD (TM * TN == 1 ? 4 : (TM * TN == 2 ? 2 : 1))
+#define MC_PLAIN false
+#include "igemm_finish.h"
 }
 
 // The products run on the bf16 matrix pipe, which multiplies sixteen times as many values per
@@ -248,11 +266,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
   if constexpr (MODE == kModeOneMask) {                                                      \
     _Pragma("unroll") for (int q = 0; q < BE / 4; ++q) {                                     \
       const int row = __builtin_amdgcn_readfirstlane((kt16)*BK + prow * BE) / 4 + q;         \
-      const int block = fast_div(row, a.div_taps_mul, a.div_taps_shift);                     \
+      const int block = fast_div(row, batch.div_taps_mul, batch.div_taps_shift);                     \
       const int tap = row - block * n_taps;                                                  \
-      const int ti = (tap * a.div_kw_mul) >> 16;                                             \
+      const int ti = (tap * batch.div_kw_mul) >> 16;                                             \
       const unsigned off = static_cast<unsigned>(block) * 4u * x_cbytes +                    \
-                           static_cast<unsigned>(ti * a.tap_h4 + (tap - ti * a.n_dw) * a.tap_w4); \
+                           static_cast<unsigned>(ti * batch.tap_h4 + (tap - ti * a.n_dw) * batch.tap_w4); \
       quad_tap[q] = row < quads ? tap : 31;                                                  \
       quad_off[q] = row < quads ? off : 0u;                                                  \
     }                                                                                        \
@@ -490,9 +508,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
   }
 #undef MC_LOADF
 
-  finish_tile<BM, BN, TM, TN, 8, TM * TN == 1 ? 4 : (TM * TN == 2 ? 2 : 1)>(
-      a, batch.slices, 0, kslice, g, mt, nt, wm0, wn0, acc, reinterpret_cast<const char*>(factors),
-      reinterpret_cast<int*>(&As[0][0][0][0][0][0]), scale_ptr, shift_ptr, yout);
+  finish_split_tile<BM, BN, TM, TN>(a, batch.slices, kslice, g, mt, nt, wm0, wn0, acc, factors,
+                                    reinterpret_cast<int*>(&As[0][0][0][0][0][0]), scale_ptr, shift_ptr, yout);
 }
 
 // Packed filter wt[g][kt][plane][kl / 8][m][kl % 8] = the bf16 terms of
