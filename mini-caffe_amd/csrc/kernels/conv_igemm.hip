@@ -767,10 +767,10 @@ struct mcConvPlan {
   // 3x3 stride 1: the Winograd path, and who decides (-1 = by size, 0 = never, 1 = always)
   WinogradState* winograd = nullptr;
   int winograd_mode = -1;
-  // fp32 products from three bf16 terms per operand (igemm_split.h): Convolution.
-  // Deconvolution and InnerProduct keep the fp32 instruction: a
-  // generator's last layers reach sums of 1e6 and more in front of a tanh when its
-  // statistics are not normalised, where the last bit of a sum decides the sign of an output.
+  // fp32 products from three bf16 terms per operand (igemm_split.h): Convolution, but for the
+  // shortest sums (short_sums).  Deconvolution and InnerProduct keep the fp32
+  // instruction: a generator's last layers reach sums of 1e6 and more in front of a tanh when
+  // its statistics are not normalised, where the last bit of a sum decides the sign of an output.
   bool split = false;
   std::vector<SubProblem> subs;
 };
@@ -879,6 +879,20 @@ LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const S
   return best;
 }
 
+// Sums too short for products from bf16 terms, which save nothing there and cost a longer
+// prologue: the fp32 kernel.  (By the layer alone, not by the batch: sums this short are not
+// sliced either, so an image's results stay the same in any batch.)  Measured, fp32 / split:
+// 3 -> 64 3x3 on 8 x 300x300 50 / 59 us, 32 -> 64 1x1 on 32 x 150x150 71 / 78, on one image 5.5 /
+// 6.7, 24 -> 48 on 8 x 56x56 6 / 9; with at most 32 output channels the split kernel leads
+// from 32 images of 56x56 on (16 -> 32: 8 / 7 us, 3 -> 32 3x3/2 on 32 x 300x300 35 / 28).
+// Pointwise 64 -> 64 on 56x56: 5.5 / 5.8 us on one image, 6.4 / 7.1 on 8, 23.6 / 24.3 on 64; with
+// more outputs or products split wins on large launches (64 -> 256 on 64 images 73 / 67).
+// Up to 8 products the error decides: the terms left out are up to 2^-24 of a
+// product, as much as rounding it, and a short sum does not round often enough to hide it.
+bool short_sums(int K, int M, bool pointwise) {
+  return K <= 8 || (M > 32 && (K <= 32 || (K <= 64 && M <= 64 && pointwise)));
+}
+
 int free_sub(SubProblem& s) {
   if (s.ktab_dev) (void)hipFree(s.ktab_dev);
   if (s.tap_dev) (void)hipFree(s.tap_dev);
@@ -944,7 +958,9 @@ int create_plan(const mcConvGeom* gp, bool inner_product, mcConvPlan** out) {
     return 0;
   }
   plan->Mpad = ceil_div(plan->M, 128) * 128;
-  plan->split = !g.transposed && !inner_product;
+  plan->split = !g.transposed && !inner_product &&
+                !short_sums(plan->Cin_g * g.kernel_h * g.kernel_w, plan->M,
+                            g.kernel_h == 1 && g.kernel_w == 1 && g.pad_h == 0 && g.pad_w == 0);
   const int HW = g.height_in * g.width_in;
   const int khkw = g.kernel_h * g.kernel_w;
 

@@ -64,7 +64,10 @@ __device__ __forceinline__ void finish_split_tile(const IgemmArgs& a, int slices
 // into three bf16 terms (split_pair; the filters once, when they are packed, the bottom's
 // values by the thread that brings them to LDS), every product of two terms is exact in
 // fp32, and of the nine products of x = h + m + l with w = h' + m' + l' the six largest are
-// summed (h h', h m', m h', m m', h l', l h'; the other three are below 2^-26 of the product).
+// summed (h h', h m', m h', m m', h l', l h'; the other three come to at most 2^-24 of the
+// product, 2^-27.4 on the average of random operands.  Summing m l' and l m' as well costs 10 to
+// 18 % of a launch; instead sums of a few products, which round too seldom to hide the
+// difference, stay with the fp32 kernel, see short_sums).
 // The sums run in fp32 accumulators: h h' in one, the five small ones in another, added once
 // after the K loop, so the large accumulator rounds once per sixteen K rows
 // where the fp32 instruction rounds sixteen times: the error against a 64-bit sum is

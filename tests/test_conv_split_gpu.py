@@ -1,8 +1,9 @@
 """Convolution on the bf16 matrix pipe with three terms per operand: the same fp32 result.
 
 Against a float64 convolution.  Any order of fp32 additions of the K products stays within
-K * 2^-24 * sum |x w| per element; the terms left out of the split are below 2^-26 of a
-product, so the bound holds with one more unit per product, which is far more than either needs.
+K * 2^-24 * sum |x w| per element; the terms left out of the split come to at most 2^-24 of a
+product (|m| <= 2^-8 and |l| <= 2^-17 of a value's power of two, so |m l' + l m'| <= 2^-24), which is
+the one more unit per product of the bound.  A single product (the fp32 kernel) is held to its one rounding.
 The norm of the error is held to half of sqrt(K) * 2^-24 of the result's for operands of
 random sign (fp32 products, one at a time, give 0.6 to 0.8 of it).
 """
@@ -106,3 +107,26 @@ def test_all_magnitudes_keep_their_bits(K, geom, sx, sw, config):
     kk = cin * k * k
     err = np.abs(run(K, x, w, 1, p, config, 1) - conv64(x, w, 1, p))
     assert np.all(err <= (kk + 1) * (2.0 ** -24 * conv64(np.abs(x), np.abs(w), 1, p) + 2.0 ** -149))
+
+
+def test_a_single_product_is_rounded_once(K):
+    """1x1 on one channel, for every combination of 512 x 512 significands: half a unit in the last place."""
+    rng = np.random.default_rng(9)
+    x = rng.uniform(1, 2, (1, 1, 16, 32)).astype(np.float32)
+    w = rng.uniform(1, 2, (512, 1, 1, 1)).astype(np.float32)
+    x[0, 0, 0, 0] = w[0] = 1.0038986          # where the left-out terms come to 2^-24.01
+    want = conv64(x, w, 1, 0)
+    err = np.abs(run(K, x, w, 1, 0, -1, 0) - want)
+    assert np.all(err <= 2.0 ** -24 * np.exp2(np.floor(np.log2(want))))
+
+
+@pytest.mark.parametrize("cin,k", [(2, 1), (5, 1), (8, 1), (9, 1), (33, 1), (4, 3), (64, 3), (576, 1)])
+def test_constant_operands(K, cin, k):
+    """Every product has the same left-out terms, so they do not average out over K."""
+    for seed in range(8):
+        rng = np.random.default_rng(seed)
+        xv, wv = (1.0038986, 1.0038986) if seed == 0 else rng.uniform(1, 2, 2)
+        x = np.full((2, cin, 20, 20), xv, np.float32)
+        w = np.full((20, cin, k, k), wv, np.float32)
+        want = conv64(x, w, 1, 0)
+        assert np.all(np.abs(run(K, x, w, 1, 0, -1, 0) - want) <= (cin * k * k + 1) * 2.0 ** -24 * want)
