@@ -835,6 +835,20 @@ int pick_split(const mcConvPlan* plan, long blocks, int KT) {
   return std::max(s, 1);
 }
 
+// Fewest chains of additions the products of an output are to be spread over: K slices times a
+// tile's own chains (SplitConfig::chains).  Rounding errors of sums of one sign grow with the
+// partial sums, so over s chains the error is s times smaller.  Over one chain each,
+// the split kernel's error is 0.32 to 0.48 of the fp32 kernel's; with at least half as many chains
+// as that kernel takes slices it stays below that kernel's in every launch (1024 -> 512 on 64 x
+// 7x7, non-negative operands, error of the norm: fp32 in five slices 1.0e-7, one chain 1.6e-7,
+// three 0.7e-7).
+int least_chains(const mcConvPlan* plan, const SubProblem& s, int num) {
+  const long pixels = (long)num * s.Hq * s.Wq;
+  const TileConfig& cfg = kConfigs[pick_config(plan, pixels)];
+  const long blocks = (long)ceil_div(plan->M, cfg.bm) * ceil_div(pixels, cfg.bn) * plan->geom.group;
+  return ceil_div(pick_split(plan, blocks, s.Kpad / (BK * cfg.ks)), 2);
+}
+
 // Tile and K slices of one launch: the pair with the smallest estimated time.  A CU works
 // through ceil(workgroups / 256) of them, each K tiles long plus a fixed part
 // (prologue, epilogue); slicing K spreads a launch of few tiles over the chip and
@@ -846,6 +860,8 @@ struct LaunchChoice {
 LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const SubProblem*>& live, int num) {
   LaunchChoice best = {3, 1};
   double best_us = 1e30;
+  int least = 1;
+  for (const SubProblem* s : live) least = std::max(least, least_chains(plan, *s, num));
   for (int c = 0; c < kNumSplitConfigs; ++c) {
     const SplitConfig& cfg = kSplitConfigs[c];
     if (plan->forced_config >= 0 ? c != plan->forced_config : cfg.stage_us == 0.f) continue;
@@ -861,7 +877,8 @@ LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const S
     }
     if (min_kt == (1 << 30)) min_kt = 1;
     const double stages = blocks > 0 ? static_cast<double>(tile_stages) / blocks : 0.;  // of a tile, on average
-    int first = 1, last = std::max(1, std::min(24, min_kt * cfg.ks / 4));
+    int first = std::min<int>(ceil_div(least, cfg.chains), min_kt);
+    int last = std::max(first, std::min(24, min_kt * cfg.ks / 4));
     if (plan->forced_split >= 1) first = last = std::min(plan->forced_split, std::max(min_kt, 1));
     for (int s = first; s <= last; ++s) {
       const double rounds = ceil_div(blocks * s, kNumCu);

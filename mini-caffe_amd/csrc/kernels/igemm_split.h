@@ -338,7 +338,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
     __builtin_amdgcn_sched_barrier(0);                                                       \
     _Pragma("unroll") for (int s = 0; s < 6 * P; ++s) {                                      \
       const int i = s % P / TN, j = s % P % TN;                                              \
-      if (s < P)                                                                             \
+      if (P == 1 && s == 0 && (buf) == 1)                                                    \
+        odd = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0][0], bv[0][0], odd, 0, 0, 0);     \
+      else if (s < P)                                                                        \
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0][i], bv[0][j], acc[i][j], 0, 0, 0); \
       else                                                                                   \
         accs[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(                                \
@@ -377,6 +379,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
   }
 
   acc16 acc[TM][TN], accs[TM][TN];  // h h', and the five small products
+  // A wavefront of one block has registers left for two chains of h h', of the even and of
+  // the odd stages: half the error of one chain, as two K slices would leave (kChains).
+  acc16 odd;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) odd[r] = 0.f;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -465,6 +472,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
+        if constexpr (TM * TN == 1) acc[i][j][r] += odd[r];
         acc[i][j][r] = (acc[i][j][r] + accs[i][j][r]) * kSplitUnscale;
         probe = __builtin_fmaf(acc[i][j][r], 0.f, probe);
       }
@@ -551,6 +559,7 @@ struct SplitConfig {
   int bm, bn;
   int ks;   // 16-row K tiles per stage
   int occ;  // workgroups per CU the kernel is built for
+  int chains;  // accumulators h h' alternates between
   // measured on full launches: a CU's time per 16-row K tile and per tile (prologue and
   // epilogue); 0 = taken on request only
   float stage_us, fixed_us;
@@ -559,7 +568,7 @@ struct SplitConfig {
 };
 
 #define MC_CONFIG(BM, BN, WM, WN, OCC, KS, STAGE, FIXED, NAME)                \
-  {BM, BN, KS, OCC, STAGE, FIXED, NAME,                                       \
+  {BM, BN, KS, OCC, BM / WM * (BN / WN) == 32 * 32 ? 2 : 1, STAGE, FIXED, NAME,                                       \
    {igemm_split_kernel<BM, BN, WM, WN, OCC, kModeMasks, KS>,                  \
     igemm_split_kernel<BM, BN, WM, WN, OCC, kModeOneMask, KS>,                \
     igemm_split_kernel<BM, BN, WM, WN, OCC, kModePointwise, KS>}}

@@ -130,3 +130,24 @@ def test_constant_operands(K, cin, k):
         w = np.full((20, cin, k, k), wv, np.float32)
         want = conv64(x, w, 1, 0)
         assert np.all(np.abs(run(K, x, w, 1, 0, -1, 0) - want) <= (cin * k * k + 1) * 2.0 ** -24 * want)
+
+
+@pytest.mark.parametrize("case", [(1024, 7, 512, 1, 64), (2048, 7, 512, 1, 64), (1024, 19, 256, 1, 8), (512, 10, 384, 3, 8)])
+def test_sums_of_one_sign(K, case):
+    """Operands of one sign, where a long chain of additions shows: n roundings of growing partial sums are
+    sqrt(n / 3) * 0.29 units of 2^-23, and s slices of n / s roundings divide that by s.  The fp32 kernel rounds once
+    per two products and takes 5 to 8 slices here; the error is held to what four such slices would leave."""
+    cin, size, cout, k, n = case
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.rand((n, cin, size, size), generator=g, device="cuda") + 1
+    w = torch.rand((cout, cin, k, k), generator=g, device="cuda") + 1
+    plan = K.ConvPlan(K.conv_geom(cin, size, size, cout, k, 2 if k == 3 else 1, k // 2))
+    plan.set_weights(w.data_ptr())
+    ho, wo = plan.output_shape()
+    y = torch.empty((n, cout, ho, wo), device="cuda")
+    plan.forward(n, x.data_ptr(), y.data_ptr())
+    torch.cuda.synchronize()
+    want = conv64(x[:2].cpu().numpy(), w.cpu().numpy(), 2 if k == 3 else 1, k // 2)
+    err = np.linalg.norm(y[:2].cpu().numpy() - want) / np.linalg.norm(want)
+    kk = cin * k * k
+    assert err <= 0.29 * 2.0 ** -23 * (np.sqrt(kk / 2 / 3) / 4 + 1)     # ... and the sum over slices and the store
