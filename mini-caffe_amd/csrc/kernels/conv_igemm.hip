@@ -1457,12 +1457,15 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
       dim3 grid(static_cast<unsigned>(max_blocks), g.group, nsub * slices);
       // A launch with less than one round of workgroups asks for enough LDS that
       // at most ceil(workgroups / CUs) of them fit a CU: the dispatcher then cannot
-      // fill some CUs to the brim and leave others short (1-3 % on such launches).
+      // fill some CUs to the brim and leave others short (1-3 % on such launches).  Never so
+      // much that a CU is closed to launches of other streams: a limit of one workgroup
+      // changes nothing on one stream (twelve ResNet-50 layers at batch 4: 149 us) and
+      // costs two streams 20 and three 33 % (91 and 84 us per chain, with a limit of one 108 and 111).
       unsigned extra_lds = 0;
       const long wgs = max_blocks * g.group * nsub * slices;
       const int per_cu = plan->split ? kSplitConfigs[choice.config].occ : 8;
       if (wgs < static_cast<long>(per_cu) * kNumCu) {
-        const int limit = std::max<long>(plan->split ? 1 : 3, ceil_div(wgs, static_cast<long>(kNumCu)));
+        const int limit = std::max<long>(3, ceil_div(wgs, static_cast<long>(kNumCu)));
         const long stat = plan->split ? 2L * stage_kt * (bm + bn) * 6 * BK + 8 * bm
                                       : 2L * stage_kt * (bm + bn) * LDK * 4;
         const long want = (160L * 1024 / limit) / 1024 * 1024;
