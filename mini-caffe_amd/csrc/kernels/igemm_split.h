@@ -251,7 +251,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
   {                                                                                          \
     const int krow = __builtin_amdgcn_readfirstlane((kt16)*BK + prow * BE);                  \
     if constexpr (PW) {                                                                      \
-      /* padding rows re-read the last channel; their filter rows are zero */                \
+      /* padding rows re-read the last channel; their filter rows are zero (an infinity there \
+         makes NaN of it, and the sum is formed again below, without padding rows) */        \
       breg[set][ks][e] = MC_LOADF(xres, xvoff, static_cast<unsigned>(min(krow + (e), kmax)) * x_cbytes); \
     } else if constexpr (MODE == kModeOneMask) {                                             \
       const unsigned pb = __builtin_amdgcn_ubfe(row_bad, quad_tap[(e) / 4], 1);              \
@@ -501,7 +502,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
             const int k = kt16 * BK + 8 * lhi + e;
             unsigned off;
             if constexpr (PW) {
-              off = voff == kNoElement ? kNoElement : voff + static_cast<unsigned>(min(k, kmax)) * x_cbytes;
+              // (a padding row is no element: an infinity of the last channel times zero is NaN)
+              off = voff == kNoElement || k > kmax ? kNoElement : voff + static_cast<unsigned>(k) * x_cbytes;
             } else {
               const int4 tap = a.ktab[k];
               const unsigned bad = MODE == kModeOneMask

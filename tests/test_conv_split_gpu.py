@@ -151,3 +151,73 @@ def test_sums_of_one_sign(K, case):
     err = np.linalg.norm(y[:2].cpu().numpy() - want) / np.linalg.norm(want)
     kk = cin * k * k
     assert err <= 0.29 * 2.0 ** -23 * (np.sqrt(kk / 2 / 3) / 4 + 1)     # ... and the sum over slices and the store
+
+
+@pytest.mark.parametrize("slices", [1, 3, 6])
+@pytest.mark.parametrize("config", [-1, 1, 4, 7])
+@pytest.mark.parametrize("geom", [
+    # cin, k, stride, pad, dilation, group, cout: padding rows of K, several slices (and more than there are
+    # stages), strides, dilations and groups in the products formed again
+    (17, 1, 1, 0, 1, 1, 20), (33, 1, 1, 0, 1, 1, 70), (129, 1, 2, 0, 1, 1, 40), (24, 3, 2, 1, 1, 2, 96), (16, 3, 1, 2, 2, 1, 33),
+    (35, 3, 1, 1, 1, 1, 24), (5, 1, 1, 0, 1, 1, 3), (8, 3, 1, 1, 1, 1, 130)])
+def test_special_values_everywhere(K, geom, config, slices):
+    """Infinities and NaN, the last channel's among them, in every way to gather and with K in slices."""
+    cin, k, s, p, d, g, cout = geom
+    rng = np.random.default_rng(12)
+    x = rng.standard_normal((2, cin, 13, 13)).astype(np.float32)
+    w = (0.1 * rng.standard_normal((cout, cin // g, k, k))).astype(np.float32)
+    for i, v in enumerate((np.inf, -np.inf, np.nan, 3.4e38)):
+        x[i % 2, cin - 1 if i < 2 else (5 * i) % cin, (3 * i) % 13, (7 * i + 2) % 13] = v
+    plan = K.ConvPlan(K.conv_geom(cin, 13, 13, cout, k, s, p, d, g))
+    plan.force_config(config)
+    plan.force_split(slices)
+    plan.force_winograd(0)
+    xd, wd = torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda()
+    ho, wo = plan.output_shape()
+    plan.set_weights(wd.data_ptr())
+    xp = torch.nn.functional.pad(torch.from_numpy(x), (p, p, p, p))
+    for relu in (False, True):
+        y = torch.full((2, cout, ho, wo), float("nan"), device="cuda")
+        plan.forward(2, xd.data_ptr(), y.data_ptr(), activation=int(relu))
+        torch.cuda.synchronize()
+        want = torch.nn.functional.conv2d(xp, torch.from_numpy(w), stride=s, dilation=d, groups=g)
+        want, got = want.numpy(), y.cpu().numpy()
+        if relu:                       # (what ReLU makes of NaN and of -inf, which it multiplies by zero, is not held here)
+            got, want = np.where(want > 0, got, 0), np.where(want > 0, want, 0)
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        assert np.array_equal(np.where(np.isinf(got), np.sign(got), 0), np.where(np.isinf(want), np.sign(want), 0))
+        ok = np.isfinite(want)
+        big = np.maximum(np.abs(want[ok]), 1.0)
+        assert np.all(np.abs(got[ok].astype(np.float64) - want[ok]) <= 20 * cin * k * k * 2.0 ** -24 * big)
+
+
+@pytest.mark.parametrize("k,n", [(17, 5), (100, 40), (33, 70)])
+def test_infinities_through_an_inner_product(K, k, n):
+    import ctypes
+    plan = K.ConvPlan.__new__(K.ConvPlan)
+    plan.handle = ctypes.c_void_p()
+    K.check_mc(K.LIB.mcInnerProductPlanCreate(k, n, 0, ctypes.byref(plan.handle)))
+    rng = np.random.default_rng(13)
+    x = rng.standard_normal((6, k)).astype(np.float32)
+    w = rng.standard_normal((n, k)).astype(np.float32)
+    x[0, k - 1], x[2, k - 1], x[4, 0] = np.inf, -np.inf, np.inf
+    xd, wd, y = torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda(), torch.full((6, n), float("nan"), device="cuda")
+    plan.set_weights(wd.data_ptr())
+    plan.forward(6, xd.data_ptr(), y.data_ptr())
+    torch.cuda.synchronize()
+    want, got = x @ w.T, y.cpu().numpy()
+    assert np.array_equal(np.isinf(got) * np.sign(got), np.isinf(want) * np.sign(want)) and not np.isnan(got).any()
+    ok = np.isfinite(want)
+    assert np.all(np.abs(got[ok] - want[ok]) <= 2 * k * 2.0 ** -24 * (np.abs(x[[1, 3, 5]]) @ np.abs(w.T)).max())
+
+
+def test_infinities_through_the_per_pixel_kernel(K):
+    """At most four channels over many pixels, K not a multiple of 16."""
+    rng = np.random.default_rng(14)
+    x = rng.standard_normal((2, 19, 200, 200)).astype(np.float32)
+    w = rng.standard_normal((3, 19, 1, 1)).astype(np.float32)
+    x[0, 18, 3, 5], x[1, 18, 199, 199] = np.inf, -np.inf
+    plan = K.ConvPlan(K.conv_geom(19, 200, 200, 3, 1, 1, 0))
+    assert plan.kernel_name(2) == "thin_f32"
+    want, got = conv64(x, w, 1, 0), run(K, x, w, 1, 0, -1, 0)
+    assert np.array_equal(np.isinf(got) * np.sign(got), np.isinf(want) * np.sign(want)) and not np.isnan(got).any()
