@@ -55,9 +55,10 @@ CAFFE_API int CaffeBlobHeight(BlobHandle blob);
 CAFFE_API int CaffeBlobWidth(BlobHandle blob);
 CAFFE_API int CaffeBlobCount(BlobHandle blob);
 CAFFE_API real_t* CaffeBlobData(BlobHandle blob);
-/* New shape of shape_size axes; may move the data pointer. */
-/* Extension: fills the blob from `count` values (all of it); in GPU mode the upload starts at once. */
+/* Extension: fills the blob from `count` values, which must be all of it.  The source has been
+   copied when the call returns and may be reused.  In GPU mode the upload starts at once. */
 CAFFE_API int CaffeBlobSetData(BlobHandle blob, const real_t* data, int count);
+/* New shape of shape_size axes; may move the data pointer. */
 CAFFE_API int CaffeBlobReshape(BlobHandle blob, int shape_size, int* shape);
 /* *shape points at shape_size ints in per-thread storage. */
 CAFFE_API int CaffeBlobShape(BlobHandle blob, int* shape_size, int** shape);
