@@ -56,7 +56,8 @@ CAFFE_API int CaffeBlobWidth(BlobHandle blob);
 CAFFE_API int CaffeBlobCount(BlobHandle blob);
 CAFFE_API real_t* CaffeBlobData(BlobHandle blob);
 /* Extension: fills the blob from `count` values, which must be all of it.  The source has been
-   copied when the call returns and may be reused.  In GPU mode the upload starts at once. */
+   copied when the call returns and may be reused.  In GPU mode the upload starts at once, on the
+   calling thread's stream; a Forward on another thread waits for it. */
 CAFFE_API int CaffeBlobSetData(BlobHandle blob, const real_t* data, int count);
 /* New shape of shape_size axes; may move the data pointer. */
 CAFFE_API int CaffeBlobReshape(BlobHandle blob, int shape_size, int* shape);

@@ -18,13 +18,11 @@ Context& Context::Get() {
   return ctx;
 }
 
-Context::Context()
-    : mode_(CPU), device_(0), stream_(nullptr), stream_ready_(false), sync_epoch_(1),
-      pool_(std::make_shared<MemoryPool>()) {}
+ThreadStream::ThreadStream() { HIP_CHECK(hipStreamCreate(&stream)); }  // default priority
 
-Context::~Context() {
-  if (stream_ready_) (void)hipStreamDestroy(stream_);
-}
+ThreadStream::~ThreadStream() { (void)hipStreamDestroy(stream); }
+
+Context::Context() : mode_(CPU), device_(0), pool_(std::make_shared<MemoryPool>()) {}
 
 bool Context::gpu_available() {
   static const bool available = [] {
@@ -41,10 +39,9 @@ void Context::SetMode(DeviceMode mode, int device) {
     HIP_CHECK(hipGetDeviceCount(&n));
     CHECK(device >= 0 && device < n) << "SetMode(GPU): invalid device id " << device << " ("
                                      << n << " device(s) present)";
-    if (stream_ready_ && device != device_) {
+    if (stream_ && device != device_) {
       Sync();
-      HIP_CHECK(hipStreamDestroy(stream_));
-      stream_ready_ = false;
+      stream_.reset();
     }
     HIP_CHECK(hipSetDevice(device));
     device_ = device;
@@ -52,18 +49,18 @@ void Context::SetMode(DeviceMode mode, int device) {
   mode_ = mode;
 }
 
-hipStream_t Context::stream() {
-  if (!stream_ready_) {
+const std::shared_ptr<ThreadStream>& Context::thread_stream() {
+  if (!stream_) {
     HIP_CHECK(hipSetDevice(device_));
-    HIP_CHECK(hipStreamCreate(&stream_));  // default priority
-    stream_ready_ = true;
+    stream_ = std::make_shared<ThreadStream>();
   }
   return stream_;
 }
 
 void Context::Sync() {
-  if (stream_ready_) HIP_CHECK(hipStreamSynchronize(stream_));
-  ++sync_epoch_;
+  if (!stream_) return;
+  HIP_CHECK(hipStreamSynchronize(stream_->stream));
+  stream_->epoch.fetch_add(1);
 }
 
 bool GPUAvailable() { return Context::gpu_available(); }
@@ -201,25 +198,27 @@ MemPoolState64 MemoryPool::GetState() {
 
 SyncedMemory::SyncedMemory(size_t size)
     : size_(size), head_(UNINITIALIZED), pool_(Context::Get().pool()), version_(0),
-      h2d_epoch_(0), h2d_pending_(false) {}
+      h2d_epoch_(0) {}
 
 SyncedMemory::~SyncedMemory() {
   // A pinned block that still feeds an asynchronous upload must not be recycled.
-  if (h2d_pending_ && Context::Get().sync_epoch() == h2d_epoch_) {
-    try {
-      Context::Get().Sync();
-    } catch (...) {
-    }
+  try {
+    wait_pending_h2d();
+  } catch (...) {
   }
   pool_->Return(host_);
   pool_->Return(dev_);
 }
 
+void SyncedMemory::set_pending_h2d() {
+  h2d_stream_ = Context::Get().thread_stream();
+  h2d_epoch_ = h2d_stream_->epoch.load();
+}
+
 void SyncedMemory::wait_pending_h2d() {
-  if (h2d_pending_) {
-    if (Context::Get().sync_epoch() == h2d_epoch_) Context::Get().Sync();
-    h2d_pending_ = false;
-  }
+  if (!h2d_stream_) return;
+  if (h2d_stream_->epoch.load() == h2d_epoch_) HIP_CHECK(hipStreamSynchronize(h2d_stream_->stream));
+  h2d_stream_.reset();
 }
 
 void SyncedMemory::to_cpu() {
@@ -253,13 +252,14 @@ void SyncedMemory::to_gpu() {
       if (!dev_.ptr) dev_ = pool_->RequestDevice(size_, Context::Get().device());
       Context& ctx = Context::Get();
       HIP_CHECK(hipMemcpyAsync(dev_.ptr, host_.ptr, size_, hipMemcpyHostToDevice, ctx.stream()));
-      h2d_pending_ = true;
-      h2d_epoch_ = ctx.sync_epoch();
+      set_pending_h2d();
       head_ = SYNCED;
       break;
     }
     case HEAD_AT_GPU:
     case SYNCED:
+      // an upload queued by another thread (Assign) is not ordered before this thread's launches
+      if (h2d_stream_ && h2d_stream_ != Context::Get().thread_stream()) wait_pending_h2d();
       break;
   }
 }
@@ -311,8 +311,7 @@ void SyncedMemory::Assign(const void* src, size_t bytes) {
     char* host = static_cast<char*>(host_.ptr) + off;
     std::memmove(host, static_cast<const char*>(src) + off, n);
     HIP_CHECK(hipMemcpyAsync(static_cast<char*>(dev_.ptr) + off, host, n, hipMemcpyHostToDevice, ctx.stream()));
-    h2d_pending_ = true;
-    h2d_epoch_ = ctx.sync_epoch();
+    set_pending_h2d();
   }
   head_ = SYNCED;
 }

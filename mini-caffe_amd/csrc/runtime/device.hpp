@@ -11,6 +11,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <map>
 #include <memory>
@@ -31,6 +32,17 @@ namespace caffe {
 
 class MemoryPool;
 
+// A thread's stream.  Shared with every block that has an upload queued on it, so that
+// another thread can wait for the upload, also after the stream's own thread has ended.
+struct ThreadStream {
+  ThreadStream();
+  ~ThreadStream();
+  hipStream_t stream = nullptr;
+  // Advanced by the thread after every synchronisation: work queued at an earlier epoch is done.
+  std::atomic<uint64_t> epoch{1};
+  DISABLE_COPY_AND_ASSIGN(ThreadStream);
+};
+
 // What the reference keeps in its thread-local `Caffe` object
 // (reference src/common.hpp:75-116, common.cpp:7-148).
 class Context {
@@ -42,22 +54,17 @@ class Context {
   void SetMode(DeviceMode mode, int device);
   int device() const { return device_; }
   // The thread's stream; created on first use in GPU mode.
-  hipStream_t stream();
+  hipStream_t stream() { return thread_stream()->stream; }
+  const std::shared_ptr<ThreadStream>& thread_stream();
   // Waits for everything queued on the stream.
   void Sync();
-  // Incremented by every Sync(); lets owners of host buffers know whether an
-  // asynchronous copy they queued can still be in flight.
-  uint64_t sync_epoch() const { return sync_epoch_; }
   const std::shared_ptr<MemoryPool>& pool() { return pool_; }
-  ~Context();
 
  private:
   Context();
   DeviceMode mode_;
   int device_;
-  hipStream_t stream_;
-  bool stream_ready_;
-  uint64_t sync_epoch_;
+  std::shared_ptr<ThreadStream> stream_;
   std::shared_ptr<MemoryPool> pool_;
 };
 
@@ -96,7 +103,9 @@ class SyncedMemory {
   void* mutable_cpu_data();
   const void* gpu_data();
   void* mutable_gpu_data();
-  // Fills the first `bytes` bytes from `src` (which may be the host copy itself).
+  // Fills the first `bytes` bytes from `src` (which may be the host copy itself).  In GPU mode
+  // the upload may be under way on the calling thread's stream when it returns; gpu_data() on
+  // another thread waits for it.
   void Assign(const void* src, size_t bytes);
   SyncedHead head() const { return head_; }
   size_t size() const { return size_; }
@@ -107,13 +116,14 @@ class SyncedMemory {
   void to_cpu();
   void to_gpu();
   void wait_pending_h2d();
+  void set_pending_h2d();
   size_t size_;
   SyncedHead head_;
   MemoryPool::Block host_, dev_;
   std::shared_ptr<MemoryPool> pool_;
   uint64_t version_;
-  uint64_t h2d_epoch_;   // sync epoch at which an async H2D was queued
-  bool h2d_pending_;
+  std::shared_ptr<ThreadStream> h2d_stream_;  // where an upload was queued that nobody has waited for
+  uint64_t h2d_epoch_;                        // ... and that stream's epoch then
   DISABLE_COPY_AND_ASSIGN(SyncedMemory);
 };
 

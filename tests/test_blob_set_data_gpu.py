@@ -45,3 +45,33 @@ def test_wrong_count_is_an_error(gpu_mode):
     blob = net.get_blob("data")
     assert LIB.CaffeBlobSetData(blob.handle, ctypes.c_void_p(x.ctypes.data), 9) == -1
     assert LIB.CaffeBlobSetData(blob.handle, None, 8) == -1
+
+
+def test_filled_by_one_thread_and_used_by_another(gpu_mode):
+    """The upload runs on the filling thread's stream, the forward on its own: the second waits for the first,
+    also when the filling thread has ended."""
+    import threading
+    from minicaffe.base import LIB, check_call
+    mc = gpu_mode
+    count = 16 << 20                                       # 64 MiB: over a millisecond on the link
+    net = identity_net(mc, (1, count))
+    net.forward(data=np.zeros((1, count), np.float32))
+    blob = net.get_blob("data")
+
+    def fill(x):
+        mc.set_runtime_mode(1, 0)
+        check_call(LIB.CaffeBlobSetData(blob.handle, ctypes.c_void_p(x.ctypes.data), count))
+
+    for i in range(1, 6):
+        x = np.full((1, count), i, np.float32)
+        t = threading.Thread(target=fill, args=(x,))
+        t.start()
+        t.join()
+        if i % 2:                                          # ... and the other way round
+            x[:] = 0                                       # the source has been copied
+            net.forward()
+        else:
+            t = threading.Thread(target=lambda: (mc.set_runtime_mode(1, 0), net.forward()))
+            t.start()
+            t.join()
+        assert np.all(net.get_blob("out").data == i)
