@@ -1,6 +1,9 @@
 #include "mc_common.h"
 #include "mchip/kernels.h"
 
+#include <cstdlib>
+#include <mutex>
+#include <shared_mutex>
 #include <utility>
 #include <vector>
 
@@ -9,6 +12,32 @@ std::string& last_error() {
   static thread_local std::string msg;
   return msg;
 }
+
+namespace {
+struct ExitGate {
+  std::shared_mutex mu;
+  bool exiting = false;
+};
+ExitGate& exit_gate() {
+  static ExitGate* gate = new ExitGate();  // never destroyed: threads may end later
+  return *gate;
+}
+}  // namespace
+
+void watch_process_exit() {
+  static const int registered = std::atexit([] {
+    std::unique_lock<std::shared_mutex> lk(exit_gate().mu);  // waits for releases under way
+    exit_gate().exiting = true;
+  });
+  (void)registered;
+}
+
+ReleaseGuard::ReleaseGuard() {
+  exit_gate().mu.lock_shared();
+  allowed_ = !exit_gate().exiting;
+}
+
+ReleaseGuard::~ReleaseGuard() { exit_gate().mu.unlock_shared(); }
 
 namespace {
 struct Workspace {
@@ -34,7 +63,12 @@ struct ThreadScratch {
     workspaces.clear();
     counters.clear();
   }
-  ~ThreadScratch() { release(); }
+  // (HIP's per-thread state is made before this object and so outlives it)
+  ThreadScratch() { (void)hipPeekAtLastError(); }
+  ~ThreadScratch() {
+    ReleaseGuard guard;
+    if (guard.allowed()) release();
+  }
 };
 thread_local ThreadScratch g_scratch;
 }  // namespace
@@ -53,6 +87,7 @@ int stream_counters(hipStream_t st, size_t count, int** out) {
     c->count = 0;
     count = (count + 4095) / 4096 * 4096;
     MC_HIP(hipMalloc(&c->ptr, count * sizeof(int)));
+    watch_process_exit();
     MC_HIP(hipMemset(c->ptr, 0, count * sizeof(int)));
     MC_HIP(hipDeviceSynchronize());  // the zeros are in place before a kernel on any stream counts
     c->count = count;
@@ -74,6 +109,7 @@ int stream_workspace(hipStream_t st, size_t bytes, float** out) {
     ws->ptr = nullptr;
     ws->bytes = 0;
     MC_HIP(hipMalloc(&ws->ptr, bytes));
+    watch_process_exit();
     ws->bytes = bytes;
   }
   *out = ws->ptr;

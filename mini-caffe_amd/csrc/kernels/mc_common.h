@@ -68,6 +68,26 @@ int stream_workspace(hipStream_t st, size_t bytes, float** out);
 // handed out.  A kernel that counts in it leaves every counter at zero again.
 int stream_counters(hipStream_t st, size_t count, int** out);
 
+// A thread releases its device memory, pinned memory and stream when it ends.  That may be
+// while the process exits: joining a thread, as Python does, need not wait for its thread-local
+// destructors, and HIP calls that meet HIP's own teardown corrupt the heap.  Such a
+// release holds a ReleaseGuard; exit() waits for those under way, and later ones find
+// allowed() false and leave everything to the end of the process.
+class ReleaseGuard {
+ public:
+  ReleaseGuard();
+  ~ReleaseGuard();
+  bool allowed() const { return allowed_; }
+  ReleaseGuard(const ReleaseGuard&) = delete;
+  ReleaseGuard& operator=(const ReleaseGuard&) = delete;
+
+ private:
+  bool allowed_;
+};
+// To be called after HIP calls that acquire what is released so: the first call registers the
+// wait, behind HIP's own exit handlers and so to run before them.
+void watch_process_exit();
+
 }  // namespace mchip
 
 #endif  // MCHIP_COMMON_H_

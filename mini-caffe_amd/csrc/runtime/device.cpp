@@ -5,6 +5,7 @@
 #include <cstdlib>
 #include <cstring>
 
+#include "mc_common.h"
 #include "mchip/kernels.h"
 
 namespace caffe {
@@ -18,11 +19,20 @@ Context& Context::Get() {
   return ctx;
 }
 
-ThreadStream::ThreadStream() { HIP_CHECK(hipStreamCreate(&stream)); }  // default priority
+ThreadStream::ThreadStream() {
+  HIP_CHECK(hipStreamCreate(&stream));  // default priority
+  mchip::watch_process_exit();
+}
 
-ThreadStream::~ThreadStream() { (void)hipStreamDestroy(stream); }
+ThreadStream::~ThreadStream() {
+  mchip::ReleaseGuard guard;
+  if (guard.allowed()) (void)hipStreamDestroy(stream);
+}
 
-Context::Context() : mode_(CPU), device_(0), pool_(std::make_shared<MemoryPool>()) {}
+Context::Context() : mode_(CPU), device_(0), pool_(std::make_shared<MemoryPool>()) {
+  // HIP's per-thread state is made before this object and so outlives it
+  if (gpu_available()) (void)hipPeekAtLastError();
+}
 
 bool Context::gpu_available() {
   static const bool available = [] {
@@ -94,7 +104,10 @@ namespace {
 size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 }  // namespace
 
-MemoryPool::~MemoryPool() { Clear(); }
+MemoryPool::~MemoryPool() {
+  mchip::ReleaseGuard guard;
+  if (guard.allowed()) Clear();
+}
 
 MemoryPool::Block MemoryPool::RequestHost(size_t size) {
   size = round_up(size ? size : 1, 256);
@@ -148,6 +161,7 @@ MemoryPool::Block MemoryPool::RequestDevice(size_t size, int device) {
     e = hipMalloc(&b.ptr, size);
   }
   CHECK(e == hipSuccess) << "hipMalloc(" << size << " bytes): " << hipGetErrorString(e);
+  mchip::watch_process_exit();
   std::lock_guard<std::mutex> lk(mu_);
   dev_total_ += size;
   return b;
