@@ -28,13 +28,17 @@ TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "igemm_resnet50_b64_pmc_traffic
 MFMA_PROFILE = os.path.join(ROOT, "profiles", "igemm_resnet50_b64_pmc_mfma_util.txt")
 
 
+def conv_sources_sha256():
+    import hashlib
+    return hashlib.sha256(b"".join(open(f, "rb").read() for f in CONV_SOURCES)).hexdigest()
+
+
 def counter_figure(path, key):
     """A figure that only a rocprofv3 --pmc run can give (HBM bytes per launch, MFMA
     utilisation), read from the committed summary of that run.  The summary ends with
     `key: value` lines, among them the SHA-256 of the convolution kernel sources it was
     taken with; a summary of another kernel version is reported as stale instead of being quoted.
     Returns (value or None, note)."""
-    import hashlib
     fields = {}
     try:
         for line in open(path):
@@ -43,12 +47,12 @@ def counter_figure(path, key):
                 fields[k.strip()] = v.strip()
     except OSError as e:
         return None, "no counter summary (%s)" % e
-    have = hashlib.sha256(b"".join(open(f, "rb").read() for f in CONV_SOURCES)).hexdigest()
+    have = conv_sources_sha256()
     rel = os.path.relpath(path, ROOT)
     if key not in fields or "conv_sources_sha256" not in fields:
         return None, "%s holds no '%s' line" % (rel, key)
     if fields["conv_sources_sha256"] != have:
-        msg = ("%s was taken with another version of conv_igemm.hip + conv_winograd.hip (sha256 %s..., tree "
+        msg = ("%s was taken with another version of the convolution kernels (sha256 %s..., tree "
                "has %s...): re-run the command it names" % (rel, fields["conv_sources_sha256"][:12], have[:12]))
         print("bench.py: STALE COUNTER SUMMARY: " + msg, file=sys.stderr)
         return None, "stale: " + msg
@@ -152,8 +156,10 @@ def main():
     LIB.mcConvTimingEnable(0)
     # achieved: the layers' algorithmic FLOPs (2 x MACs of the direct sum) over the device time
     # of their launches (one launch per contraction).  A 3x3 layer on the Winograd path counts
-    # with its direct-sum FLOPs; mfma_issued_* is what the matrix pipe was actually handed in
-    # the same time (2.25 times fewer products for those layers).
+    # with its direct-sum FLOPs; mfma_issued_* is the matrix pipe's work in the same time, in fp32
+    # FLOPs that would take it as long: 2.25 times fewer products for those layers, and 6/16 of the
+    # direct sum for the layers that multiply bf16 terms (six products for one, each sixteen
+    # times as fast).
     secs = tot_ms.value * 1e-3
     achieved = fl.value / secs / 1e12 if secs > 0 else 0.0
     issued_tflops = issued.value / secs / 1e12 if secs > 0 else 0.0
@@ -163,10 +169,11 @@ def main():
     roofline = {"bound": "mfma", "achieved": round(achieved, 2), "peak": FP32_MFMA_PEAK_TFLOPS,
                 "unit": "TFLOP/s", "frac": round(achieved / FP32_MFMA_PEAK_TFLOPS, 4),
                 "frac_is": "direct-sum FLOPs of all contractions over their device time, against the fp32 MFMA peak: what "
-                           "the layers are worth; the matrix pipe's own utilisation is mfma_issued_frac (the Winograd "
-                           "layers hand it 2.25 times fewer products)",
+                           "the layers are worth, which may pass 1; the matrix pipe's share of its peak rate is "
+                           "mfma_issued_frac (the Winograd layers hand it 2.25 times fewer fp32 products, the other "
+                           "convolutions six bf16 products for one, which take it 6/16 of the time)",
                 "traffic": traffic, "traffic_source": traffic_note,
-                "kernel": "igemm_f32 / winograd_fused (Convolution + InnerProduct, fused BN/Scale/ReLU epilogue; "
+                "kernel": "igemm_split / winograd_fused / igemm_f32 (Convolution + InnerProduct, fused BN/Scale/ReLU epilogue; "
                           "%d of the %d contractions per step are 3x3 stride-1 layers run as F(2x2,3x3) Winograd "
                           "in one launch each)" % (wino.value // steps, launches.value // steps),
                 "launches_per_step": launches.value // steps,
@@ -499,7 +506,8 @@ def configs_report(path, mc, craft, zoo, LIB):
         del net
     lines.append("dir-eq TF/s: the contractions' direct-sum FLOPs over the device time of their launches (a 3x3 layer on "
                  "the Winograd path counts with its direct-sum FLOPs, so this rate can pass the matrix peak); issued "
-                 "TF/s / of peak: what the matrix pipe was handed in the same time, against 157.3 TFLOP/s.")
+                 "TF/s / of peak: what the matrix pipe was handed in the same time, in fp32 FLOPs that take it as long "
+                 "(products of bf16 terms: 6/16 of the direct sum), against 157.3 TFLOP/s.")
     lines.append("CPU column: one pass of the oracle (reference algorithm: per-image im2col + OpenBLAS sgemm, "
                  "unfused layers) on %d host threads at batch 1/4/1/1/8/2." % oracle.openblas_threads())
     with open(path, "w") as f:
@@ -560,8 +568,9 @@ def layer_roofline(path, batch):
     the launch comes.  Bytes = bottom + top + filter, each once.  Two rates per layer: the
     direct sum's FLOPs over the time (what the layer is worth; a Winograd launch can exceed
     the matrix peak on this scale, so no fraction is printed for it) and the FLOPs the matrix
-    pipe was handed (padding of tiles included, 2.25 times fewer products on the Winograd
-    path) with their share of the fp32 peak."""
+    pipe was handed, in fp32 FLOPs that take it as long (2.25 times fewer products on the Winograd
+    path, 6/16 of the direct sum where six products of bf16 terms make one), with their share
+    of the fp32 peak.  The matrix roofline of a layer is that of the kernel it runs on."""
     import torch
     from minicaffe import kernels as K
     from minicaffe.base import LIB
@@ -588,12 +597,15 @@ def layer_roofline(path, batch):
         plan.set_weights(w.data_ptr())
         fl = plan.flops(batch)
         nbytes = 4.0 * (x.numel() + y.numel() + w.numel())
-        t_mfma, t_hbm = fl / (FP32_MFMA_PEAK_TFLOPS * 1e6), nbytes / (HBM_PEAK_GBS * 1e3)
-        roof = max(t_mfma, t_hbm)
         winograd = plan.kernel_name(batch) == "winograd_f32"
         # a layer the library runs on the Winograd path is also timed on the direct one
         for mode in ((-1, 0) if winograd else (-1,)):
             plan.force_winograd(mode)
+            name = plan.kernel_name(batch)
+            # six bf16 products for one, at sixteen times the rate
+            peak = FP32_MFMA_PEAK_TFLOPS * (16 / 6 if name.startswith("igemm_split") else 1)
+            t_mfma, t_hbm = fl / (peak * 1e6), nbytes / (HBM_PEAK_GBS * 1e3)
+            roof = max(t_mfma, t_hbm)
             for _ in range(5):
                 plan.forward(batch, x.data_ptr(), y.data_ptr(), activation=K.ACT_RELU, stream=stream)
             torch.cuda.synchronize()
@@ -621,15 +633,18 @@ def layer_roofline(path, batch):
                 "%d->%d %dx%d/%d @%d" % (cin, cout, k, k, s_, h), cnt, fl / 1e9, nbytes / 1e6, fl / nbytes,
                 "mfma" if t_mfma >= t_hbm else "hbm", roof, us, fl / us / 1e6, issued.value / us / 1e6,
                 100 * issued.value / us / 1e6 / FP32_MFMA_PEAK_TFLOPS,
-                "" if not winograd else ("Winograd F(2x2,3x3), one fused launch" if mode == -1
-                                         else "(same layer pinned to the direct path; not in the total)")))
+                name + ("" if mode == -1 else " (same layer pinned to the direct path; not in the total)")))
         del x, y, w, plan
     lines.append("all 53 convolutions: direct-sum roofline %.0f us, measured %.0f us (direct-sum equivalent %.1f%% of the "
                  "per-layer roofline); issued to the matrix pipe: %.1f%% of the fp32 peak over the same time"
                  % (sum_roof, sum_meas, 100 * sum_roof / sum_meas,
                     100 * sum_issued / sum_meas / 1e6 / FP32_MFMA_PEAK_TFLOPS))
-    lines.append("roof us = max(FLOP / 157.3 TFLOP/s, bytes / 8 TB/s) with the FLOPs and bytes of the direct sum; 20 "
+    lines.append("roof us = max(FLOP / peak, bytes / 8 TB/s) with the FLOPs and bytes of the direct sum; peak = 157.3 TFLOP/s "
+                 "(fp32 products), 419.5 for igemm_split (six bf16 products for one at sixteen times the rate); 20 "
                  "back-to-back calls between two events.")
+    lines.append("")
+    lines.append("conv_sources_sha256: " + conv_sources_sha256())
+    lines.append("date: " + time.strftime("%Y-%m-%d"))
     with open(path, "w") as f:
         f.write("\n".join(lines) + "\n")
 

@@ -151,8 +151,9 @@ int mcConvWinogradDefault(int mode);
  * events recorded on the launch stream.  mcConvTimingCollect waits for them,
  * returns the summed device time, the number of contractions and their
  * algorithmic FLOPs (those of the direct sum), and clears the list;
- * mcConvTimingCollectDetail also returns the FLOPs handed to the matrix pipe
- * (fewer on the Winograd path) and the number of Winograd contractions. */
+ * mcConvTimingCollectDetail also returns what was handed to the matrix pipe, in fp32
+ * FLOPs that take it as long (fewer than the direct sum on the Winograd path, and 6/16 of it where
+ * six products of bf16 terms make one), and the number of Winograd contractions. */
 int mcConvTimingEnable(int on);
 int mcConvTimingCollect(double* total_ms, long* launches, double* flops);
 int mcConvTimingCollectDetail(double* total_ms, long* launches, double* flops, double* issued_flops,

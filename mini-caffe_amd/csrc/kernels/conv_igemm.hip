@@ -1,4 +1,6 @@
-// Implicit-GEMM Convolution / Deconvolution for gfx950 (fp32 MFMA).
+// Implicit-GEMM Convolution / Deconvolution / InnerProduct for gfx950: fp32 accuracy, by fp32
+// MFMA (igemm_kernel: Deconvolution, InnerProduct, short sums) or by three bf16 terms per operand
+// on the bf16 matrix pipe (igemm_split.h: all other Convolutions).
 //
 // The contraction the reference performs per image as im2col + sgemm
 // (reference src/layers/base_conv_layer.cpp:254-271, src/util/im2col.cpp:19-55)
@@ -19,9 +21,10 @@
 // Tiling: 256 threads = 4 wavefronts per workgroup, BM x BN output tile,
 // K step 16, LDS double buffer filled from registers (global loads for tile
 // t+1 are in flight while tile t is multiplied).  Each wavefront owns a grid of
-// 32x32 accumulators fed by v_mfma_f32_32x32x2_f32.  Filters are repacked once
-// into K-major, zero-padded [g][Kpad][Mpad] so that A-tile loads are aligned
-// float4 rows and need no predicates.
+// 32x32 accumulators, fed by v_mfma_f32_32x32x2_f32 (v_mfma_f32_32x32x16_bf16 in the
+// split kernel).  Filters are repacked once, zero-padded, into the tiles the K loop loads
+// (pack_weights_kernel, pack_split_kernel), so that A-tile loads are aligned 16-byte rows and
+// need no predicates.
 #include "conv_internal.h"
 #include "mc_common.h"
 #include "mchip/kernels.h"
@@ -726,6 +729,7 @@ const TileConfig kConfigs[] = {
       igemm_kernel<64, 64, 2, 2, 4, kModePointwise, 2>}},
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
+static_assert(kNumConfigs == kNumSplitConfigs, "mcConvPlanForceConfig takes one range of numbers for both kernels");
 
 // One stride-1 gather problem: the whole Convolution, or one output-parity
 // class of a Deconvolution.
@@ -787,7 +791,11 @@ namespace {
 struct TimedLaunch {
   hipEvent_t start, stop;
   double flops;   // algorithmic: what the layer's direct sum takes
-  double issued;  // what the matrix pipe is given (less on the Winograd path)
+  // What the matrix pipe is given, in fp32 FLOPs of the same time: less than `flops` on the
+  // Winograd path, 6/16 of them where six products of bf16 terms, each sixteen times as fast,
+  // make one.
+  double issued;
+  bool winograd;
   const char* name;
 };
 thread_local bool g_timing = false;
@@ -1269,6 +1277,7 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
       MC_HIP(hipEventCreate(&tl.start));
       MC_HIP(hipEventCreate(&tl.stop));
       tl.flops = tl.issued = mcConvPlanFlops(plan, num);
+      tl.winograd = false;
       tl.name = "depthwise_f32";
       MC_HIP(hipEventRecord(tl.start, st));
     }
@@ -1354,7 +1363,9 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
   if (timed) {
     MC_HIP(hipEventCreate(&tl.start));
     MC_HIP(hipEventCreate(&tl.stop));
-    tl.flops = tl.issued = flops;
+    tl.flops = flops;
+    tl.issued = plan->split && !thin ? flops * (6. / 16.) : flops;
+    tl.winograd = false;
     tl.name = thin ? "thin_f32"
                    : plan->split ? kSplitConfigs[choice.config].name : kConfigs[choice.config].name;
     MC_HIP(hipEventRecord(tl.start, st));
@@ -1528,6 +1539,7 @@ int conv_forward(const mcConvPlan* plan, int num, const float* bottom, float* to
       MC_HIP(hipEventCreate(&tl.stop));
       tl.flops = mcConvPlanFlops(plan, num);
       tl.issued = winograd_issued_flops(plan->winograd, num);
+      tl.winograd = true;
       tl.name = "winograd_f32";
       MC_HIP(hipEventRecord(tl.start, st));
     }
@@ -1602,7 +1614,7 @@ int mcConvTimingCollectDetail(double* total_ms, long* launches, double* flops, d
     ms += e;
     fl += t.flops;
     is += t.issued;
-    wino += t.issued != t.flops;
+    wino += t.winograd;
     (void)hipEventDestroy(t.start);
     (void)hipEventDestroy(t.stop);
   }

@@ -558,10 +558,12 @@ bool winograd_fits(const WinogradState* w, int /*num*/) {
 // 8x8: 101 / 156; VGG's 64 -> 64 on 300x300, batch 8: 295 / 423, 512 -> 512 on 38x38:
 // 245 / 430; the RPN head 1024 -> 512 on 38x63: 110 / 197; SSD's merged heads 512 -> 100
 // on 38x38: 86 / 124, 1024 -> 150 on 19x19: 66 / 97, 512 -> 150 on 10x10: 35 / 39).
-// (Those direct times are of fp32 products.  With products from bf16 terms the direct path
-// comes close and this one still leads: 64 -> 64 @56 95 us against 100, 128 @28 92 / 98,
-// 256 @14 82 / 90, 512 @7 85 / 88; batch 8: 64 @300 300 / 310, 128 @150 236 / 260, 256 @75
-// 241 / 259, 512 @38 245 / 270; RPN head 105 / 131.)
+// Those direct times are of fp32 products.  Against products from bf16 terms, with the best
+// direct tile of all, this path still leads on launches that fill the chip: batch 64, 64 -> 64 @56
+// 100.5 us against 98.7 (even), 128 @28 86 / 93, 256 @14 80 / 88, 512 @7 86.5 / 88.7; batch 8, 64 @300
+// 295 / 322, 128 @150 236 / 258, 256 @75 236 / 259, 512 @38 239 / 269, 512 @19 84.6 / 85.8; RPN head
+// 108 / 130.  On smaller ones it no longer does, and the rule below has not followed: batch 8,
+// 64 @56 24.6 us against 21.0, 128 @28 26.0 / 21.8, 256 @14 28.3 / 21.2, 512 @7 37.2 / 23.9.
 // What loses: 32 input channels (the loop is four rounds long: 56 / 47 us), an
 // output tile that is half padding (64 -> 32: 86 / 82), and launches of a few tiles,
 // whose time is this kernel's longer prologue and finish (256 -> 150 on 5x5 maps, 9

@@ -68,19 +68,21 @@ __device__ __forceinline__ void finish_split_tile(const IgemmArgs& a, int slices
 // product, 2^-27.4 on the average of random operands.  Summing m l' and l m' as well costs 10 to
 // 18 % of a launch; instead sums of a few products, which round too seldom to hide the
 // difference, stay with the fp32 kernel, see short_sums).
-// The sums run in fp32 accumulators: h h' in one, the five small ones in another, added once
-// after the K loop, so the large accumulator rounds once per sixteen K rows
-// where the fp32 instruction rounds sixteen times: the error against a 64-bit sum is
-// about a third of the fp32 instruction's (K = 576, random operands: 1.4e-7 against 4.1e-7
-// of the norm; all six in one accumulator: 3.6e-7, and on non-negative bottoms above it).
+// The sums run in fp32 accumulators: h h' in one or two, the five small ones in another, added
+// once after the K loop, so the large accumulator rounds a few times per sixteen K rows
+// where the fp32 instruction rounds eight: over one chain of additions the error against a
+// 64-bit sum is 0.32 to 0.48 of the fp32 instruction's (512 -> 2048 on 64 x 7x7, five
+// distributions of operands; all six products in one accumulator: up to 1.17 of it).  How many
+// chains a launch needs beside that: least_chains.
 // Unlike fp32 products, which keep the vector ALU of every co-resident wavefront waiting,
 // bf16 products overlap with it: six VALU instructions per product cost nothing measurable
 // with four wavefronts per SIMD.
 //
-// What bounds it: the matrix pipe at the clock the chip holds under this load (about 1.7 GHz):
-// 1024 -> 1024 1x1 over 16 384 pixels 171 us, 201 TFLOP/s, 68 % of the cycles (fp32 products: 261
-// us); small K on large maps: HBM (64 -> 256 1x1 on 64 x 56x56: 77 -> 61 us, 4.2 TB/s); single
-// images: the latency of a slice's loads (512 -> 512 3x3 on one 7x7 map: 21.8 -> 16.4 us).
+// What bounds it: the matrix pipe at the clock the chip holds under this load:
+// 1024 -> 1024 1x1 over 16 384 pixels 174 us, 197 TFLOP/s (fp32 products: 261 us); small K on
+// large maps: HBM (64 -> 256 1x1 on 64 x 56x56: 77 -> 67 us, 3.8 TB/s); single
+// images: the latency of a slice's loads (512 -> 512 3x3 on one 7x7 map: 21 -> 16 us).
+// The two multiplications by 2^24 per pair of bottom values cost 2 % of a full launch.
 //
 // Values the split cannot hold (infinities, NaN, magnitudes of 2^103 and above) and sums of
 // 2^80 and above leave an accumulator non-finite.  A wavefront that finds one after the K loop
@@ -90,8 +92,8 @@ __device__ __forceinline__ void finish_split_tile(const IgemmArgs& a, int slices
 // MODE selects how the K loop finds and guards the elements it gathers:
 //   kModeMasks     tap table + one "outside the image" bit mask per tap row and
 //                  per tap column (any kernel up to 31 x 31 taps);
-//   kModeOneMask   tap table + one mask with a bit per (row, column) tap pair,
-//                  for kernels with at most 31 taps (3x3, 5x5) and a channel
+//   kModeOneMask   one mask with a bit per (row, column) tap pair, the taps' offsets from
+//                  the scalar unit, for kernels with at most 31 taps (3x3, 5x5) and a channel
 //                  count that is a multiple of 4: the K rows are then ordered
 //                  (channel block of 4, tap, channel in block), so four
 //                  consecutive rows share one tap and one validity test;
@@ -575,16 +577,16 @@ struct SplitConfig {
     igemm_split_kernel<BM, BN, WM, WN, OCC, kModeOneMask, KS>,                \
     igemm_split_kernel<BM, BN, WM, WN, OCC, kModePointwise, KS>}}
 const SplitConfig kSplitConfigs[] = {
-    MC_CONFIG(128, 128, 2, 2, 2, 1, 0.56f, 3.3f, "igemm_f32_128x128"),
-    MC_CONFIG(128, 64, 2, 2, 3, 1, 0.363f, 0.9f, "igemm_f32_128x64"),
-    MC_CONFIG(64, 128, 2, 2, 3, 1, 0.377f, 1.2f, "igemm_f32_64x128"),
+    MC_CONFIG(128, 128, 2, 2, 2, 1, 0.56f, 3.3f, "igemm_split_128x128"),
+    MC_CONFIG(128, 64, 2, 2, 3, 1, 0.363f, 0.9f, "igemm_split_128x64"),
+    MC_CONFIG(64, 128, 2, 2, 3, 1, 0.377f, 1.2f, "igemm_split_64x128"),
     // (3, 5 and 6, taken on request only, are other places' tiles: each instance is many
     // seconds of compilation, and none of their own shapes was the best of any layer measured)
-    MC_CONFIG(64, 64, 2, 2, 3, 2, 0.f, 0.f, "igemm_f32_64x64x32"),
-    MC_CONFIG(32, 128, 1, 4, 4, 1, 0.215f, 0.6f, "igemm_f32_32x128"),
-    MC_CONFIG(32, 128, 1, 4, 4, 1, 0.f, 0.f, "igemm_f32_32x128"),
-    MC_CONFIG(64, 128, 2, 2, 3, 1, 0.f, 0.f, "igemm_f32_64x128"),
-    MC_CONFIG(64, 64, 2, 2, 3, 2, 0.21f, 0.8f, "igemm_f32_64x64x32"),
+    MC_CONFIG(64, 64, 2, 2, 3, 2, 0.f, 0.f, "igemm_split_64x64x32"),
+    MC_CONFIG(32, 128, 1, 4, 4, 1, 0.215f, 0.6f, "igemm_split_32x128"),
+    MC_CONFIG(32, 128, 1, 4, 4, 1, 0.f, 0.f, "igemm_split_32x128"),
+    MC_CONFIG(64, 128, 2, 2, 3, 1, 0.f, 0.f, "igemm_split_64x128"),
+    MC_CONFIG(64, 64, 2, 2, 3, 2, 0.21f, 0.8f, "igemm_split_64x64x32"),
 };
 #undef MC_CONFIG
 constexpr int kNumSplitConfigs = sizeof(kSplitConfigs) / sizeof(kSplitConfigs[0]);

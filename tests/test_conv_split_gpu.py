@@ -38,7 +38,7 @@ def run(K, x, w, s, p, config, slices):
     return y.cpu().numpy()
 
 
-@pytest.mark.parametrize("config", [0, 1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("config", [0, 1, 2, 3, 4, 5, 6, 7])     # (3, 5 and 6 are the tiles of 7, 4 and 2)
 @pytest.mark.parametrize("case", [
     # cin, size, cout, kernel, stride, pad, batch, slices: one K tile to many, odd and even numbers of
     # stages, rows and pixels on both sides of a tile's edge, all three ways to gather
