@@ -306,7 +306,9 @@ void* SyncedMemory::mutable_gpu_data() {
 // A large blob goes to pinned memory a piece at a time, each piece on its way to the device
 // while the next one is copied; a host copy of the whole blob first leaves the copy engine
 // waiting (batch of 64 images, 38.5 MB: 6.25 ms per ResNet-50 pass, 5.47 in pieces of 2 MiB).
-// Only for all of the block: a part would leave the two copies different behind it.
+// Only for all of the block: a part would leave the two copies different behind it.  (A blob
+// that has been larger keeps its larger block, so later, smaller arrays are copied whole and
+// uploaded by the forward.)
 void SyncedMemory::Assign(const void* src, size_t bytes) {
   CHECK_LE(bytes, size_) << "SyncedMemory::Assign: more bytes than the block holds";
   Context& ctx = Context::Get();
