@@ -519,7 +519,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 #define MC_FACTORS(row) (&As[0][0][row][BK])
 #define MC_ARRIVED (reinterpret_cast<int*>(&As[0][0][0][0]))
 #define MC_SLICES batch.slices
-#define MC_AHEAD 1
+#define MC_AHEAD (OCC == 8 ? 2 : 1)
 #define MC_PLAIN PW4
 #include "igemm_finish.h"
 }
