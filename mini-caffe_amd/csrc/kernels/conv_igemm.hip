@@ -729,7 +729,7 @@ const TileConfig kConfigs[] = {
       igemm_kernel<64, 64, 2, 2, 4, kModePointwise, 2>}},
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
-static_assert(kNumConfigs == kNumSplitConfigs, "mcConvPlanForceConfig takes one range of numbers for both kernels");
+static_assert(kNumConfigs <= kNumSplitConfigs, "mcConvPlanForceConfig: the fp32 kernel's tiles come first");
 
 // One stride-1 gather problem: the whole Convolution, or one output-parity
 // class of a Deconvolution.
@@ -808,7 +808,7 @@ thread_local std::vector<TimedLaunch> g_timed;
 // larger tiles everywhere their extra reuse could matter.  Narrow outputs
 // (<= 32 channels per group) use the 32-row tiles instead of padding M to 64.
 int pick_config(const mcConvPlan* plan, long pixels) {
-  if (plan->forced_config >= 0) return plan->forced_config;
+  if (plan->forced_config >= 0 && plan->forced_config < kNumConfigs) return plan->forced_config;
   const int M = plan->M;
   int bm = 64, bn = 64;
   if (M <= 32) {
@@ -870,15 +870,30 @@ int least_chains(const mcConvPlan* plan, const SubProblem& s, int num) {
 struct LaunchChoice {
   int config, slices;
 };
+
+// Whether igemm_small_kernel can run the launch: no tap table, and rows past K may be read past
+// the last channel, so that the offsets of a flagged pixel stay below 2^32.
+constexpr int kSmallMaxTiles = 1024;  // 32 KB of taps
+bool fits_small(const mcConvPlan* plan, const std::vector<const SubProblem*>& live, int num) {
+  if (plan->force_general || live.size() != 1) return false;
+  const SubProblem& s = *live[0];
+  const long plane = (long)plan->geom.height_in * plan->geom.width_in;
+  return (s.pointwise || s.one_mask) && (long)num * plan->geom.channels_in * plane < (1L << 27) &&
+         (s.Kpad + BK) * plane < (1L << 27) && (long)s.Kpad * plan->Mpad * 6 < (1L << 31) &&
+         (s.pointwise || s.Kpad / BK <= kSmallMaxTiles);
+}
 LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const SubProblem*>& live, int num) {
   LaunchChoice best = {3, 1};
   double best_us = 1e30;
   int least = 1;
+  const bool small_ok = fits_small(plan, live, num);
+  int forced = plan->forced_config;
+  if (forced >= kNumConfigs && !small_ok) forced = 7;
   for (const SubProblem* s : live) least = std::max(least, least_chains(plan, *s, num));
   for (int c = 0; c < kNumSplitConfigs; ++c) {
     const SplitConfig& cfg = kSplitConfigs[c];
-    if (plan->forced_config >= 0 ? c != plan->forced_config : cfg.stage_us == 0.f) continue;
-    if (plan->forced_config < 0 && cfg.bm == 32 && plan->M > 32) continue;
+    if (cfg.waves || (forced >= 0 ? c != forced : cfg.stage_us == 0.f)) continue;
+    if (forced < 0 && cfg.bm == 32 && plan->M > 32) continue;
     const long mt = ceil_div(plan->M, cfg.bm);
     long blocks = 0, tile_stages = 0;
     int min_kt = 1 << 30;
@@ -900,6 +915,36 @@ LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const S
                                                    : (rounds < 2 ? 2. : rounds < 3 ? 1.4 : rounds < 4 ? 1.15 : 1.);
       double us = rounds * (stages / s * cfg.stage_us * alone + cfg.fixed_us);
       if (s > 1) us += 1.2 + 0.26 * s + 2e-6 * blocks * s * cfg.bm * cfg.bn;
+      if (us < best_us) {
+        best_us = us;
+        best = {c, s};
+      }
+    }
+  }
+  if (!small_ok || (forced >= 0 && forced < kNumConfigs)) return best;
+  // The small-launch kernel, whose time is a fixed part, the longer of a wavefront's K tiles one
+  // after the other and a CU's share of all of them, and what slices cost.  The constants fit
+  // 1400 launches of 105 layers (10 % rms: 3x3 and 5x5 1 us of taps; strided bottoms 1.75
+  // times the gather); the tiles above take 3 us more than their estimate.  Taken where it is ahead by
+  // more than the estimates' error: over those layers 1648 us, always the best kernel and
+  // slices 1611, without this kernel 1939.
+  best_us = forced >= 0 ? 1e30 : 0.9 * (best_us + 3.0);
+  const SubProblem& sub = *live[0];
+  const int KT = sub.Kpad / BK;
+  const long tiles = (long)ceil_div(plan->M, 32) * ceil_div((long)num * sub.Hq * sub.Wq, 32) * plan->geom.group;
+  for (int c = kNumConfigs; c < kNumSplitConfigs; ++c) {
+    const SplitConfig& cfg = kSplitConfigs[c];
+    if (forced >= 0 && c != forced) continue;
+    int first = std::max(1, std::min(ceil_div(least, cfg.chains), KT));
+    int last = std::max(first, std::min(16, KT / (2 * cfg.waves)));
+    if (plan->forced_split >= 1) first = last = std::min(plan->forced_split, std::max(KT, 1));
+    for (int s = first; s <= last; ++s) {
+      const double wgs = static_cast<double>(tiles) * s;
+      const double per_wave = ceil_div(ceil_div(KT, s), cfg.waves);
+      const double share = std::ceil(wgs / kNumCu) * per_wave * cfg.waves * (0.25 / 4) * (sub.q_sw > 1 ? 1.75 : 1.);
+      double us = 3.0 + (sub.pointwise ? 0. : 1.) + std::max(0.31 * per_wave, share) +
+                  wgs / kNumCu * (cfg.waves > 4 ? 1.05 : 0.55);
+      if (s > 1) us += 1.7 + 0.0021 * wgs;
       if (us < best_us) {
         best_us = us;
         best = {c, s};
@@ -1223,7 +1268,8 @@ int mcConvPlanForceConfig(mcConvPlan* plan, int config) {
   // compare the pointwise and one-mask fast paths against it)
   plan->force_general = config >= 100;
   if (config >= 100) config -= 100;
-  MC_REQUIRE(config >= -1 && config < kNumConfigs, "mcConvPlanForceConfig: no such configuration");
+  MC_REQUIRE(config >= -1 && config < (plan->split ? kNumSplitConfigs : kNumConfigs),
+             "mcConvPlanForceConfig: no such configuration");
   plan->forced_config = config;
   return 0;
 }
@@ -1244,6 +1290,97 @@ int mcConvPlanForceSplit(mcConvPlan* plan, int slices) {
 }  // extern "C"
 
 namespace {
+
+// One launch of igemm_small_kernel.
+int launch_small(const mcConvPlan* plan, const SubProblem& s, const LaunchChoice& choice, int num,
+                 const float* bottom, float* top, const mcEpilogue* ep, hipStream_t st, float* top_second,
+                 int c_first) {
+  const mcConvGeom& g = plan->geom;
+  const SplitConfig& cfg = kSplitConfigs[choice.config];
+  const long in_count = (long)num * g.channels_in * g.height_in * g.width_in;
+  const long shift = (long)s.tap_shift + s.pix_shift;
+  SmallArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.x = reinterpret_cast<const float*>(reinterpret_cast<const char*>(bottom) - shift);
+  a.x_bytes = static_cast<unsigned>(in_count * 4 + shift);
+  a.pix_shift = s.pix_shift;
+  a.wt = s.wt_split_dev;
+  a.y = top;
+  a.y_second = top_second;
+  a.c_first = c_first;
+  a.scale = ep ? ep->scale : nullptr;
+  a.shift = ep ? ep->shift : nullptr;
+  a.residual = ep ? ep->residual : nullptr;
+  a.act = ep ? ep->activation : MC_ACT_NONE;
+  a.slope = ep ? ep->negative_slope : 0.f;
+  a.HqWq = s.Hq * s.Wq;
+  a.Wq = s.Wq;
+  a.P = num * a.HqWq;
+  make_fast_div(a.HqWq, (unsigned long long)a.P + 512, &a.div_hw_mul, &a.div_hw_shift);
+  make_fast_div(a.Wq, (unsigned long long)a.HqWq + 1, &a.div_w_mul, &a.div_w_shift);
+  a.H = g.height_in;
+  a.W = g.width_in;
+  a.q_sh = s.q_sh;
+  a.q_sw = s.q_sw;
+  a.in_oh = s.in_oh;
+  a.in_ow = s.in_ow;
+  a.x_cbytes = g.height_in * g.width_in * 4;
+  a.x_nstride = g.channels_in * g.height_in * g.width_in;
+  a.x_gstride = plan->Cin_g * g.height_in * g.width_in;
+  a.K = s.K;
+  a.KT = s.Kpad / BK;
+  a.slices = choice.slices;
+  a.kt_per_slice = ceil_div(std::max(a.KT, 1), a.slices);
+  a.M = plan->M;
+  a.Mpad = plan->Mpad;
+  a.MT = ceil_div(plan->M, cfg.bm);
+  a.NT = ceil_div(a.P, cfg.bn);
+  a.groups = g.group;
+  const long tiles = (long)a.MT * a.NT * g.group, wgs = tiles * a.slices;
+  MC_REQUIRE(wgs < (1L << 31), "mcConvForward: grid too large");
+  a.pixels_fastest = 6. * plan->M * g.group * s.K > 4. * in_count;
+  make_fast_div(a.pixels_fastest ? a.NT : a.MT, wgs + 1, &a.div_inner_mul, &a.div_inner_shift);
+  make_fast_div(a.pixels_fastest ? a.MT : a.NT, wgs + 1, &a.div_outer_mul, &a.div_outer_shift);
+  make_fast_div(g.group, wgs + 1, &a.div_group_mul, &a.div_group_shift);
+  a.y_cstride = plan->Ho * plan->Wo;
+  a.y_nstride = g.channels_out * plan->Ho * plan->Wo;
+  if (s.one_mask) {
+    a.n_dh = static_cast<int>(s.tap_dh.size());
+    a.n_dw = static_cast<int>(s.tap_dw.size());
+    make_fast_div(a.n_dh * a.n_dw, (unsigned long long)s.Kpad / 4 + 1, &a.div_taps_mul, &a.div_taps_shift);
+    a.div_kw_mul = 65536 / a.n_dw + 1;  // exact for the at most 31 taps
+    a.tap_h4 = g.dilation_h * g.width_in * 4;
+    a.tap_w4 = g.dilation_w * 4;
+    a.dil_h = g.dilation_h;
+    a.dil_w = g.dilation_w;
+  }
+  a.ktab = s.ktab_dev;
+  if (a.slices > 1) {
+    a.partial_tiles = static_cast<int>(tiles);
+    if (stream_workspace(st, sizeof(float) * tiles * cfg.bm * cfg.bn * a.slices, &a.partial)) return -1;
+    if (stream_counters(st, static_cast<size_t>(tiles), &a.counters)) return -1;
+  }
+  TimedLaunch tl;
+  const bool timed = g_timing;
+  if (timed) {
+    MC_HIP(hipEventCreate(&tl.start));
+    MC_HIP(hipEventCreate(&tl.stop));
+    tl.flops = 2.0 * a.P * plan->M * g.group * s.K;
+    tl.issued = tl.flops * (6. / 16.);
+    tl.winograd = false;
+    tl.name = cfg.name;
+    MC_HIP(hipEventRecord(tl.start, st));
+  }
+  const bool pointwise = s.pointwise;
+  const unsigned taps_lds = pointwise ? 0u : 32u * a.kt_per_slice;
+  cfg.small[pointwise ? kModePointwise : kModeOneMask]<<<static_cast<unsigned>(wgs), 64 * cfg.waves, taps_lds, st>>>(a);
+  MC_LAUNCH_CHECK();
+  if (timed) {
+    MC_HIP(hipEventRecord(tl.stop, st));
+    g_timed.push_back(tl);
+  }
+  return 0;
+}
 
 // top_second != nullptr: the plan's output channels [0, c_first) go to `top`, the
 // others to top_second.
@@ -1329,6 +1466,12 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
   if (min_kt == (1 << 30)) min_kt = 1;
   // (the per-pixel kernel writes one top only)
   const bool thin = !top_second && use_thin(plan, num);
+  if (!thin && plan->split && kSplitConfigs[choice.config].waves) {
+    LaunchChoice small = choice;
+    // (a request for one slice means two where there are two tops, as below)
+    if (top_second && plan->forced_split == 1) small.slices = 2;
+    return launch_small(plan, *live[0], small, num, bottom, top, ep, st, top_second, c_first);
+  }
   // slices are chosen for the plan as a whole: all sub-problems of a launch run
   // side by side
   // Two tops are told apart by the pass that sums the slices, so such a launch

@@ -559,6 +559,8 @@ __global__ void pack_split_kernel(const float* __restrict__ w, uint16_t* __restr
   }
 }
 
+#include "igemm_small.h"
+
 struct SplitConfig {
   int bm, bn;
   int ks;   // 16-row K tiles per stage
@@ -569,13 +571,20 @@ struct SplitConfig {
   float stage_us, fixed_us;
   const char* name;
   void (*kernel[3])(const IgemmBatch);  // indexed by mode
+  // igemm_small_kernel, whose tiles are taken for small launches: wavefronts that share K and the
+  // kernels by mode (0 and null: igemm_split_kernel)
+  int waves;
+  void (*small[3])(const SmallArgs);
 };
 
 #define MC_CONFIG(BM, BN, WM, WN, OCC, KS, STAGE, FIXED, NAME)                \
   {BM, BN, KS, OCC, BM / WM * (BN / WN) == 32 * 32 ? 2 : 1, STAGE, FIXED, NAME,                                       \
    {igemm_split_kernel<BM, BN, WM, WN, OCC, kModeMasks, KS>,                  \
     igemm_split_kernel<BM, BN, WM, WN, OCC, kModeOneMask, KS>,                \
-    igemm_split_kernel<BM, BN, WM, WN, OCC, kModePointwise, KS>}}
+    igemm_split_kernel<BM, BN, WM, WN, OCC, kModePointwise, KS>}, 0, {nullptr, nullptr, nullptr}}
+#define MC_SMALL(NW, NAME)                                                   \
+  {32, 32, 1, 16 / NW, NW, 0.f, 0.f, NAME, {nullptr, nullptr, nullptr}, NW,  \
+   {nullptr, igemm_small_kernel<NW, 1, kModeOneMask>, igemm_small_kernel<NW, 1, kModePointwise>}}
 const SplitConfig kSplitConfigs[] = {
     MC_CONFIG(128, 128, 2, 2, 2, 1, 0.56f, 3.3f, "igemm_split_128x128"),
     MC_CONFIG(128, 64, 2, 2, 3, 1, 0.363f, 0.9f, "igemm_split_128x64"),
@@ -587,7 +596,10 @@ const SplitConfig kSplitConfigs[] = {
     MC_CONFIG(32, 128, 1, 4, 4, 1, 0.f, 0.f, "igemm_split_32x128"),
     MC_CONFIG(64, 128, 2, 2, 3, 1, 0.f, 0.f, "igemm_split_64x128"),
     MC_CONFIG(64, 64, 2, 2, 3, 2, 0.21f, 0.8f, "igemm_split_64x64x32"),
+    MC_SMALL(4, "igemm_split_32x32_k4"),
+    MC_SMALL(8, "igemm_split_32x32_k8"),
 };
 #undef MC_CONFIG
+#undef MC_SMALL
 constexpr int kNumSplitConfigs = sizeof(kSplitConfigs) / sizeof(kSplitConfigs[0]);
 
