@@ -328,6 +328,17 @@ int mcProposalRest(const float* scores, const float* bbox, const float* im_info,
                    int A, int H, int W, int feat_stride, float min_size, int pre_nms_topn,
                    int post_nms_topn, float nms_thresh, void* workspace, size_t workspace_bytes,
                    float* rois, float* roi_scores, int* num_rois, int* state, void* stream);
+/* What mcProposal queues behind step 1, for a caller of mcProposalHead that found
+ * state[1] = 0: same arguments, and the workspace as mcProposalHead left it.  Where only the
+ * order of equal scores among the best 512 proposals was open, SortBBox is replayed through
+ * the partitions that hold them and the scan repeated; otherwise (and when that does not
+ * settle the result) as mcProposalRest.  Always ends with state[1] = 1.  No counterpart in the
+ * reference. */
+int mcProposalContinue(const float* scores, const float* bbox, const float* im_info, const float* anchors,
+                       int A, int H, int W, int feat_stride, float min_size, int pre_nms_topn,
+                       int post_nms_topn, float nms_thresh, void* workspace, size_t workspace_bytes,
+                       float* rois, float* roi_scores, int* num_rois, int* state, void* stream);
+
 
 /* Measurement hook (no counterpart in the reference): while enabled on the calling
  * thread every mcProposal* call records HIP events between its stages on the launch

@@ -154,14 +154,16 @@ __global__ __launch_bounds__(256) void proposal_order_gather_kernel(
 // the result as complete.
 constexpr int kHeadWant = 512;                        // = kScanRows, one super-block of the scan
 constexpr int kHeadThreads = kSortThreads;
-constexpr int kHeadPer = 44;                          // keys per thread
-constexpr int kHeadMaxN = kHeadPer * kHeadThreads;    // 22528 proposals
+// keys per thread: for tables of up to 22 528 and up to 36 864 proposals
+constexpr int kHeadPer = 44, kHeadPerLarge = 72;
+constexpr int kHeadMaxN = kHeadPerLarge * kHeadThreads;
 
 // info[0] = number of ordered entries m >= want (the keys at or below the want-th smallest),
 // 0 when the head could not be ordered here (more candidates than the kernel holds: equal
 // scores in crowds; the full-size path takes over).  out_keys / out_order[0 .. m): (key
 // ascending = score descending, index ascending); the boxes and scores of the first
 // `want` of them go to sorted_boxes / sorted_scores.
+template <int PER>
 __global__ __launch_bounds__(kHeadThreads) void proposal_head_kernel(
     const uint32_t* __restrict__ keys, int n, int want, uint32_t* __restrict__ out_keys,
     int* __restrict__ out_order, int* __restrict__ info, const float4* __restrict__ boxes,
@@ -171,15 +173,15 @@ __global__ __launch_bounds__(kHeadThreads) void proposal_head_kernel(
   const int tid = threadIdx.x;
   // any thread may hold any key: coalesced loads, key i in thread i % threads (no branches
   // around the loads: all of them are in flight together)
-  uint32_t rk[kHeadPer];
+  uint32_t rk[PER];
 #pragma unroll
-  for (int j = 0; j < kHeadPer; ++j) rk[j] = keys[min(tid + j * kHeadThreads, n - 1)];
+  for (int j = 0; j < PER; ++j) rk[j] = keys[min(tid + j * kHeadThreads, n - 1)];
   __builtin_amdgcn_sched_barrier(0);  // (or each load is waited for before the next is issued)
 #pragma unroll
-  for (int j = 0; j < kHeadPer; ++j)
+  for (int j = 0; j < PER; ++j)
     rk[j] = tid + j * kHeadThreads < n ? min(rk[j], 0xfffffffeu) : 0xffffffffu;  // (all ones: no entry)
   uint32_t key, idx;
-  const int m = block_select_smallest<kHeadPer>(rk, want, &sel, &key, &idx);
+  const int m = block_select_smallest<PER>(rk, want, &sel, &key, &idx);
   if (m == 0) {  // uniform
     if (tid == 0) info[0] = 0;
     return;
@@ -208,31 +210,43 @@ __global__ __launch_bounds__(512) void proposal_head_check_kernel(
     const float4* __restrict__ sorted_boxes, const float* __restrict__ sorted_scores,
     float* __restrict__ rois, float* __restrict__ roi_scores, int* __restrict__ state) {
   __shared__ unsigned char alive[kHeadWant];
-  __shared__ int s_need;
+  __shared__ int s_need, s_members;
+  __shared__ unsigned short s_kept[kHeadWant];
+  __shared__ uint32_t s_member[kHeadWant];  // (first of the group << 16) | member
   const int z = threadIdx.x;
   const int m = info[0];
   const int count = *num_kept;
-  if (z == 0) s_need = (m == 0 || flags[2] == 0) ? 1 : 0;
+  const bool reached = m != 0 && flags[2] != 0;
+  if (z == 0) s_need = reached ? 0 : 1;
   // the last candidate the scan examined
   const int last = count >= max_keep ? kept[max_keep - 1] : want - 1;
   bool member = false;
   int first = z;
   if (z < kHeadWant) alive[z] = 0;
+  if (z < count) s_kept[z] = static_cast<unsigned short>(kept[z]);  // (at most kHeadWant)
+  if (z == 0) s_members = 0;
+  __syncthreads();
   if (m > 0 && z < want) {
     const uint32_t k = head_keys[z];
     member = (z > 0 && head_keys[z - 1] == k) || (z + 1 < m && head_keys[z + 1] == k);
     if (member) {
       while (first > 0 && head_keys[first - 1] == k) --first;
-      bool live = true;
-      if (first <= last) {
-        for (int r = 0; r < count && live; ++r) {
-          const int kb = kept[r];
-          if (kb >= first) break;  // kept[] ascends
-          live = !((mask[static_cast<size_t>(kb) * stride + (z >> 6)] >> (z & 63)) & 1ull);
-        }
-      }
-      alive[z] = live ? 1 : 0;
+      alive[z] = 1;
+      if (first <= last)
+        s_member[atomicAdd(&s_members, 1)] = (static_cast<uint32_t>(first) << 16) | static_cast<uint32_t>(z);
     }
+  }
+  __syncthreads();
+  // A member is dead when a kept box before its group suppresses it: a wavefront per member, 64 kept
+  // boxes at a time (by a thread of its own, one kept box after the other, 41 us for a dozen members).
+  for (int k = z >> 6; k < s_members; k += kHeadWant / 64) {
+    const int who = static_cast<int>(s_member[k] & 0xffffu), before = static_cast<int>(s_member[k] >> 16);
+    bool dead = false;
+    for (int r = z & 63; r < count; r += 64) {
+      const int kb = s_kept[r];
+      if (kb < before) dead = dead || ((mask[static_cast<size_t>(kb) * stride + (who >> 6)] >> (who & 63)) & 1ull);
+    }
+    if (__any(dead) && (z & 63) == 0) alive[who] = 0;
   }
   __syncthreads();
   if (member && first == z && z <= last) {
@@ -249,6 +263,8 @@ __global__ __launch_bounds__(512) void proposal_head_check_kernel(
   if (z == 0) {
     flags[3] = complete;
     if (!complete) flags[2] = 0;
+    flags[5] = reached && !complete ? 1 : 0;  // only the order of equal scores is open
+    flags[7] = 1;                             // (tie_head_kernel clears it)
     if (state != nullptr) {  // (the step was called by itself)
       state[0] = 0;
       state[1] = complete;
@@ -724,9 +740,13 @@ constexpr int kFastChunksPerWave = (kFastChunks + kFastWaves - 1) / kFastWaves;
 constexpr int kFastRegChunks = 8;         // chunks per wavefront whose moved places wait in registers
 constexpr int kFastMaxLong = kFastMaxN / kFastWaveSeg + 2;
 
-struct FastLds {
-  uint32_t kv[kFastMaxN];                 // (dense rank << 16) | original index, by place
-  unsigned short tab[kFastMaxN + 2];      // rank -> place: smaller scores up from lo + 1,
+// KV: what a place holds, its rank or key in the upper half and the original index in the lower 16
+// bits; N places.
+template <typename KV, int N>
+struct FastLdsOf {
+  typedef KV Entry;
+  KV kv[N];                               // (dense rank << 16) | original index, by place
+  unsigned short tab[N + 2];              // rank -> place: smaller scores up from lo + 1,
                                           // larger scores down from hi
   unsigned long long ms[kFastChunks], mb[kFastChunks];  // ballots of the workgroup path
   uint32_t cpre[kFastChunks + 1];         // exclusive chunk prefix (smaller low, larger high half)
@@ -738,6 +758,12 @@ struct FastLds {
   int n_pairs;
   int n_seg[2], n_long[2], moved_s, moved_b, failed;
 };
+typedef FastLdsOf<uint32_t, kFastMaxN> FastLds;
+
+__device__ __forceinline__ uint32_t fast_rank(uint32_t kv) { return kv >> 16; }
+__device__ __forceinline__ uint32_t fast_rank(unsigned long long kv) { return static_cast<uint32_t>(kv >> 32); }
+__device__ __forceinline__ int fast_index(uint32_t kv) { return static_cast<int>(kv & 0xffffu); }
+__device__ __forceinline__ int fast_index(unsigned long long kv) { return static_cast<int>(kv & 0xffffu); }
 
 // Per-place step shared by both paths.  (ms, mb): ballots of the place's chunk, (ps, pb):
 // smaller / larger scores in the chunks before it.  Returns true when the place moves.
@@ -777,18 +803,21 @@ __device__ __forceinline__ bool fast_move(const FastSeg& g, const unsigned short
 }
 
 // Pairs of equal neighbours (j, j + 1) of the sorted keys with j < x (counted for j < num_top).
-__device__ __forceinline__ int fast_pairs_before(const FastLds* s, int x) {
+template <typename Lds>
+__device__ __forceinline__ int fast_pairs_before(const Lds* s, int x) {
   const int w = x >> 6;
   return s->pair_pre[w] + __popcll(s->pair_bits[w] & ((1ull << (x & 63)) - 1ull));
 }
 // True when such a pair touches the sorted places [a, b]: some j in [a - 1, b].
-__device__ __forceinline__ bool fast_touched(const FastLds* s, int a, int b) {
+template <typename Lds>
+__device__ __forceinline__ bool fast_touched(const Lds* s, int a, int b) {
   return fast_pairs_before(s, b + 1) - fast_pairs_before(s, max(a - 1, 0)) > 0;
 }
 
 // After the moves of a partition: place the pivot, close or queue the two children.
 // Called by one thread.
-__device__ __forceinline__ void fast_finish(FastLds* s, const FastSeg& g, uint32_t pivot, int u,
+template <typename Lds>
+__device__ __forceinline__ void fast_finish(Lds* s, const FastSeg& g, typename Lds::Entry pivot, int u,
                                             int t, int num_top, int* __restrict__ order_out,
                                             int next) {
   const int h = t == 0 ? g.lo : (t > u ? s->tab[g.hi + 1 - t] : s->tab[g.lo + u]);
@@ -797,14 +826,14 @@ __device__ __forceinline__ void fast_finish(FastLds* s, const FastSeg& g, uint32
     return;
   }
   s->kv[h] = pivot;
-  if (h < num_top) order_out[h] = static_cast<int>(pivot & 0xffffu);
+  if (h < num_top) order_out[h] = fast_index(pivot);
 #pragma unroll
   for (int side = 0; side < 2; ++side) {
     const int a = side == 0 ? g.lo : h + 1, b = side == 0 ? h - 1 : g.hi;
     if (a > b) continue;
     if (side == 1 && a >= num_top) continue;  // the reference does not sort past num_top
     if (a == b) {
-      if (a < num_top) order_out[a] = static_cast<int>(s->kv[a] & 0xffffu);
+      if (a < num_top) order_out[a] = fast_index(s->kv[a]);
       continue;
     }
     if (fast_touched(s, a, b)) {
@@ -850,6 +879,364 @@ __device__ __forceinline__ uint32_t fast_chunk_scan(FastLds* s, int C, int lane)
     run += cnt[j];
   }
   return __shfl(inc, 63, 64);
+}
+
+// A partition of at most 64 places and everything below it, by one wavefront in registers: lane l
+// holds place lo + l, the tables of the i-th smaller and larger score are lane permutations,
+// and the sub-partitions still open wait in the lanes of `stack`.  (Level by level through LDS each
+// of them costs 2 to 5 us, here about 0.4.)
+template <typename Lds>
+__device__ __forceinline__ void fast_small(const Lds* s, int lo, int hi, int num_top,
+                                           int* __restrict__ order_out) {
+  const int lane = threadIdx.x & 63;
+  const int len = hi - lo + 1;
+  typedef typename Lds::Entry KV;
+  KV kv = s->kv[min(lo + lane, hi)];
+  // bit x: sorted places lo - 1 + x and lo + x are a pair of equal scores; one more bit for x = 64
+  unsigned long long pairs;
+  {
+    const int from = max(lo - 1, 0), w = from >> 6, sh = from & 63;
+    pairs = s->pair_bits[w] >> sh;
+    if (sh) pairs |= s->pair_bits[w + 1] << (64 - sh);
+    if (lo == 0) pairs <<= 1;
+  }
+  const bool pair_last = len == 64 && ((s->pair_bits[hi >> 6] >> (hi & 63)) & 1ull);
+  // [a, b] in lanes holds or borders on a pair: bits a .. b + 1
+  auto touched = [&](int a, int b) {
+    const unsigned long long upto = b + 1 >= 63 ? ~0ull : (1ull << (b + 2)) - 1ull;
+    return ((pairs & upto) >> a) != 0 || (b == 63 && pair_last);
+  };
+  auto done = [&](int place) {  // the lane that holds `place` has its final score
+    if (lane == place && lo + place < num_top) order_out[lo + place] = fast_index(kv);
+  };
+  const unsigned long long lt = (1ull << lane) - 1ull;
+  int stack = 0, depth = 0;
+  int a = 0, b = len - 1;
+  for (int steps = 0; steps < 64; ++steps) {  // (every step places a pivot)
+    const KV pivot = __shfl(kv, a, 64);
+    const uint32_t K = fast_rank(pivot), d = fast_rank(kv);
+    const bool in = lane > a && lane <= b;
+    const bool is_s = in && d > K, is_b = in && d < K;
+    const unsigned long long ms = __ballot(is_s), mb = __ballot(is_b);
+    const int nB = __popcll(mb);
+    bool left = false, right = false;
+    int h = a;
+    if (ms == 0 && mb == 0) {  // all equal: nothing moves
+      if (lane >= a && lane <= b && lo + lane < num_top) order_out[lo + lane] = fast_index(kv);
+    } else {
+      // 1-based ranks: smaller from the left, larger from the right; slot 0 takes what is neither
+      const int rs = is_s ? __popcll(ms & lt) + 1 : 0, rb = is_b ? __popcll(mb & ~lt) : 0;
+      const int L = __builtin_amdgcn_ds_permute(rs * 4, lane), R = __builtin_amdgcn_ds_permute(rb * 4, lane);
+      const int r0 = __shfl(R, rs, 64), r1 = __shfl(R, min(rs + 1, 63), 64), l0 = __shfl(L, rb, 64);
+      const int u = __popcll(__ballot(is_s && rs <= nB && r0 > lane));
+      const int t = __popcll(__ballot(is_s && rs + 1 <= nB && r1 > lane)) + (nB >= 1 ? 1 : 0);
+      const int first_b = __builtin_amdgcn_readlane(R, 1);
+      h = t == 0 ? a : (t > u ? __builtin_amdgcn_readlane(R, t) : __builtin_amdgcn_readlane(L, u));
+      int from = lane;
+      if (lane == a && t >= 1) from = first_b;
+      if (is_s && rs + 1 <= t && rs <= u) from = r1;
+      if (is_b && rb <= u && rb <= t) from = l0;
+      kv = __shfl(kv, from, 64);
+      if (lane == h) kv = pivot;
+      done(h);
+      if (h - 1 == a) done(a);
+      else left = h - 1 > a && touched(a, h - 1);
+      if (lo + h + 1 < num_top) {  // the reference does not sort past num_top
+        if (h + 1 == b) done(b);
+        else right = h + 1 < b && touched(h + 1, b);
+      }
+    }
+    if (left && right) {
+      if (lane == depth) stack = ((h + 1) << 8) | b;
+      ++depth;
+    }
+    if (left) {
+      b = h - 1;
+    } else if (right) {
+      a = h + 1;
+    } else {
+      if (depth == 0) return;
+      --depth;
+      const int e = __builtin_amdgcn_readlane(stack, depth);
+      a = e >> 8;
+      b = e & 255;
+    }
+  }
+}
+
+// Replays the open partitions listed in `s` (level 0) down to the last one, places below num_top
+// only; the places that become final go to `order`.  True when that succeeded.
+template <typename Lds>
+__device__ __forceinline__ bool fast_levels(Lds& s, int n, int num_top, uint2* __restrict__ stage,
+                                            int* __restrict__ order) {
+  typedef typename Lds::Entry KV;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // Every level shortens every open partition by at least its pivot: at most n levels.
+  int n_cur = s.n_seg[0], n_cur_long = s.n_long[0], cur = 0, levels_left = n + 1;
+  __syncthreads();
+  while (n_cur + n_cur_long > 0 && levels_left-- > 0) {
+    const int next = cur ^ 1;
+    // ---- long partitions: the whole workgroup, one after the other ----
+    // Every wavefront takes a run of consecutive chunks, so that the counts before a
+    // chunk are the wavefront's running sums on top of the totals of the wavefronts
+    // before it; ballots are taken again in every pass instead of being stored.
+    for (int si = 0; si < n_cur_long; ++si) {
+      const uint32_t sg = s.seg_long[cur][si];
+      FastSeg g;
+      g.lo = static_cast<int>(sg >> 16);
+      g.hi = static_cast<int>(sg & 0xffffu);
+      const KV pivot = s.kv[g.lo];
+      const uint32_t K = fast_rank(pivot);
+      const int places = g.hi - g.lo;  // without the pivot
+      const int C = (places + 63) >> 6;
+      const int Cw = (C + kFastWaves - 1) / kFastWaves;
+      const int c_begin = min(wave * Cw, C), c_end = min(c_begin + Cw, C);
+      if (tid == 0) {
+        s.moved_s = 0;
+        s.moved_b = 0;
+      }
+      {
+        int cs = 0, cb = 0;
+        for (int c = c_begin; c < c_end; ++c) {
+          const int q = g.lo + 1 + (c << 6) + lane;
+          const uint32_t d = q <= g.hi ? fast_rank(s.kv[q]) : K;
+          cs += __popcll(__ballot(d > K));  // larger rank = smaller score
+          cb += __popcll(__ballot(d < K));
+        }
+        if (lane == 0) s.wave_cnt[wave] = static_cast<uint32_t>(cs) | (static_cast<uint32_t>(cb) << 16);
+      }
+      __syncthreads();
+      uint32_t before = 0, total = 0;
+#pragma unroll
+      for (int w = 0; w < kFastWaves; ++w) {
+        const uint32_t v = s.wave_cnt[w];
+        before += w < wave ? v : 0u;
+        total += v;
+      }
+      g.nS = static_cast<int>(total & 0xffffu);
+      g.nB = static_cast<int>(total >> 16);
+      if (g.nS == 0 && g.nB == 0) {
+        // every score equals the pivot's: nothing ever moves in here
+        for (int q = g.lo + tid; q <= g.hi && q < num_top; q += kFastThreads)
+          order[q] = fast_index(s.kv[q]);
+        __syncthreads();  // wave_cnt is reused by the next partition
+        continue;
+      }
+      {
+        int ps = static_cast<int>(before & 0xffffu), pb = static_cast<int>(before >> 16);
+        for (int c = c_begin; c < c_end; ++c) {
+          const int q = g.lo + 1 + (c << 6) + lane;
+          const uint32_t d = q <= g.hi ? fast_rank(s.kv[q]) : K;
+          const unsigned long long ms = __ballot(d > K), mb = __ballot(d < K);
+          bool is_s, is_b;
+          int rank;
+          fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
+          if (is_s) s.tab[g.lo + rank] = static_cast<unsigned short>(q);
+          if (is_b) s.tab[g.hi + 1 - rank] = static_cast<unsigned short>(q);
+          ps += __popcll(ms);
+          pb += __popcll(mb);
+        }
+      }
+      __syncthreads();
+      // A moved place is read by its own lane and written to its destination after
+      // every read of the partition is done.  Up to kFastRegChunks chunks per wavefront
+      // it waits in registers, in longer partitions (the first few levels) in `stage`.
+      int u = 0, t = 0;
+      int ps = static_cast<int>(before & 0xffffu), pb = static_cast<int>(before >> 16);
+      if (Cw <= kFastRegChunks) {
+        KV keep_kv[kFastRegChunks];
+        int keep_to[kFastRegChunks];
+#pragma unroll
+        for (int k = 0; k < kFastRegChunks; ++k) {
+          const int c = c_begin + k;
+          keep_to[k] = -1;
+          if (c < c_end) {
+            const int q = g.lo + 1 + (c << 6) + lane;
+            const KV mine = q <= g.hi ? s.kv[q] : pivot;
+            const uint32_t d = fast_rank(mine);
+            const unsigned long long ms = __ballot(d > K), mb = __ballot(d < K);
+            bool is_s, is_b;
+            int rank, dest = 0;
+            fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
+            const bool mv = fast_move(g, s.tab, q, is_s, is_b, rank, &dest);
+            if (mv) {
+              keep_to[k] = dest;
+              keep_kv[k] = mine;
+            }
+            u += __popcll(__ballot(mv && is_s));
+            t += __popcll(__ballot(mv && is_b));
+            ps += __popcll(ms);
+            pb += __popcll(mb);
+          }
+        }
+        if (lane == 0) {
+          if (u) atomicAdd(&s.moved_s, u);
+          if (t) atomicAdd(&s.moved_b, t);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kFastRegChunks; ++k)
+          if (keep_to[k] >= 0) s.kv[keep_to[k]] = keep_kv[k];
+      } else {
+        for (int c = c_begin; c < c_end; ++c) {
+          const int q = g.lo + 1 + (c << 6) + lane;
+          const KV mine = q <= g.hi ? s.kv[q] : pivot;
+          const uint32_t d = fast_rank(mine);
+          const unsigned long long ms = __ballot(d > K), mb = __ballot(d < K);
+          bool is_s, is_b;
+          int rank, dest = 0;
+          fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
+          const bool mv = fast_move(g, s.tab, q, is_s, is_b, rank, &dest);
+          if (q <= g.hi) stage[q] = make_uint2(mv ? static_cast<uint32_t>(mine) : 0u, mv ? static_cast<uint32_t>(dest) : 0xffffffffu);
+          u += __popcll(__ballot(mv && is_s));
+          t += __popcll(__ballot(mv && is_b));
+          ps += __popcll(ms);
+          pb += __popcll(mb);
+        }
+        if (lane == 0) {
+          if (u) atomicAdd(&s.moved_s, u);
+          if (t) atomicAdd(&s.moved_b, t);
+        }
+        __syncthreads();
+        // every lane reads back what it staged itself, four loads in flight
+        for (int c0 = c_begin; c0 < c_end; c0 += 4) {
+          uint2 e[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int q = g.lo + 1 + ((c0 + j) << 6) + lane;
+            e[j] = (c0 + j < c_end && q <= g.hi) ? stage[q] : make_uint2(0u, 0xffffffffu);
+          }
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (e[j].y != 0xffffffffu) s.kv[e[j].y] = e[j].x;
+        }
+      }
+      __syncthreads();
+      // One thread places the pivot and queues the children while the others go on to
+      // the next partition: it touches the rank table and places of this partition
+      // only, and the counters it reads are reset by itself.
+      if (tid == 0) fast_finish(&s, g, pivot, s.moved_s, s.moved_b, num_top, order, next);
+    }
+    // ---- short partitions: one wavefront each ----
+    for (int si = wave; si < n_cur; si += kFastWaves) {
+      const uint32_t sg = s.seg[cur][si];
+      FastSeg g;
+      g.lo = static_cast<int>(__builtin_amdgcn_readfirstlane(sg >> 16));
+      g.hi = static_cast<int>(__builtin_amdgcn_readfirstlane(sg & 0xffffu));
+      if (g.hi - g.lo < 64) {
+        fast_small(&s, g.lo, g.hi, num_top, order);
+        continue;
+      }
+      const KV pivot = s.kv[g.lo];
+      const uint32_t K = fast_rank(pivot);
+      const int places = g.hi - g.lo;
+      const int C = (places + 63) >> 6;
+      // The wavefront walks the chunks in order, so the counts before a chunk are running
+      // sums and nothing but the rank table is stored; the ballots are taken again in
+      // every pass (one LDS read and two compares).
+      g.nS = 0;
+      g.nB = 0;
+      for (int c = 0; c < C; ++c) {
+        const int q = g.lo + 1 + (c << 6) + lane;
+        const uint32_t d = q <= g.hi ? fast_rank(s.kv[q]) : K;
+        g.nS += __popcll(__ballot(d > K));
+        g.nB += __popcll(__ballot(d < K));
+      }
+      if (g.nS == 0 && g.nB == 0) {
+        for (int q = g.lo + lane; q <= g.hi && q < num_top; q += 64)
+          order[q] = fast_index(s.kv[q]);
+        continue;
+      }
+      int ps = 0, pb = 0;
+      for (int c = 0; c < C; ++c) {
+        const int q = g.lo + 1 + (c << 6) + lane;
+        const uint32_t d = q <= g.hi ? fast_rank(s.kv[q]) : K;
+        const unsigned long long ms = __ballot(d > K), mb = __ballot(d < K);
+        bool is_s, is_b;
+        int rank;
+        fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
+        if (is_s) s.tab[g.lo + rank] = static_cast<unsigned short>(q);
+        if (is_b) s.tab[g.hi + 1 - rank] = static_cast<unsigned short>(q);
+        ps += __popcll(ms);
+        pb += __popcll(mb);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      int u = 0, t = 0;
+      ps = 0;
+      pb = 0;
+      if (C <= kFastRegChunks) {
+        KV keep_kv[kFastRegChunks];
+        int keep_to[kFastRegChunks];
+#pragma unroll
+        for (int c = 0; c < kFastRegChunks; ++c) {
+          keep_to[c] = -1;
+          if (c < C) {
+            const int q = g.lo + 1 + (c << 6) + lane;
+            const KV mine = q <= g.hi ? s.kv[q] : pivot;
+            const uint32_t d = fast_rank(mine);
+            const unsigned long long ms = __ballot(d > K), mb = __ballot(d < K);
+            bool is_s, is_b;
+            int rank, dest = 0;
+            fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
+            const bool mv = fast_move(g, s.tab, q, is_s, is_b, rank, &dest);
+            if (mv) {
+              keep_to[c] = dest;
+              keep_kv[c] = mine;
+            }
+            u += __popcll(__ballot(mv && is_s));
+            t += __popcll(__ballot(mv && is_b));
+            ps += __popcll(ms);
+            pb += __popcll(mb);
+          }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int c = 0; c < kFastRegChunks; ++c)
+          if (keep_to[c] >= 0) s.kv[keep_to[c]] = keep_kv[c];
+      } else {
+        for (int c = 0; c < C; ++c) {
+          const int q = g.lo + 1 + (c << 6) + lane;
+          const KV mine = q <= g.hi ? s.kv[q] : pivot;
+          const uint32_t d = fast_rank(mine);
+          const unsigned long long ms = __ballot(d > K), mb = __ballot(d < K);
+          bool is_s, is_b;
+          int rank, dest = 0;
+          fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
+          const bool mv = fast_move(g, s.tab, q, is_s, is_b, rank, &dest);
+          if (q <= g.hi) stage[q] = make_uint2(mv ? static_cast<uint32_t>(mine) : 0u, mv ? static_cast<uint32_t>(dest) : 0xffffffffu);
+          u += __popcll(__ballot(mv && is_s));
+          t += __popcll(__ballot(mv && is_b));
+          ps += __popcll(ms);
+          pb += __popcll(mb);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        // every lane reads back what it staged itself, four loads in flight
+        for (int c0 = 0; c0 < C; c0 += 4) {
+          uint2 e[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int q = g.lo + 1 + ((c0 + j) << 6) + lane;
+            e[j] = q <= g.hi ? stage[q] : make_uint2(0u, 0xffffffffu);
+          }
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (e[j].y != 0xffffffffu) s.kv[e[j].y] = e[j].x;
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (lane == 0) fast_finish(&s, g, pivot, u, t, num_top, order, next);
+    }
+    __syncthreads();
+    n_cur = s.failed ? 0 : min(s.n_seg[next], kFastMaxSegs);
+    n_cur_long = s.failed ? 0 : min(s.n_long[next], kFastMaxLong);
+    if (tid == 0) {  // the lists that were just walked receive the level after next
+      s.n_seg[cur] = 0;
+      s.n_long[cur] = 0;
+    }
+    cur = next;
+    __syncthreads();
+  }
+  return n_cur + n_cur_long == 0 && !s.failed;
 }
 
 __global__ __launch_bounds__(kFastThreads) void tie_replay_fast_kernel(
@@ -907,272 +1294,297 @@ __global__ __launch_bounds__(kFastThreads) void tie_replay_fast_kernel(
     }
   }
   __syncthreads();
-
-  // Every level shortens every open partition by at least its pivot: at most n levels.
-  int n_cur = s.n_seg[0], n_cur_long = s.n_long[0], cur = 0, levels_left = n + 1;
-  __syncthreads();
-  while (n_cur + n_cur_long > 0 && levels_left-- > 0) {
-    const int next = cur ^ 1;
-    // ---- long partitions: the whole workgroup, one after the other ----
-    // Every wavefront takes a run of consecutive chunks, so that the counts before a
-    // chunk are the wavefront's running sums on top of the totals of the wavefronts
-    // before it; ballots are taken again in every pass instead of being stored.
-    for (int si = 0; si < n_cur_long; ++si) {
-      const uint32_t sg = s.seg_long[cur][si];
-      FastSeg g;
-      g.lo = static_cast<int>(sg >> 16);
-      g.hi = static_cast<int>(sg & 0xffffu);
-      const uint32_t pivot = s.kv[g.lo];
-      const uint32_t K = pivot >> 16;
-      const int places = g.hi - g.lo;  // without the pivot
-      const int C = (places + 63) >> 6;
-      const int Cw = (C + kFastWaves - 1) / kFastWaves;
-      const int c_begin = min(wave * Cw, C), c_end = min(c_begin + Cw, C);
-      if (tid == 0) {
-        s.moved_s = 0;
-        s.moved_b = 0;
-      }
-      {
-        int cs = 0, cb = 0;
-        for (int c = c_begin; c < c_end; ++c) {
-          const int q = g.lo + 1 + (c << 6) + lane;
-          const uint32_t d = q <= g.hi ? s.kv[q] >> 16 : K;
-          cs += __popcll(__ballot(d > K));  // larger rank = smaller score
-          cb += __popcll(__ballot(d < K));
-        }
-        if (lane == 0) s.wave_cnt[wave] = static_cast<uint32_t>(cs) | (static_cast<uint32_t>(cb) << 16);
-      }
-      __syncthreads();
-      uint32_t before = 0, total = 0;
-#pragma unroll
-      for (int w = 0; w < kFastWaves; ++w) {
-        const uint32_t v = s.wave_cnt[w];
-        before += w < wave ? v : 0u;
-        total += v;
-      }
-      g.nS = static_cast<int>(total & 0xffffu);
-      g.nB = static_cast<int>(total >> 16);
-      if (g.nS == 0 && g.nB == 0) {
-        // every score equals the pivot's: nothing ever moves in here
-        for (int q = g.lo + tid; q <= g.hi && q < num_top; q += kFastThreads)
-          order[q] = static_cast<int>(s.kv[q] & 0xffffu);
-        __syncthreads();  // wave_cnt is reused by the next partition
-        continue;
-      }
-      {
-        int ps = static_cast<int>(before & 0xffffu), pb = static_cast<int>(before >> 16);
-        for (int c = c_begin; c < c_end; ++c) {
-          const int q = g.lo + 1 + (c << 6) + lane;
-          const uint32_t d = q <= g.hi ? s.kv[q] >> 16 : K;
-          const unsigned long long ms = __ballot(d > K), mb = __ballot(d < K);
-          bool is_s, is_b;
-          int rank;
-          fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
-          if (is_s) s.tab[g.lo + rank] = static_cast<unsigned short>(q);
-          if (is_b) s.tab[g.hi + 1 - rank] = static_cast<unsigned short>(q);
-          ps += __popcll(ms);
-          pb += __popcll(mb);
-        }
-      }
-      __syncthreads();
-      // A moved place is read by its own lane and written to its destination after
-      // every read of the partition is done.  Up to kFastRegChunks chunks per wavefront
-      // it waits in registers, in longer partitions (the first few levels) in `stage`.
-      int u = 0, t = 0;
-      int ps = static_cast<int>(before & 0xffffu), pb = static_cast<int>(before >> 16);
-      if (Cw <= kFastRegChunks) {
-        uint32_t keep_kv[kFastRegChunks];
-        int keep_to[kFastRegChunks];
-#pragma unroll
-        for (int k = 0; k < kFastRegChunks; ++k) {
-          const int c = c_begin + k;
-          keep_to[k] = -1;
-          if (c < c_end) {
-            const int q = g.lo + 1 + (c << 6) + lane;
-            const uint32_t mine = q <= g.hi ? s.kv[q] : pivot;
-            const uint32_t d = mine >> 16;
-            const unsigned long long ms = __ballot(d > K), mb = __ballot(d < K);
-            bool is_s, is_b;
-            int rank, dest = 0;
-            fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
-            const bool mv = fast_move(g, s.tab, q, is_s, is_b, rank, &dest);
-            if (mv) {
-              keep_to[k] = dest;
-              keep_kv[k] = mine;
-            }
-            u += __popcll(__ballot(mv && is_s));
-            t += __popcll(__ballot(mv && is_b));
-            ps += __popcll(ms);
-            pb += __popcll(mb);
-          }
-        }
-        if (lane == 0) {
-          if (u) atomicAdd(&s.moved_s, u);
-          if (t) atomicAdd(&s.moved_b, t);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < kFastRegChunks; ++k)
-          if (keep_to[k] >= 0) s.kv[keep_to[k]] = keep_kv[k];
-      } else {
-        for (int c = c_begin; c < c_end; ++c) {
-          const int q = g.lo + 1 + (c << 6) + lane;
-          const uint32_t mine = q <= g.hi ? s.kv[q] : pivot;
-          const uint32_t d = mine >> 16;
-          const unsigned long long ms = __ballot(d > K), mb = __ballot(d < K);
-          bool is_s, is_b;
-          int rank, dest = 0;
-          fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
-          const bool mv = fast_move(g, s.tab, q, is_s, is_b, rank, &dest);
-          if (q <= g.hi) stage[q] = make_uint2(mv ? mine : 0u, mv ? static_cast<uint32_t>(dest) : 0xffffffffu);
-          u += __popcll(__ballot(mv && is_s));
-          t += __popcll(__ballot(mv && is_b));
-          ps += __popcll(ms);
-          pb += __popcll(mb);
-        }
-        if (lane == 0) {
-          if (u) atomicAdd(&s.moved_s, u);
-          if (t) atomicAdd(&s.moved_b, t);
-        }
-        __syncthreads();
-        // every lane reads back what it staged itself, four loads in flight
-        for (int c0 = c_begin; c0 < c_end; c0 += 4) {
-          uint2 e[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int q = g.lo + 1 + ((c0 + j) << 6) + lane;
-            e[j] = (c0 + j < c_end && q <= g.hi) ? stage[q] : make_uint2(0u, 0xffffffffu);
-          }
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (e[j].y != 0xffffffffu) s.kv[e[j].y] = e[j].x;
-        }
-      }
-      __syncthreads();
-      // One thread places the pivot and queues the children while the others go on to
-      // the next partition: it touches the rank table and places of this partition
-      // only, and the counters it reads are reset by itself.
-      if (tid == 0) fast_finish(&s, g, pivot, s.moved_s, s.moved_b, num_top, order, next);
-    }
-    // ---- short partitions: one wavefront each ----
-    for (int si = wave; si < n_cur; si += kFastWaves) {
-      const uint32_t sg = s.seg[cur][si];
-      FastSeg g;
-      g.lo = static_cast<int>(sg >> 16);
-      g.hi = static_cast<int>(sg & 0xffffu);
-      const uint32_t pivot = s.kv[g.lo];
-      const uint32_t K = pivot >> 16;
-      const int places = g.hi - g.lo;
-      const int C = (places + 63) >> 6;
-      // The wavefront walks the chunks in order, so the counts before a chunk are running
-      // sums and nothing but the rank table is stored; the ballots are taken again in
-      // every pass (one LDS read and two compares).
-      g.nS = 0;
-      g.nB = 0;
-      for (int c = 0; c < C; ++c) {
-        const int q = g.lo + 1 + (c << 6) + lane;
-        const uint32_t d = q <= g.hi ? s.kv[q] >> 16 : K;
-        g.nS += __popcll(__ballot(d > K));
-        g.nB += __popcll(__ballot(d < K));
-      }
-      if (g.nS == 0 && g.nB == 0) {
-        for (int q = g.lo + lane; q <= g.hi && q < num_top; q += 64)
-          order[q] = static_cast<int>(s.kv[q] & 0xffffu);
-        continue;
-      }
-      int ps = 0, pb = 0;
-      for (int c = 0; c < C; ++c) {
-        const int q = g.lo + 1 + (c << 6) + lane;
-        const uint32_t d = q <= g.hi ? s.kv[q] >> 16 : K;
-        const unsigned long long ms = __ballot(d > K), mb = __ballot(d < K);
-        bool is_s, is_b;
-        int rank;
-        fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
-        if (is_s) s.tab[g.lo + rank] = static_cast<unsigned short>(q);
-        if (is_b) s.tab[g.hi + 1 - rank] = static_cast<unsigned short>(q);
-        ps += __popcll(ms);
-        pb += __popcll(mb);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      int u = 0, t = 0;
-      ps = 0;
-      pb = 0;
-      if (C <= kFastRegChunks) {
-        uint32_t keep_kv[kFastRegChunks];
-        int keep_to[kFastRegChunks];
-#pragma unroll
-        for (int c = 0; c < kFastRegChunks; ++c) {
-          keep_to[c] = -1;
-          if (c < C) {
-            const int q = g.lo + 1 + (c << 6) + lane;
-            const uint32_t mine = q <= g.hi ? s.kv[q] : pivot;
-            const uint32_t d = mine >> 16;
-            const unsigned long long ms = __ballot(d > K), mb = __ballot(d < K);
-            bool is_s, is_b;
-            int rank, dest = 0;
-            fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
-            const bool mv = fast_move(g, s.tab, q, is_s, is_b, rank, &dest);
-            if (mv) {
-              keep_to[c] = dest;
-              keep_kv[c] = mine;
-            }
-            u += __popcll(__ballot(mv && is_s));
-            t += __popcll(__ballot(mv && is_b));
-            ps += __popcll(ms);
-            pb += __popcll(mb);
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-        for (int c = 0; c < kFastRegChunks; ++c)
-          if (keep_to[c] >= 0) s.kv[keep_to[c]] = keep_kv[c];
-      } else {
-        for (int c = 0; c < C; ++c) {
-          const int q = g.lo + 1 + (c << 6) + lane;
-          const uint32_t mine = q <= g.hi ? s.kv[q] : pivot;
-          const uint32_t d = mine >> 16;
-          const unsigned long long ms = __ballot(d > K), mb = __ballot(d < K);
-          bool is_s, is_b;
-          int rank, dest = 0;
-          fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
-          const bool mv = fast_move(g, s.tab, q, is_s, is_b, rank, &dest);
-          if (q <= g.hi) stage[q] = make_uint2(mv ? mine : 0u, mv ? static_cast<uint32_t>(dest) : 0xffffffffu);
-          u += __popcll(__ballot(mv && is_s));
-          t += __popcll(__ballot(mv && is_b));
-          ps += __popcll(ms);
-          pb += __popcll(mb);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        // every lane reads back what it staged itself, four loads in flight
-        for (int c0 = 0; c0 < C; c0 += 4) {
-          uint2 e[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int q = g.lo + 1 + ((c0 + j) << 6) + lane;
-            e[j] = q <= g.hi ? stage[q] : make_uint2(0u, 0xffffffffu);
-          }
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (e[j].y != 0xffffffffu) s.kv[e[j].y] = e[j].x;
-        }
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      if (lane == 0) fast_finish(&s, g, pivot, u, t, num_top, order, next);
-    }
-    __syncthreads();
-    n_cur = s.failed ? 0 : min(s.n_seg[next], kFastMaxSegs);
-    n_cur_long = s.failed ? 0 : min(s.n_long[next], kFastMaxLong);
-    if (tid == 0) {  // the lists that were just walked receive the level after next
-      s.n_seg[cur] = 0;
-      s.n_long[cur] = 0;
-    }
-    cur = next;
-    __syncthreads();
-  }
-  if (tid == 0 && n_cur + n_cur_long == 0 && !s.failed) {
+  const bool ok = fast_levels(s, n, num_top, stage, order);
+  if (tid == 0 && ok) {
     flag[1] = 1;
     flag[0] = 3;  // reported to the caller: equal scores, order replayed by this kernel
   }
+}
+
+// ---- equal scores among the best 512 proposals only --------------------------------
+//
+// When the head of the table settles everything but the order of a few of its own equal
+// scores, only the partitions that hold one of those pairs matter, and these lie at the
+// front: every level has at most one long partition to follow (a pivot of rank 512 and
+// more leaves the places before it, a smaller one the places behind it and a short rest).  So
+// neither the table's sorted order nor dense ranks of all scores are needed.  One
+// workgroup keeps the whole table on chip, the keys by place in registers (place 64 c + lane in
+// wavefront c % 16), the original indices and the table of larger scores in LDS, and only
+// the elements that change places inside the followed partition move.  From 1024 places
+// on fast_levels goes on.  What bounds it: one CU's instruction issue in the
+// five passes over the partition per level (10 us for the first levels of 21 546 proposals, three to
+// nine levels), then the dependent levels below 1024 places (25 to 50 us).  21 546 proposals with two to
+// eight pairs among the best 512: 126 us on the average, where sorting the whole table and
+// replaying all its equal scores takes 81 + 205; 33 696 proposals, whose replay walked every
+// partition through memory: mcProposal 1500 -> 205 us.
+constexpr int kTieThreads = 1024, kTieWaves = kTieThreads / 64;
+// keys per thread, for the two sizes of table that the head takes
+constexpr int kTieSlots = kHeadPer / 2, kTieSlotsLarge = kHeadPerLarge / 2;
+static_assert(kTieThreads == 2 * kHeadThreads, "half as many keys per thread");
+constexpr int kTieStop = 1024;
+constexpr int kTieLevels = 64;                      // more (nearly sorted tables) are left to the full-size path
+static_assert(kTieThreads == kFastThreads, "fast_levels is for the same workgroup");
+
+template <int SLOTS>
+struct TieChainLds {
+  unsigned short idx[SLOTS * kTieThreads];   // original index, by place
+  unsigned short big[SLOTS * kTieThreads];   // place of the i-th larger score from the right, i from 0
+  uint32_t cnt[SLOTS * kTieWaves];       // chunks of 64 places: smaller (low half) / larger scores: of a chunk, then before it
+  unsigned short small_idx[kHeadWant];   // index at the i-th smaller score from the left
+  uint32_t pivot, total;
+  int u, t, last;
+};
+
+template <int SLOTS>
+__global__ __launch_bounds__(kTieThreads) void tie_head_kernel(
+    const uint32_t* __restrict__ keys, int n, int want, const uint32_t* __restrict__ head_keys,
+    int* __restrict__ order, const float4* __restrict__ boxes, const float* __restrict__ scores,
+    float4* __restrict__ sorted_boxes, float* __restrict__ sorted_scores, int* __restrict__ flags) {
+  if (flags[3] != 0 || flags[5] == 0) return;  // uniform
+  __shared__ __attribute__((aligned(16))) union {
+    TieChainLds<SLOTS> chain;
+    FastLdsOf<unsigned long long, 2 * kTieThreads> fast;  // (whole keys: no dense ranks to find)
+  } lds;
+  __shared__ unsigned long long pairs[kHeadWant / 64];  // bit j: sorted places j and j + 1 are equal
+  __shared__ uint32_t pending[kTieLevels + 1];          // short partitions left behind (lo << 16 | hi)
+  TieChainLds<SLOTS>& s = lds.chain;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  auto below = [](unsigned long long m) {  // bits of lower lanes
+    return static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(m >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(m), 0u)));
+  };
+  const int m = flags[4];  // places of the head that are ordered, `want` and more
+  if (wave < kHeadWant / 64) {
+    const bool eq = tid < want && tid + 1 < m && head_keys[tid] == head_keys[tid + 1];
+    const unsigned long long b = __ballot(eq);
+    if (lane == 0) pairs[wave] = b;
+  }
+  uint32_t key[SLOTS];
+#pragma unroll
+  for (int j = 0; j < SLOTS; ++j) key[j] = keys[min(((j * kTieWaves + wave) << 6) + lane, n - 1)];
+  __builtin_amdgcn_sched_barrier(0);  // (or each load is waited for before the next is issued)
+#pragma unroll
+  for (int j = 0; j < SLOTS; ++j) {
+    const int q = ((j * kTieWaves + wave) << 6) + lane;
+    s.idx[q] = static_cast<unsigned short>(q);
+  }
+  __syncthreads();
+  // True when a pair of the head touches the sorted places [a, b]: some j in [a - 1, b].
+  auto touched = [&](int a, int b) {
+    const int from = max(a - 1, 0), to = min(b, want - 1);
+    bool any = false;
+#pragma unroll
+    for (int w = 0; w < kHeadWant / 64; ++w) {
+      const int f = from - 64 * w, l = to - 64 * w;  // bits f .. l of word w
+      if (l < 0 || f > 63) continue;
+      const unsigned long long upto = l >= 63 ? ~0ull : (1ull << (l + 1)) - 1ull;
+      const unsigned long long below = f <= 0 ? 0ull : (1ull << f) - 1ull;
+      any = any || (pairs[w] & upto & ~below) != 0;
+    }
+    return any;
+  };
+
+  // All of what follows is uniform over the workgroup except the elements themselves.
+  int lo = 0, hi = n - 1, n_pending = 0, level = 0;
+  bool open = n >= 2;
+  while (open && hi - lo + 1 > kTieStop) {
+    if (++level > kTieLevels) return;
+    const int c_first = lo >> 6, c_last = hi >> 6;
+#pragma unroll
+    for (int j = 0; j < SLOTS; ++j)
+      if (((j * kTieWaves + wave) << 6) + lane == lo) s.pivot = key[j];
+    if (tid == 0) {
+      s.u = s.t = 0;
+      s.last = -1;
+    }
+    __syncthreads();
+    const uint32_t P = s.pivot;
+    const unsigned short pivot_idx = s.idx[lo];
+  // (the thread's first place is hidden from the compiler, which otherwise keeps the places and LDS
+  // addresses of all slots in registers, and spills)
+#define MC_EACH_CHUNK                                           \
+  int q0 = tid;                                                 \
+  asm volatile("" : "+v"(q0));                                  \
+  const int c0 = __builtin_amdgcn_readfirstlane(q0 >> 6);       \
+  _Pragma("unroll") for (int j = 0; j < SLOTS; ++j) {           \
+    const int c = c0 + j * kTieWaves;                           \
+    if (c < c_first || c > c_last) continue;                    \
+    const int q = q0 + j * kTieThreads;                         \
+    const bool in = static_cast<unsigned>(q - lo - 1) < static_cast<unsigned>(hi - lo); \
+    const bool is_s = in && key[j] > P, is_b = in && key[j] < P;
+#define MC_END_CHUNK __builtin_amdgcn_sched_barrier(0); }
+    {
+    MC_EACH_CHUNK
+      const uint32_t packed = static_cast<uint32_t>(__popcll(__ballot(is_s))) |
+                              (static_cast<uint32_t>(__popcll(__ballot(is_b))) << 16);
+      if (lane == 0) s.cnt[c] = packed;
+    MC_END_CHUNK
+    }
+    __syncthreads();
+    if (wave == 0) {  // counts before each chunk
+      constexpr int kRun = (SLOTS * kTieWaves + 63) / 64;
+      uint32_t cnt[kRun], sum = 0;
+#pragma unroll
+      for (int k = 0; k < kRun; ++k) {
+        const int c = lane * kRun + k;
+        cnt[k] = c >= c_first && c <= c_last ? s.cnt[c] : 0u;
+        sum += cnt[k];
+      }
+      uint32_t inc = sum;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t up = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += up;
+      }
+      uint32_t run = inc - sum;
+#pragma unroll
+      for (int k = 0; k < kRun; ++k) {
+        const int c = lane * kRun + k;
+        if (c >= c_first && c <= c_last) s.cnt[c] = run;
+        run += cnt[k];
+      }
+      if (lane == 63) s.total = inc;
+    }
+    __syncthreads();
+    const int nS = static_cast<int>(s.total & 0xffffu), nB = static_cast<int>(s.total >> 16);
+    if (nS == 0 && nB == 0) {  // every score equals the pivot's: nothing moves in here
+      for (int q = lo + tid; q <= hi && q < want; q += kTieThreads) order[q] = s.idx[q];
+      open = false;
+      break;
+    }
+    {
+    MC_EACH_CHUNK
+      const unsigned long long mb = __ballot(is_b);
+      const int rank = nB - (static_cast<int>(s.cnt[c] >> 16) + below(mb));  // (its own bit not counted)
+      if (is_b) s.big[rank - 1] = static_cast<unsigned short>(q);
+      (void)is_s;
+    MC_END_CHUNK
+    }
+    __syncthreads();
+    {
+      // of the smaller scores: how many change places with a larger one (u), how many take the next
+      // larger one in (t, with the first, which goes to the pivot's place), the last that moves
+      int u = 0, t = 0, last = -1;
+      MC_EACH_CHUNK
+        const unsigned long long ms = __ballot(is_s);
+        const int i = static_cast<int>(s.cnt[c] & 0xffffu) + below(ms) + 1;
+        const bool moves = is_s && i <= nB && s.big[i - 1] > q;
+        const bool takes = is_s && i + 1 <= nB && s.big[i] > q;
+        const unsigned long long mv = __ballot(moves);
+        u += __popcll(mv);
+        t += __popcll(__ballot(takes));
+        if (mv != 0) last = (c << 6) + 63 - __clzll(static_cast<long long>(mv));
+        (void)is_b;
+      MC_END_CHUNK
+      if (lane == 0) {
+        if (u) atomicAdd(&s.u, u);
+        if (t) atomicAdd(&s.t, t);
+        if (last >= 0) atomicMax(&s.last, last);
+      }
+    }
+    __syncthreads();
+    const int u = s.u, t = s.t + (nB >= 1 ? 1 : 0);
+    const int h = t == 0 ? lo : (t > u ? s.big[t - 1] : s.last);
+    if ((t != u && t != u + 1) || h < lo || h > hi) return;  // cannot happen; the full-size path redoes the job
+    const bool left = h - 1 > lo && touched(lo, h - 1), left_one = h - 1 == lo;
+    const bool right = h + 1 < hi && h + 1 < want && touched(h + 1, hi), right_one = h + 1 == hi && h + 1 < want;
+    if (right || right_one) {
+      // (u <= h - lo < want: the places before the pivot's)
+      MC_EACH_CHUNK
+        const unsigned long long ms = __ballot(is_s);
+        const int i = static_cast<int>(s.cnt[c] & 0xffffu) + below(ms) + 1;
+        if (is_s && i <= u) s.small_idx[i - 1] = s.idx[q];
+        (void)is_b;
+      MC_END_CHUNK
+    }
+    // the places before h: a smaller score's is taken by the next larger one from the right,
+    // which stands at h or behind it
+    if (left || left_one) {
+      MC_EACH_CHUNK
+        const unsigned long long ms = __ballot(is_s);
+        const int i = static_cast<int>(s.cnt[c] & 0xffffu) + below(ms) + 1;
+        const bool first = q == lo;
+        if (q < h && ((first && t >= 1) || (is_s && i + 1 <= t))) {
+          const unsigned short from = s.idx[s.big[first ? 0 : i]];
+          key[j] = keys[from];
+          // (a smaller score's old index is still wanted for small_idx by its own lane only, above)
+          s.idx[q] = from;
+        }
+        (void)is_b;
+      MC_END_CHUNK
+    }
+    __syncthreads();
+    // the places behind h: a larger score's is taken by the smaller one of its rank.  (These are the u
+    // first larger scores from the right; counted from h on, because the places before it have
+    // new scores by now.)
+    if (right || right_one) {
+      MC_EACH_CHUNK
+        const unsigned long long mb = __ballot(is_b && q > h);
+        const int before = c == (h >> 6) ? 0 : static_cast<int>(s.cnt[c] >> 16) - (nB - u);
+        const int i = u - (before + below(mb));
+        if (is_b && q > h && i >= 1 && i <= u) {
+          const unsigned short from = s.small_idx[i - 1];
+          key[j] = keys[from];
+          s.idx[q] = from;
+        }
+        (void)is_s;
+      MC_END_CHUNK
+    }
+    __syncthreads();
+    if (tid == 0) {
+      s.idx[h] = pivot_idx;
+      if (h < want) order[h] = pivot_idx;
+      if (left_one && lo < want) order[lo] = s.idx[lo];
+      if (right_one) order[h + 1] = s.idx[h + 1];
+      if (left && right) pending[n_pending] = (static_cast<uint32_t>(lo) << 16) | static_cast<uint32_t>(h - 1);
+    }
+    if (left && right) ++n_pending;
+    if (right) lo = h + 1;
+    else if (left) hi = h - 1;
+    else open = false;
+    __syncthreads();
+  }
+#undef MC_EACH_CHUNK
+#undef MC_END_CHUNK
+  __syncthreads();
+  // What is left lies before place m2: the partitions left behind and the last one.
+  int m2 = open ? hi + 1 : 0;
+  for (int k = 0; k < n_pending; ++k) m2 = max(m2, static_cast<int>(pending[k] & 0xffffu) + 1);
+  if (m2 > 2 * kTieThreads) return;  // cannot happen: fewer than 512 places before one of at most kTieStop
+  if (m2 > 0) {
+    // (slots 0 and 1 hold places tid and 1024 + tid)
+    const uint32_t k0 = key[0], k1 = key[1];
+    const uint32_t i0 = s.idx[tid], i1 = s.idx[kTieThreads + tid];
+    __syncthreads();
+    auto& f = lds.fast;
+    f.kv[tid] = (static_cast<unsigned long long>(k0) << 32) | i0;
+    f.kv[kTieThreads + tid] = (static_cast<unsigned long long>(k1) << 32) | i1;
+    if (tid < 2 * kTieThreads / 64 + 2) {
+      f.pair_bits[tid] = tid < kHeadWant / 64 ? pairs[tid] : 0ull;
+      int before = 0;
+      for (int w = 0; w < min(tid, kHeadWant / 64); ++w) before += __popcll(pairs[w]);
+      f.pair_pre[tid] = static_cast<unsigned short>(before);
+    }
+    if (tid == 0) {
+      f.n_seg[0] = f.n_seg[1] = f.n_long[0] = f.n_long[1] = 0;
+      f.failed = 0;
+      for (int k = 0; k <= n_pending; ++k) {
+        if (k == n_pending && !open) break;
+        const uint32_t e = k < n_pending ? pending[k] : (static_cast<uint32_t>(lo) << 16) | static_cast<uint32_t>(hi);
+        if (static_cast<int>((e & 0xffffu) - (e >> 16)) + 1 > kFastWaveSeg) f.seg_long[0][f.n_long[0]++] = e;
+        else f.seg[0][f.n_seg[0]++] = e;
+      }
+    }
+    __syncthreads();
+    if (!fast_levels(f, m2, want, nullptr, order)) return;  // uniform
+  }
+  __syncthreads();
+  if (tid < want) {  // want <= 512
+    const int o = order[tid];
+    sorted_boxes[tid] = boxes[o];
+    sorted_scores[tid] = scores[o];
+  }
+  if (tid == 0) flags[7] = 0;
 }
 
 // mask[i][cb] bit j: box cb*64+j (> i) overlaps box i by more than thr, with
@@ -1278,10 +1690,11 @@ __device__ inline unsigned long long wave_uniform(unsigned long long v) {
 __global__ __launch_bounds__(kScanThreads) void nms_scan_kernel(
     const unsigned long long* __restrict__ mask, int n, int nb, int stride, int max_keep,
     int* __restrict__ kept, int* __restrict__ num_kept, int* __restrict__ done, int final_part,
-    int resume, const unsigned long long* __restrict__ colmask) {
+    int resume, const unsigned long long* __restrict__ colmask, const int* __restrict__ skip = nullptr,
+    int* __restrict__ complete = nullptr) {
   extern __shared__ unsigned long long removed[];  // nb words
   __shared__ unsigned long long subcol[kScanRows];  // colmask of the super-block's boxes
-  if (done != nullptr && *done != 0) return;  // uniform
+  if ((done != nullptr && *done != 0) || (skip != nullptr && *skip != 0)) return;  // uniform
   __shared__ unsigned long long sub[kScanRows * kScanBlocks];
   __shared__ int sb_kept[kScanRows];
   __shared__ int s_count, s_ns;
@@ -1440,7 +1853,10 @@ __global__ __launch_bounds__(kScanThreads) void nms_scan_kernel(
   }
   if (tid == 0) {
     *num_kept = s_count;
-    if (done != nullptr && (final_part || s_count >= max_keep)) *done = 1;
+    if (done != nullptr && (final_part || s_count >= max_keep)) {
+      *done = 1;
+      if (complete != nullptr) *complete = 2;  // settled by the head with its equal scores in order
+    }
   }
 }
 
@@ -1453,10 +1869,10 @@ __global__ void proposal_gather_kernel(const float4* __restrict__ sorted_boxes,
                                        int* __restrict__ state, int state_ints) {
   // what the caller learns: state[0] = which equal-score replay ran, state[1] = the result is final
   if (state != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
-    state[0] = flags[0];
+    state[0] = flags[3] == 2 ? 3 : flags[0];
     if (state_ints > 1) state[1] = 1;
   }
-  if (flags[3] != 0) return;  // the head step wrote the rows
+  if (flags[3] == 1) return;  // the head step wrote the rows
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= *num_kept) return;
   const float4 b = sorted_boxes[kept[r]];
@@ -1566,7 +1982,9 @@ int static_scratch(void** out) {
 
 // Steps of run_proposal: the head of the table alone, the full-size path alone, or both
 // (the second then skips itself on the device when the first one settled the result).
-constexpr int kStepHead = 1, kStepRest = 2;
+// Between the two, where the head is there to start from: its equal scores in the
+// reference's order, and its scan again.
+constexpr int kStepHead = 1, kStepRest = 2, kStepTies = 4;
 
 // state (device, optional): [0] which equal-score replay ran (0 none, 1 general, 3 few
 // ties), [1] 1 when rois / num_rois are final.
@@ -1599,6 +2017,8 @@ int run_proposal(int steps, const float* scores, const float* bbox, const float*
   float* sscores = reinterpret_cast<float*>(ws + L.sorted_scores);
   unsigned long long* mask = reinterpret_cast<unsigned long long*>(ws + L.mask);
   int* kept = reinterpret_cast<int*>(ws + L.kept);
+  // flags: [3] is 2 and [0] stays 0 when the head settled the result with its equal scores
+  // replayed; [5] only their order is open, [7] the head's second scan has nothing to do.
   // flags: [0] equal scores among the first pre + 1 sorted places (| 2: the few-ties replay
   // took them), [1] few-ties replay done, [2] the scan settled the result, [3] the head of
   // the table settled it (the full-size path skips itself), [4] entries the head ordered
@@ -1621,17 +2041,19 @@ int run_proposal(int steps, const float* scores, const float* bbox, const float*
   };
   MC_HIP(mark(0));
   // foreground scores are the second half of the score blob (proposal_layer.cpp:295)
-  proposal_decode_kernel<<<ceil_div(n, 256), 256, 0, st>>>(scores + n, bbox, anchors, im_info, A, H,
-                                                          W, feat_stride, min_size, boxes, k0,
-                                                          korig, v0, sc, flags);
-  MC_LAUNCH_CHECK();
+  if (steps != (kStepTies | kStepRest)) {  // (those go on from the head step)
+    proposal_decode_kernel<<<ceil_div(n, 256), 256, 0, st>>>(scores + n, bbox, anchors, im_info, A, H,
+                                                            W, feat_stride, min_size, boxes, k0,
+                                                            korig, v0, sc, flags);
+    MC_LAUNCH_CHECK();
+  }
   // The head can settle the result only if post_nms_topn kept boxes fit it (or it is the
   // whole table).
   const bool head_possible = n <= kHeadMaxN && (post_nms_topn < kHeadWant || pre <= kHeadWant);
+  const int want = pre < kHeadWant ? pre : kHeadWant, head_nb = ceil_div(want, 64);
   if ((steps & kStepHead) && head_possible) {
-    const int want = pre < kHeadWant ? pre : kHeadWant, head_nb = ceil_div(want, 64);
-    proposal_head_kernel<<<1, kHeadThreads, 0, st>>>(korig, n, want, k1, v1, head_info, boxes, sc,
-                                                     sboxes, sscores);
+    auto head_kernel = n <= kHeadPer * kHeadThreads ? proposal_head_kernel<kHeadPer> : proposal_head_kernel<kHeadPerLarge>;
+    head_kernel<<<1, kHeadThreads, 0, st>>>(korig, n, want, k1, v1, head_info, boxes, sc, sboxes, sscores);
     MC_LAUNCH_CHECK();
     MC_HIP(mark(1));
     nms_mask_kernel<<<head_nb * (head_nb + 1) / 2, 256, 0, st>>>(sboxes, want, nms_thresh, nb, head_nb,
@@ -1648,6 +2070,18 @@ int run_proposal(int steps, const float* scores, const float* bbox, const float*
     MC_HIP(mark(1));
   }
   MC_HIP(mark(2));
+  const bool ties = (steps & kStepTies) && head_possible;
+  if (ties && !g_force_general_replay) {
+    auto tie_kernel = n <= kTieSlots * kTieThreads ? tie_head_kernel<kTieSlots> : tie_head_kernel<kTieSlotsLarge>;
+    tie_kernel<<<1, kTieThreads, 0, st>>>(korig, n, want, k1, v1, boxes, sc, sboxes, sscores, flags);
+    MC_LAUNCH_CHECK();
+    nms_mask_kernel<<<head_nb * (head_nb + 1) / 2, 256, 0, st>>>(sboxes, want, nms_thresh, nb, head_nb,
+                                                               mask, colmask, flags + 7);
+    MC_LAUNCH_CHECK();
+    nms_scan_kernel<<<1, kScanThreads, sizeof(unsigned long long) * head_nb, st>>>(
+        mask, want, head_nb, nb, post_nms_topn, kept, num_rois, done, want == pre, 0, colmask, flags + 7, complete);
+    MC_LAUNCH_CHECK();
+  }
   if (steps & kStepRest) {
     if (n <= kSortLdsMax)
       proposal_sort_lds_kernel<<<1, kSortThreads, 0, st>>>(k0, v0, n, pre, flags, complete);
@@ -1674,21 +2108,24 @@ int run_proposal(int steps, const float* scores, const float* bbox, const float*
     // candidate: first the best kScanRows candidates among themselves (a corner of the
     // overlap matrix, one super-block of the scan).  If that settles the result the
     // full-size launches behind it return at once; otherwise they fill the whole matrix and
-    // the scan resumes behind the first super-block.  (`done` is also set when the head
-    // step was complete: all four launches return at once then.)
-    const int head = pre < kScanRows ? pre : kScanRows, head_nb = ceil_div(head, 64);
-    nms_mask_kernel<<<head_nb * (head_nb + 1) / 2, 256, 0, st>>>(sboxes, head, nms_thresh, nb, head_nb, mask,
-                                                               colmask, done);
-    MC_LAUNCH_CHECK();
-    nms_scan_kernel<<<1, kScanThreads, sizeof(unsigned long long) * head_nb, st>>>(
-        mask, head, head_nb, nb, post_nms_topn, kept, num_rois, done, head == pre, 0, colmask);
-    MC_LAUNCH_CHECK();
-    if (head < pre) {
+    // the scan resumes behind the first super-block.  Where the head step has already tried
+    // the corner, the full size comes at once.  (`done` is also set when the head was complete: all
+    // return at once then.)
+    const int head = pre < kScanRows ? pre : kScanRows, corner_nb = ceil_div(head, 64);
+    if (!ties) {
+      nms_mask_kernel<<<corner_nb * (corner_nb + 1) / 2, 256, 0, st>>>(sboxes, head, nms_thresh, nb, corner_nb, mask,
+                                                                     colmask, done);
+      MC_LAUNCH_CHECK();
+      nms_scan_kernel<<<1, kScanThreads, sizeof(unsigned long long) * corner_nb, st>>>(
+          mask, head, corner_nb, nb, post_nms_topn, kept, num_rois, done, head == pre, 0, colmask);
+      MC_LAUNCH_CHECK();
+    }
+    if (ties || head < pre) {
       nms_mask_kernel<<<std::min(nb * (nb + 1) / 2, 8 * kNumCu), 256, 0, st>>>(sboxes, pre, nms_thresh, nb, nb,
                                                                              mask, colmask, done);
       MC_LAUNCH_CHECK();
       nms_scan_kernel<<<1, kScanThreads, sizeof(unsigned long long) * nb, st>>>(
-          mask, pre, nb, nb, post_nms_topn, kept, num_rois, done, 1, 1, colmask);
+          mask, pre, nb, nb, post_nms_topn, kept, num_rois, done, 1, ties ? 0 : 1, colmask);
       MC_LAUNCH_CHECK();
     }
     proposal_gather_kernel<<<ceil_div(post_nms_topn, 256), 256, 0, st>>>(
@@ -1727,7 +2164,7 @@ int mcProposal(const float* scores, const float* bbox, const float* im_info, con
                int A, int H, int W, int feat_stride, float min_size, int pre_nms_topn,
                int post_nms_topn, float nms_thresh, void* workspace, size_t workspace_bytes,
                float* rois, float* roi_scores, int* num_rois, int* tie_flag, void* stream) {
-  return run_proposal(kStepHead | kStepRest, scores, bbox, im_info, anchors, A, H, W, feat_stride,
+  return run_proposal(kStepHead | kStepTies | kStepRest, scores, bbox, im_info, anchors, A, H, W, feat_stride,
                       min_size, pre_nms_topn, post_nms_topn, nms_thresh, workspace, workspace_bytes,
                       rois, roi_scores, num_rois, tie_flag, 1, stream);
 }
@@ -1747,6 +2184,15 @@ int mcProposalRest(const float* scores, const float* bbox, const float* im_info,
                    int post_nms_topn, float nms_thresh, void* workspace, size_t workspace_bytes,
                    float* rois, float* roi_scores, int* num_rois, int* state, void* stream) {
   return run_proposal(kStepRest, scores, bbox, im_info, anchors, A, H, W, feat_stride, min_size,
+                      pre_nms_topn, post_nms_topn, nms_thresh, workspace, workspace_bytes, rois,
+                      roi_scores, num_rois, state, 2, stream);
+}
+
+int mcProposalContinue(const float* scores, const float* bbox, const float* im_info, const float* anchors,
+                       int A, int H, int W, int feat_stride, float min_size, int pre_nms_topn,
+                       int post_nms_topn, float nms_thresh, void* workspace, size_t workspace_bytes,
+                       float* rois, float* roi_scores, int* num_rois, int* state, void* stream) {
+  return run_proposal(kStepTies | kStepRest, scores, bbox, im_info, anchors, A, H, W, feat_stride, min_size,
                       pre_nms_topn, post_nms_topn, nms_thresh, workspace, workspace_bytes, rois,
                       roi_scores, num_rois, state, 2, stream);
 }
@@ -1796,7 +2242,7 @@ int mcProposalStatic(const float* scores, const float* bbox, const float* im_inf
              need, kStaticScratchBytes);
   void* ws = nullptr;
   if (static_scratch(&ws) != 0) return -1;
-  return run_proposal(kStepHead | kStepRest, scores, bbox, im_info, anchors, A, H, W, feat_stride,
+  return run_proposal(kStepHead | kStepTies | kStepRest, scores, bbox, im_info, anchors, A, H, W, feat_stride,
                       min_size, pre_nms_topn, post_nms_topn, nms_thresh, ws, kStaticScratchBytes, rois,
                       roi_scores, num_rois, tie_flag, 1, stream);
 }

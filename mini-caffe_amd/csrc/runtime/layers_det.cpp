@@ -89,7 +89,7 @@ class ProposalLayer : public Layer {
     int num_rois = 0;
     for (int step = 0; step < 2; ++step) {
       int* counters = counters_.mutable_gpu_data();
-      MC_CHECK((step == 0 ? mcProposalHead : mcProposalRest)(
+      MC_CHECK((step == 0 ? mcProposalHead : mcProposalContinue)(
           bottom[0]->gpu_data(), bottom[1]->gpu_data(), bottom[2]->gpu_data(), anchors_.gpu_data(), A,
           H, W, feat_stride_, static_cast<float>(min_size_), pre_nms_topn_, post_nms_topn_,
           nms_thresh_, workspace_.mutable_gpu_data(), bytes, top[0]->mutable_gpu_data(),

@@ -88,6 +88,7 @@ LIB.mcProposal.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,
                            c_void_p, c_void_p, c_void_p, c_void_p]
 LIB.mcProposalHead.argtypes = LIB.mcProposal.argtypes
 LIB.mcProposalRest.argtypes = LIB.mcProposal.argtypes
+LIB.mcProposalContinue.argtypes = LIB.mcProposal.argtypes
 LIB.mcProposalTimingEnable.argtypes = [c_int]
 LIB.mcProposalForceGeneralReplay.argtypes = [c_int]
 LIB.mcProposalTimingCollect.argtypes = [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(c_long)]

@@ -1,0 +1,86 @@
+"""Proposal where only the order of equal scores among the best 512 proposals is open.
+
+mcProposal and mcProposalHead + mcProposalContinue replay the reference's quicksort through the partitions
+that hold those scores only; the rows equal the CPU path's bit for bit.  Tables up to the
+largest that the head takes, runs of equal scores, scores in an order that makes the quicksort follow the
+short or the long side, few candidates, and a result that the head cannot settle after all.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def K(gpu_mode):
+    from minicaffe import kernels
+    return kernels
+
+
+def run(K, scores, bbox, im_info, pre, post, steps):
+    A, H, W = 9, scores.shape[2], scores.shape[3]
+    size = ctypes.c_size_t()
+    K.check_mc(K.LIB.mcProposalWorkspaceSize(A * H * W, pre, post, ctypes.byref(size)))
+    ws = torch.full((size.value,), 255, dtype=torch.uint8, device="cuda")
+    t = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (scores, bbox, im_info, oracle.generate_anchors().astype(np.float32))]
+    rois, rs = torch.full((post, 5), float("nan"), device="cuda"), torch.zeros(post, device="cuda")
+    cnt = torch.zeros(3, dtype=torch.int32, device="cuda")
+
+    def call(fn):
+        K.check_mc(fn(*[x.data_ptr() for x in t], A, H, W, 16, 16.0, pre, post, 0.7, ws.data_ptr(), size.value,
+                      rois.data_ptr(), rs.data_ptr(), cnt.data_ptr(), cnt.data_ptr() + 4, None))
+        torch.cuda.synchronize()
+    if not steps:
+        call(K.LIB.mcProposal)
+    else:
+        call(K.LIB.mcProposalHead)
+        if int(cnt[2].item()) == 0:
+            call(K.LIB.mcProposalContinue)
+            assert int(cnt[2].item()) == 1
+    n = int(cnt[0].item())
+    return rois[:n].cpu().numpy(), rs[:n].cpu().numpy(), int(cnt[1].item())
+
+
+@pytest.mark.parametrize("hw,pre,post,order", [
+    ((38, 63), 6000, 300, "random"), ((20, 20), 6000, 200, "random"), ((12, 10), 6000, 150, "random"),   # 1080 places
+    ((11, 9), 6000, 100, "random"),                         # 891: no long partition at all
+    ((6, 5), 300, 100, "random"), ((38, 63), 400, 150, "random"),
+    ((40, 63), 6000, 300, "random"),                        # 22 680: the larger selection
+    ((64, 64), 6000, 300, "random"),                        # 36 864: the largest table
+    ((64, 65), 6000, 300, "random"),                        # beyond it: the full-size path
+    ((38, 63), 6000, 300, "worst first"), ((38, 63), 6000, 300, "best first"), ((38, 63), 6000, 300, "waves"),
+    ((38, 63), 6000, 511, "random")])                       # hardly settled by 512 candidates
+@pytest.mark.parametrize("seed", range(4))
+def test_rows_equal_the_reference(K, hw, pre, post, order, seed):
+    rng = np.random.default_rng(40 + seed)
+    A, (H, W) = 9, hw
+    n = A * H * W
+    fg = rng.permutation(n).astype(np.float32) / n * 0.9 + 0.05
+    if order == "worst first":
+        fg[:40] = np.sort(fg[:40])
+    elif order == "best first":        # pivots of small rank: short rests before the followed partition
+        top = np.argsort(-fg)[:60]
+        fg[:60], fg[top] = fg[top].copy(), fg[:60].copy()
+    elif order == "waves":
+        fg = (0.05 + 0.9 * np.abs(np.sin(np.arange(n) * 0.37 + seed))).astype(np.float32)
+    best = np.argsort(-fg, kind="stable")
+    head = min(512, n, pre)
+    for k in range(1 + 3 * seed):      # pairs and runs, neighbours in order or not, one at the head's end
+        at = int(rng.integers(0, head - 6))
+        fg[best[at:at + int(rng.integers(2, 6))]] = fg[best[at]]
+    if seed == 3:
+        fg[rng.choice(best[:head], 2, replace=False)] = fg[best[head // 2]]
+    scores = rng.random((1, 2 * A, H, W)).astype(np.float32)
+    scores[0, A:] = fg.reshape(H, W, A).transpose(2, 0, 1)
+    bbox = (rng.standard_normal((1, 4 * A, H, W)) * 0.2).astype(np.float32)
+    im_info = np.array([H * 16, W * 16, 1.0], np.float32)
+    want_rois, want_scores = oracle.proposal({"pre_nms_topn": pre, "post_nms_topn": post, "nms_thresh": 0.7}, scores, bbox,
+                                             im_info, 2)
+    for steps in (False, True):
+        rois, rs, _ = run(K, scores, bbox, im_info, pre, post, steps)
+        assert np.array_equal(rois, want_rois) and np.array_equal(rs, want_scores), steps
