@@ -882,7 +882,9 @@ bool fits_small(const mcConvPlan* plan, const std::vector<const SubProblem*>& li
          (s.Kpad + BK) * plane < (1L << 27) && (long)s.Kpad * plan->Mpad * 6 < (1L << 31) &&
          (s.pointwise || s.Kpad / BK <= kSmallMaxTiles);
 }
-LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const SubProblem*>& live, int num) {
+// (forced_split: as in the plan, 0 = choose.)
+LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const SubProblem*>& live, int num,
+                               int forced_split) {
   LaunchChoice best = {3, 1};
   double best_us = 1e30;
   int least = 1;
@@ -907,7 +909,7 @@ LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const S
     const double stages = blocks > 0 ? static_cast<double>(tile_stages) / blocks : 0.;  // of a tile, on average
     int first = std::min<int>(ceil_div(least, cfg.chains), min_kt);
     int last = std::max(first, std::min(24, min_kt * cfg.ks / 4));
-    if (plan->forced_split >= 1) first = last = std::min(plan->forced_split, std::max(min_kt, 1));
+    if (forced_split >= 1) first = last = std::min(forced_split, std::max(min_kt, 1));
     for (int s = first; s <= last; ++s) {
       const double rounds = ceil_div(blocks * s, kNumCu);
       // few wavefronts to hide the gather's latency (and that of the tap table, if any)
@@ -923,11 +925,14 @@ LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const S
   }
   if (!small_ok || (forced >= 0 && forced < kNumConfigs)) return best;
   // The small-launch kernel, whose time is a fixed part, the longer of a wavefront's K tiles one
-  // after the other and a CU's share of all of them, and what slices cost.  The constants fit
-  // 1400 launches of 105 layers (10 % rms: 3x3 and 5x5 1 us of taps; strided bottoms 1.75
-  // times the gather); the tiles above take 3 us more than their estimate.  Taken where it is ahead by
-  // more than the estimates' error: over those layers 1648 us, always the best kernel and
-  // slices 1611, without this kernel 1939.
+  // after the other and a SIMD's share of all of them, and what slices cost.  The constants fit
+  // 1400 launches of 105 layers (10 % rms; 3x3 and 5x5 0.9 us of taps; strided bottoms 1.7
+  // times the gather; a second workgroup of eight wavefronts finds no room on a CU); the tiles
+  // above take 3 us more than their estimate.  Taken where it is ahead by more than the
+  // estimates' error, and not above 40 K tiles to a SIMD, where the larger tiles read each
+  // operand less often (1024 -> 256 1x1 @14: 8 images, 32 tiles, 12.1 us against 16.6; 12 images, 48
+  // tiles, 17.1 against 16.1; 32 images 35.6 against 28.5).  Over 26 layers of ResNet-50, GoogLeNet
+  // and the SSDs at 1 to 32 images 6.78 ms without this kernel, 6.27 with it.
   best_us = forced >= 0 ? 1e30 : 0.9 * (best_us + 3.0);
   const SubProblem& sub = *live[0];
   const int KT = sub.Kpad / BK;
@@ -937,14 +942,16 @@ LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const S
     if (forced >= 0 && c != forced) continue;
     int first = std::max(1, std::min(ceil_div(least, cfg.chains), KT));
     int last = std::max(first, std::min(16, KT / (2 * cfg.waves)));
-    if (plan->forced_split >= 1) first = last = std::min(plan->forced_split, std::max(KT, 1));
+    if (forced_split >= 1) first = last = std::min(forced_split, std::max(KT, 1));
     for (int s = first; s <= last; ++s) {
       const double wgs = static_cast<double>(tiles) * s;
       const double per_wave = ceil_div(ceil_div(KT, s), cfg.waves);
-      const double share = std::ceil(wgs / kNumCu) * per_wave * cfg.waves * (0.25 / 4) * (sub.q_sw > 1 ? 1.75 : 1.);
-      double us = 3.0 + (sub.pointwise ? 0. : 1.) + std::max(0.31 * per_wave, share) +
-                  wgs / kNumCu * (cfg.waves > 4 ? 1.05 : 0.55);
-      if (s > 1) us += 1.7 + 0.0021 * wgs;
+      const double tiles_per_simd = std::ceil(wgs / kNumCu) * per_wave * cfg.waves / 4;
+      if (forced < 0 && tiles_per_simd > 40) continue;
+      const double share = tiles_per_simd * 0.26 * (sub.q_sw > 1 ? 1.7 : 1.);
+      double us = 2.9 + (sub.pointwise ? 0. : 0.9) + std::max(0.335 * per_wave, share) +
+                  wgs / kNumCu * (cfg.waves > 4 ? 2.6 : 0.61);
+      if (s > 1) us += 1.75 + 0.0021 * wgs;
       if (us < best_us) {
         best_us = us;
         best = {c, s};
@@ -1438,8 +1445,10 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
     max_pixels = std::max(max_pixels, pixels);
   }
   if (live.empty()) return 0;
+  // (a request for one slice means two where there are two tops, see below)
+  const int forced_split = top_second && plan->forced_split == 1 ? 2 : plan->forced_split;
   const LaunchChoice choice =
-      plan->split ? pick_split_launch(plan, live, num) : LaunchChoice{pick_config(plan, max_pixels), 0};
+      plan->split ? pick_split_launch(plan, live, num, forced_split) : LaunchChoice{pick_config(plan, max_pixels), 0};
   const int bm = plan->split ? kSplitConfigs[choice.config].bm : kConfigs[choice.config].bm;
   const int bn = plan->split ? kSplitConfigs[choice.config].bn : kConfigs[choice.config].bn;
   const int stage_kt = plan->split ? kSplitConfigs[choice.config].ks : kConfigs[choice.config].ks;
@@ -1466,12 +1475,8 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
   if (min_kt == (1 << 30)) min_kt = 1;
   // (the per-pixel kernel writes one top only)
   const bool thin = !top_second && use_thin(plan, num);
-  if (!thin && plan->split && kSplitConfigs[choice.config].waves) {
-    LaunchChoice small = choice;
-    // (a request for one slice means two where there are two tops, as below)
-    if (top_second && plan->forced_split == 1) small.slices = 2;
-    return launch_small(plan, *live[0], small, num, bottom, top, ep, st, top_second, c_first);
-  }
+  if (!thin && plan->split && kSplitConfigs[choice.config].waves)
+    return launch_small(plan, *live[0], choice, num, bottom, top, ep, st, top_second, c_first);
   // slices are chosen for the plan as a whole: all sub-problems of a launch run
   // side by side
   // Two tops are told apart by the pass that sums the slices, so such a launch
@@ -1788,7 +1793,7 @@ const char* mcConvPlanKernelName(const mcConvPlan* plan, int num) {
   if (!plan || plan->subs.empty()) return "";
   if (takes_winograd(plan, num)) return "winograd_f32";
   if (use_thin(plan, num)) return "thin_f32";
-  if (plan->split) return kSplitConfigs[pick_split_launch(plan, {&plan->subs[0]}, num).config].name;
+  if (plan->split) return kSplitConfigs[pick_split_launch(plan, {&plan->subs[0]}, num, plan->forced_split).config].name;
   const auto& s = plan->subs[0];
   return kConfigs[pick_config(plan, (long)num * s.Hq * s.Wq)].name;
 }

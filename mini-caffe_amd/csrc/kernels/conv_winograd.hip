@@ -562,8 +562,11 @@ bool winograd_fits(const WinogradState* w, int /*num*/) {
 // direct tile of all, this path still leads on launches that fill the chip: batch 64, 64 -> 64 @56
 // 100.5 us against 98.7 (even), 128 @28 86 / 93, 256 @14 80 / 88, 512 @7 86.5 / 88.7; batch 8, 64 @300
 // 295 / 322, 128 @150 236 / 258, 256 @75 236 / 259, 512 @38 239 / 269, 512 @19 84.6 / 85.8; RPN head
-// 108 / 130.  On smaller ones it no longer does, and the rule below has not followed: batch 8,
-// 64 @56 24.6 us against 21.0, 128 @28 26.0 / 21.8, 256 @14 28.3 / 21.2, 512 @7 37.2 / 23.9.
+// 108 / 130.  On smaller ones it does not.  Tile-rounds of a launch and us, this path against the
+// best direct kernel: 1344 (512 -> 150 @10 b8) 39 / 20, 1568 (64 @56, 128 @28, 256 @14 b8) 25 / 23, 27 / 23,
+// 29 / 22, 1968 (128 -> 192 @24 b9) 30 / 26, 2048 (512 @7 b8) 38 / 25, 2448 (284 -> 214 @46) 32 / 24; 3136 (128
+// @56 b4) 36 / 38, 3888 (64 -> 192 @48 b9) 32 / 42, 4704 (96 @56 b8) 39.5 / 40, 6144 (1024 -> 256 @38) 57 / 63,
+// 6272 (256 @28 b8) 53.5 / 53, 7980 (276 -> 251 @60 b2) 63 / 73, 9600 (1024 -> 150 @19 b8) 71 / 91.
 // What loses: 32 input channels (the loop is four rounds long: 56 / 47 us), an
 // output tile that is half padding (64 -> 32: 86 / 82), and launches of a few tiles,
 // whose time is this kernel's longer prologue and finish (256 -> 150 on 5x5 maps, 9
@@ -578,7 +581,7 @@ bool winograd_pays(const WinogradState* w, int num) {
   // blocks for nine outputs (16 x 4 products against 36 x 9 / 4 useful ones)
   if (10L * w->Ho * w->Wo < 26L * ((w->Ho + 1) / 2) * ((w->Wo + 1) / 2)) return false;
   const long tiles = (long)w->MT * ceil_div(blocks, kTileT);
-  return tiles * (w->KT / 2) >= 1200;
+  return tiles * (w->KT / 2) >= 2800;
 }
 
 int winograd_set_weights(WinogradState* w, const float* weights, hipStream_t st) {

@@ -565,7 +565,7 @@ struct SplitConfig {
   int bm, bn;
   int ks;   // 16-row K tiles per stage
   int occ;  // workgroups per CU the kernel is built for
-  int chains;  // accumulators h h' alternates between
+  int chains;  // accumulators h h' alternates between (small: two per run, the second of a third of it)
   // measured on full launches: a CU's time per 16-row K tile and per tile (prologue and
   // epilogue); 0 = taken on request only
   float stage_us, fixed_us;
@@ -583,7 +583,7 @@ struct SplitConfig {
     igemm_split_kernel<BM, BN, WM, WN, OCC, kModeOneMask, KS>,                \
     igemm_split_kernel<BM, BN, WM, WN, OCC, kModePointwise, KS>}, 0, {nullptr, nullptr, nullptr}}
 #define MC_SMALL(NW, NAME)                                                   \
-  {32, 32, 1, 16 / NW, NW, 0.f, 0.f, NAME, {nullptr, nullptr, nullptr}, NW,  \
+  {32, 32, 1, 16 / NW, 3 * NW / 2, 0.f, 0.f, NAME, {nullptr, nullptr, nullptr}, NW,  \
    {nullptr, igemm_small_kernel<NW, 1, kModeOneMask>, igemm_small_kernel<NW, 1, kModePointwise>}}
 const SplitConfig kSplitConfigs[] = {
     MC_CONFIG(128, 128, 2, 2, 2, 1, 0.56f, 3.3f, "igemm_split_128x128"),
