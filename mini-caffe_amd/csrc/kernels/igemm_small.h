@@ -4,14 +4,21 @@
 // A launch of a few dozen 64x64 tiles (a single image through a classifier, a detector's heads)
 // is a chain of latencies: a K stage's loads, its barrier, and above all the sum of the many
 // slices it takes to occupy the chip, 16 KB of partial sums per slice that the last workgroup
-// of a tile fetches a few slices at a time.  Here a tile is 32 channels x 32 TN pixels and
+// of a tile fetches a few slices at a time.  Here a tile is 32 channels x 32 pixels and
 // each of the NW wavefronts of its workgroup multiplies a run of K tiles of its own: operands
 // go from memory to the registers that the matrix instruction reads, without LDS, without a
 // barrier, DEPTH K tiles ahead; the NW blocks of sums then meet in LDS.  Four times as many
 // tiles and NW runs each occupy the chip with a quarter or less of the slices, and what a
-// slice leaves in memory is 4 TN KB.  The price is that every operand is fetched and split
+// slice leaves in memory is 4 KB.  The price is that every operand is fetched and split
 // by each wavefront that multiplies it (four times the traffic of a 64x64 tile per
 // product), which larger launches do not earn back: see pick_split_launch.
+//
+// What bounds it: on one image the fixed 3 us of a launch (dispatch, arguments, first loads, the
+// meeting of the wavefronts), 0.33 us per K tile of a wavefront, and 2 us where slices are summed.
+// us per launch, the 64x64 tile / this: 64 -> 64 3x3 on one 56x56 map 10.6 / 6.5, 128 -> 128 @28
+// 12.3 / 8.9, 256 -> 256 @14 14.0 / 9.4, 512 -> 512 @7 16.3 / 10.6, 256 -> 1024 1x1 @14 7.9 / 4.5,
+// 1024 -> 256 10.0 / 6.5, 512 -> 2048 @7 8.2 / 5.9, 2048 -> 512 11.3 / 7.8, 512 -> 24 3x3 @10 17.4 / 7.8.
+// Sixteen wavefronts to a workgroup instead of slices: 13.6 us where four slices take 10.3.
 //
 // Lane l of the 32x32x16 product holds K rows 8 (l / 32) .. + 7 of filter row / pixel l % 32: of
 // the packed filter 16 contiguous bytes per plane, of the bottom eight dwords, each
@@ -47,11 +54,12 @@ struct SmallArgs {
   const int4* ktab;
 };
 
-template <int NW, int TN, int MODE>
+template <int NW, int MODE>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 16 ? 4 : 2, 4))) void igemm_small_kernel(
     const SmallArgs a) {
   static_assert(MODE == kModeOneMask || MODE == kModePointwise, "no tap table here");
   constexpr bool PW = MODE == kModePointwise;
+  constexpr int TN = 1;                     // 32-pixel blocks of a tile (two measured no better anywhere)
   constexpr int BN = 32 * TN;
   constexpr int EPT = 32 * BN / (NW * 64);  // sums a thread finishes: consecutive rows of a pixel
   constexpr int DEPTH = 3;                  // K tiles on their way

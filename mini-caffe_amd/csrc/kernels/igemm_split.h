@@ -584,7 +584,7 @@ struct SplitConfig {
     igemm_split_kernel<BM, BN, WM, WN, OCC, kModePointwise, KS>}, 0, {nullptr, nullptr, nullptr}}
 #define MC_SMALL(NW, NAME)                                                   \
   {32, 32, 1, 16 / NW, 3 * NW / 2, 0.f, 0.f, NAME, {nullptr, nullptr, nullptr}, NW,  \
-   {nullptr, igemm_small_kernel<NW, 1, kModeOneMask>, igemm_small_kernel<NW, 1, kModePointwise>}}
+   {nullptr, igemm_small_kernel<NW, kModeOneMask>, igemm_small_kernel<NW, kModePointwise>}}
 const SplitConfig kSplitConfigs[] = {
     MC_CONFIG(128, 128, 2, 2, 2, 1, 0.56f, 3.3f, "igemm_split_128x128"),
     MC_CONFIG(128, 64, 2, 2, 3, 1, 0.363f, 0.9f, "igemm_split_128x64"),
