@@ -28,6 +28,7 @@
 #include "conv_internal.h"
 #include "mc_common.h"
 #include "mchip/kernels.h"
+#include "small_rows.h"
 
 #include <algorithm>
 #include <cstring>
@@ -871,8 +872,8 @@ struct LaunchChoice {
   int config, slices;
 };
 
-// Whether igemm_small_kernel can run the launch: no tap table, and rows past K may be read past
-// the last channel, so that the offsets of a flagged pixel stay below 2^32.
+// Whether igemm_small_kernel can run the launch: no tap table, and the offsets of a flagged
+// pixel, rows past K included, stay below 2^32.
 constexpr int kSmallMaxTiles = 1024;  // 32 KB of taps
 bool fits_small(const mcConvPlan* plan, const std::vector<const SubProblem*>& live, int num) {
   if (plan->force_general || live.size() != 1) return false;
@@ -1380,7 +1381,8 @@ int launch_small(const mcConvPlan* plan, const SubProblem& s, const LaunchChoice
   }
   const bool pointwise = s.pointwise;
   const unsigned taps_lds = pointwise ? 0u : 32u * a.kt_per_slice;
-  cfg.small[pointwise ? kModePointwise : kModeOneMask]<<<static_cast<unsigned>(wgs), 64 * cfg.waves, taps_lds, st>>>(a);
+  const int kernel = !pointwise ? 0 : small_needs_tail(s.K, s.Kpad) ? 2 : 1;
+  cfg.small[kernel]<<<static_cast<unsigned>(wgs), 64 * cfg.waves, taps_lds, st>>>(a);
   MC_LAUNCH_CHECK();
   if (timed) {
     MC_HIP(hipEventRecord(tl.stop, st));

@@ -54,10 +54,12 @@ struct SmallArgs {
   const int4* ktab;
 };
 
-template <int NW, int MODE>
+// TAIL: a pointwise launch whose K is not a multiple of 32, so that the last K tiles hold rows of padding.
+template <int NW, int MODE, bool TAIL>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 16 ? 4 : 2, 4))) void igemm_small_kernel(
     const SmallArgs a) {
   static_assert(MODE == kModeOneMask || MODE == kModePointwise, "no tap table here");
+  static_assert(MODE == kModePointwise || !TAIL, "taps: padding rows have a tap that no pixel has");
   constexpr bool PW = MODE == kModePointwise;
   constexpr int TN = 1;                     // 32-pixel blocks of a tile (two measured no better anywhere)
   constexpr int BN = 32 * TN;
@@ -198,8 +200,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 1
   float breg[DEPTH][TN][8];
 #define MC_LOADF(voff, soff) \
   __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xres, voff, soff, 0))
-  // Rows past K: their filter rows are zero.  Pointwise they read what follows the last
-  // channel (nothing past the blob's end); an infinity there makes NaN of a sum, which is
+  // Rows past K (TAIL): their filter rows are zero.  They read what follows the last channel,
+  // nothing past the blob's end (small_rows.h); an infinity there makes NaN of a sum, which is
   // then formed again below, without padding rows.
 #define MC_LOAD(set, kt)                                                                      \
   {                                                                                           \
@@ -209,7 +211,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 1
     if constexpr (PW) {                                                                       \
       _Pragma("unroll") for (int j = 0; j < TN; ++j)                                          \
         _Pragma("unroll") for (int e = 0; e < 8; ++e) breg[set][j][e] =                       \
-            MC_LOADF(voff[j], static_cast<unsigned>(kt_ * BK + e) * x_cbytes);                \
+            MC_LOADF(small_lane_offset<TAIL>(voff[j], kt_, e, x_cbytes),                      \
+                     small_scalar_offset<TAIL>(kt_, e, x_cbytes));                            \
     } else {                                                                                  \
       const int4 two = taps[kt_ - kt_begin][lhi];                                             \
       _Pragma("unroll") for (int h = 0; h < 2; ++h)                                           \

@@ -572,7 +572,8 @@ struct SplitConfig {
   const char* name;
   void (*kernel[3])(const IgemmBatch);  // indexed by mode
   // igemm_small_kernel, whose tiles are taken for small launches: wavefronts that share K and the
-  // kernels by mode (0 and null: igemm_split_kernel)
+  // kernels for taps, for pointwise launches, and for those whose last K tiles hold padding
+  // (0 and null: igemm_split_kernel)
   int waves;
   void (*small[3])(const SmallArgs);
 };
@@ -584,7 +585,8 @@ struct SplitConfig {
     igemm_split_kernel<BM, BN, WM, WN, OCC, kModePointwise, KS>}, 0, {nullptr, nullptr, nullptr}}
 #define MC_SMALL(NW, NAME)                                                   \
   {32, 32, 1, 16 / NW, 3 * NW / 2, 0.f, 0.f, NAME, {nullptr, nullptr, nullptr}, NW,  \
-   {nullptr, igemm_small_kernel<NW, kModeOneMask>, igemm_small_kernel<NW, kModePointwise>}}
+   {igemm_small_kernel<NW, kModeOneMask, false>, igemm_small_kernel<NW, kModePointwise, false>, \
+    igemm_small_kernel<NW, kModePointwise, true>}}
 const SplitConfig kSplitConfigs[] = {
     MC_CONFIG(128, 128, 2, 2, 2, 1, 0.56f, 3.3f, "igemm_split_128x128"),
     MC_CONFIG(128, 64, 2, 2, 3, 1, 0.363f, 0.9f, "igemm_split_128x64"),

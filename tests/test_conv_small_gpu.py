@@ -111,3 +111,28 @@ def test_two_tops(K, config, c_first, slices):
     plan.forward(n, x.data_ptr(), whole.data_ptr(), shift=b.data_ptr())
     plan.forward_two_tops(n, x.data_ptr(), first.data_ptr(), c_first, second.data_ptr(), shift=b.data_ptr())
     assert torch.equal(first, whole[:, :c_first]) and torch.equal(second, whole[:, c_first:])
+
+
+@pytest.mark.parametrize("config", CONFIGS)
+@pytest.mark.parametrize("cin", [9, 15, 16, 17, 24, 31, 48, 49, 65, 144, 150])
+def test_nothing_behind_the_last_channel_is_read(K, config, cin):
+    """Padding rows of a pointwise launch: the same bits whatever follows the blob in memory."""
+    h, cout = 7, 20
+    g = torch.Generator(device="cuda").manual_seed(6)
+    w = torch.randn((cout, cin, 1, 1), generator=g, device="cuda")
+    room = torch.zeros((cin + 40, h, h), device="cuda")       # the blob, and 40 more planes
+    room[:cin] = torch.randn((cin, h, h), generator=g, device="cuda")
+    plan = K.ConvPlan(K.conv_geom(cin, h, h, cout, 1))
+    plan.force_config(config)
+    plan.force_split(1)
+    assert "32x32" in plan.kernel_name(1)
+    plan.set_weights(w.data_ptr())
+    tops = []
+    for behind in (0.0, float("inf"), float("nan"), 1e30):
+        room[cin:] = behind
+        y = torch.full((1, cout, h, h), float("nan"), device="cuda")
+        plan.forward(1, room.data_ptr(), y.data_ptr())
+        tops.append(y)
+    assert all(torch.equal(tops[0], t) for t in tops[1:])
+    want, mag = conv64(room[None, :cin], w), conv64(room[None, :cin].abs(), w.abs())
+    assert ((tops[0].double() - want).abs() <= (cin + 1) * 2.0 ** -24 * mag + 1e-30).all()
