@@ -225,11 +225,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 1
     }                                                                                         \
   }
   // h h' in two accumulators in turn, the five small products of terms in another
-  // (igemm_split_kernel): with a third of the tiles in a chain of its own the error is that of the
-  // larger tiles or below it (5x5 with K = 2400 in eight runs: 9.0e-8 of the norm, 10.9e-8
-  // with one chain, 9.4e-8 with 64x64 tiles).  The last one or two tiles go to the first chain:
-  // a run of two would round once more for the second than it rounds less.
-#define MC_MULTIPLY(set, other)                                                               \
+  // (igemm_split_kernel).  A sum that starts in the matrix instruction is rounded less than one that goes
+  // on there, so the last tiles of an unfinished turn take one accumulator each: a run of up to two
+  // tiles has no sum that goes on.
+#define MC_MULTIPLY(set, chain)                                                               \
   _Pragma("unroll") for (int j = 0; j < TN; ++j) {                                            \
     unsigned bt[3][4];                                                                        \
     _Pragma("unroll") for (int q = 0; q < 4; ++q)                                             \
@@ -239,8 +238,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 1
       av[q] = __builtin_bit_cast(bf16x8, areg[set][q]);                                       \
       bv[q] = __builtin_bit_cast(bf16x8, u32x4{bt[q][0], bt[q][1], bt[q][2], bt[q][3]});      \
     }                                                                                         \
-    if (other) odd[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0], bv[0], odd[j], 0, 0, 0); \
-    else acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0], bv[0], acc[j], 0, 0, 0);     \
+    chain[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0], bv[0], chain[j], 0, 0, 0);      \
     small[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0], bv[1], small[j], 0, 0, 0);      \
     small[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[1], bv[0], small[j], 0, 0, 0);      \
     small[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[1], bv[1], small[j], 0, 0, 0);      \
@@ -268,15 +266,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 1
       for (int d = 0; d < DEPTH; ++d) {
         // (the barriers are for the compiler's scheduler, which would gather the loads of all
         // sets at the end of the loop)
-        MC_MULTIPLY(d, d % 2)
+        if (d % 2) MC_MULTIPLY(d, odd) else MC_MULTIPLY(d, acc)
         __builtin_amdgcn_sched_barrier(0);
         MC_LOAD(d, min(kt + d + DEPTH, last))
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-#pragma unroll
-    for (int d = 0; d < DEPTH - 1; ++d)
-      if (kt + d < w_end) MC_MULTIPLY(d, false)
+    static_assert(DEPTH == 3, "at most two tiles are left");
+    if (kt < w_end) MC_MULTIPLY(0, acc)
+    if (kt + 1 < w_end) MC_MULTIPLY(1, odd)
   }
 #undef MC_LOAD
 #undef MC_MULTIPLY
@@ -286,7 +284,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 1
   for (int j = 0; j < TN; ++j)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      acc[j][r] = (acc[j][r] + odd[j][r] + small[j][r]) * kSplitUnscale;
+      acc[j][r] = (acc[j][r] + (odd[j][r] + small[j][r])) * kSplitUnscale;
       probe = __builtin_fmaf(acc[j][r], 0.f, probe);
     }
   if (__any(probe != 0.f)) {
@@ -326,15 +324,14 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 1
   float v[EPT];
 #pragma unroll
   for (int i = 0; i < EPT; ++i) {
-    // (in pairs: fewer roundings of large sums than one after the other)
-    float part[NW];
+    // (In 64 bits: one rounding instead of one per addition.  With this and the chains above the
+    // error is below that of 64x64 tiles for every K; in the norm, ReLU'd operands: 64 -> 256 1x1
+    // @14 3.9e-8 (in 32 bits 4.8, tiles 4.0), 128 -> 512 @28 4.3 (5.1, 4.8), 96 -> 100 5x5 6.7
+    // (8.0, 8.5).  0.0 to 0.1 us of a launch.)
+    double sum = sums[0][erow + i][tid % BN];
 #pragma unroll
-    for (int w = 0; w < NW; ++w) part[w] = sums[w][erow + i][tid % BN];
-#pragma unroll
-    for (int step = 1; step < NW; step *= 2)
-#pragma unroll
-      for (int w = 0; w < NW; w += 2 * step) part[w] += part[w + step];
-    v[i] = part[0];
+    for (int w = 1; w < NW; ++w) sum += sums[w][erow + i][tid % BN];
+    v[i] = static_cast<float>(sum);
   }
 
   if (a.counters != nullptr) {

@@ -136,3 +136,31 @@ def test_nothing_behind_the_last_channel_is_read(K, config, cin):
     assert all(torch.equal(tops[0], t) for t in tops[1:])
     want, mag = conv64(room[None, :cin], w), conv64(room[None, :cin].abs(), w.abs())
     assert ((tops[0].double() - want).abs() <= (cin + 1) * 2.0 ** -24 * mag + 1e-30).all()
+
+
+@pytest.mark.parametrize("geom", [
+    # cin, size, cout, k: runs of one K tile per wavefront, of two, of some, slices
+    (64, 14, 256, 1), (96, 14, 256, 1), (96, 9, 40, 1), (128, 28, 512, 1), (160, 14, 256, 1), (288, 14, 256, 1), (512, 7, 2048, 1),
+    (1024, 10, 126, 1), (16, 20, 64, 3), (32, 20, 64, 3), (96, 24, 100, 5)])
+@pytest.mark.parametrize("relu", [False, True])
+def test_error_is_not_above_the_larger_tiles(K, geom, relu):
+    """Against float64, where this kernel is chosen: its error in the norm is bounded by that of the
+    64x64 tiles, whose launches it took over."""
+    cin, h, cout, k = geom
+    for seed in (1, 2):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        x = torch.randn((1, cin, h, h), generator=g, device="cuda")
+        w = torch.randn((cout, cin, k, k), generator=g, device="cuda")
+        x = x.clamp(min=0) if relu else x
+        plan = K.ConvPlan(K.conv_geom(cin, h, h, cout, k, 1, k // 2))
+        plan.force_winograd(0)
+        plan.set_weights(w.data_ptr())
+        want = conv64(x, w, padding=k // 2)
+        errors = []
+        for config, name in ((-1, "32x32"), (7, "64x64")):
+            plan.force_config(config)
+            assert name in plan.kernel_name(1)
+            y = torch.full((1, cout, h, h), float("nan"), device="cuda")
+            plan.forward(1, x.data_ptr(), y.data_ptr())
+            errors.append((y.double() - want).norm().item())
+        assert errors[0] <= errors[1]
