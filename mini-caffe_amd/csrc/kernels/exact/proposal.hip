@@ -970,6 +970,13 @@ template <typename Lds>
 __device__ __forceinline__ bool fast_levels(Lds& s, int n, int num_top, uint2* __restrict__ stage,
                                             int* __restrict__ order) {
   typedef typename Lds::Entry KV;
+  // Moved places wait in registers where a wavefront has few enough chunks, which short partitions
+  // always leave it.  `stage` holds 32 bits of an entry: tables with wider ones must be small
+  // enough to do without.
+  constexpr int kRegPlaces = kFastRegChunks * 64;
+  constexpr bool kStaged = sizeof(Lds::kv) / sizeof(KV) > kFastWaves * kRegPlaces;
+  static_assert(kFastWaveSeg <= kRegPlaces, "short partitions wait in registers");
+  static_assert(!kStaged || sizeof(KV) == sizeof(uint32_t), "a staged entry is 32 bits");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // Every level shortens every open partition by at least its pivot: at most n levels.
   int n_cur = s.n_seg[0], n_cur_long = s.n_long[0], cur = 0, levels_left = n + 1;
@@ -1077,7 +1084,7 @@ __device__ __forceinline__ bool fast_levels(Lds& s, int n, int num_top, uint2* _
 #pragma unroll
         for (int k = 0; k < kFastRegChunks; ++k)
           if (keep_to[k] >= 0) s.kv[keep_to[k]] = keep_kv[k];
-      } else {
+      } else if constexpr (kStaged) {
         for (int c = c_begin; c < c_end; ++c) {
           const int q = g.lo + 1 + (c << 6) + lane;
           const KV mine = q <= g.hi ? s.kv[q] : pivot;
@@ -1087,7 +1094,7 @@ __device__ __forceinline__ bool fast_levels(Lds& s, int n, int num_top, uint2* _
           int rank, dest = 0;
           fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
           const bool mv = fast_move(g, s.tab, q, is_s, is_b, rank, &dest);
-          if (q <= g.hi) stage[q] = make_uint2(mv ? static_cast<uint32_t>(mine) : 0u, mv ? static_cast<uint32_t>(dest) : 0xffffffffu);
+          if (q <= g.hi) stage[q] = make_uint2(mv ? mine : 0u, mv ? static_cast<uint32_t>(dest) : 0xffffffffu);
           u += __popcll(__ballot(mv && is_s));
           t += __popcll(__ballot(mv && is_b));
           ps += __popcll(ms);
@@ -1164,37 +1171,12 @@ __device__ __forceinline__ bool fast_levels(Lds& s, int n, int num_top, uint2* _
       int u = 0, t = 0;
       ps = 0;
       pb = 0;
-      if (C <= kFastRegChunks) {
-        KV keep_kv[kFastRegChunks];
-        int keep_to[kFastRegChunks];
+      KV keep_kv[kFastRegChunks];
+      int keep_to[kFastRegChunks];
 #pragma unroll
-        for (int c = 0; c < kFastRegChunks; ++c) {
-          keep_to[c] = -1;
-          if (c < C) {
-            const int q = g.lo + 1 + (c << 6) + lane;
-            const KV mine = q <= g.hi ? s.kv[q] : pivot;
-            const uint32_t d = fast_rank(mine);
-            const unsigned long long ms = __ballot(d > K), mb = __ballot(d < K);
-            bool is_s, is_b;
-            int rank, dest = 0;
-            fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
-            const bool mv = fast_move(g, s.tab, q, is_s, is_b, rank, &dest);
-            if (mv) {
-              keep_to[c] = dest;
-              keep_kv[c] = mine;
-            }
-            u += __popcll(__ballot(mv && is_s));
-            t += __popcll(__ballot(mv && is_b));
-            ps += __popcll(ms);
-            pb += __popcll(mb);
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-        for (int c = 0; c < kFastRegChunks; ++c)
-          if (keep_to[c] >= 0) s.kv[keep_to[c]] = keep_kv[c];
-      } else {
-        for (int c = 0; c < C; ++c) {
+      for (int c = 0; c < kFastRegChunks; ++c) {
+        keep_to[c] = -1;
+        if (c < C) {
           const int q = g.lo + 1 + (c << 6) + lane;
           const KV mine = q <= g.hi ? s.kv[q] : pivot;
           const uint32_t d = fast_rank(mine);
@@ -1203,26 +1185,20 @@ __device__ __forceinline__ bool fast_levels(Lds& s, int n, int num_top, uint2* _
           int rank, dest = 0;
           fast_ranks(g, ms, mb, ps, pb, lane, &is_s, &is_b, &rank);
           const bool mv = fast_move(g, s.tab, q, is_s, is_b, rank, &dest);
-          if (q <= g.hi) stage[q] = make_uint2(mv ? static_cast<uint32_t>(mine) : 0u, mv ? static_cast<uint32_t>(dest) : 0xffffffffu);
+          if (mv) {
+            keep_to[c] = dest;
+            keep_kv[c] = mine;
+          }
           u += __popcll(__ballot(mv && is_s));
           t += __popcll(__ballot(mv && is_b));
           ps += __popcll(ms);
           pb += __popcll(mb);
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        // every lane reads back what it staged itself, four loads in flight
-        for (int c0 = 0; c0 < C; c0 += 4) {
-          uint2 e[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int q = g.lo + 1 + ((c0 + j) << 6) + lane;
-            e[j] = q <= g.hi ? stage[q] : make_uint2(0u, 0xffffffffu);
-          }
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (e[j].y != 0xffffffffu) s.kv[e[j].y] = e[j].x;
-        }
       }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int c = 0; c < kFastRegChunks; ++c)
+        if (keep_to[c] >= 0) s.kv[keep_to[c]] = keep_kv[c];
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       if (lane == 0) fast_finish(&s, g, pivot, u, t, num_top, order, next);
     }
