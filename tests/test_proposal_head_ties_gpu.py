@@ -43,7 +43,20 @@ def run(K, scores, bbox, im_info, pre, post, steps):
             call(K.LIB.mcProposalContinue)
             assert int(cnt[2].item()) == 1
     n = int(cnt[0].item())
-    return rois[:n].cpu().numpy(), rs[:n].cpu().numpy(), int(cnt[1].item())
+    return rois[:n].cpu().numpy(), rs[:n].cpu().numpy(), ws
+
+
+def flags(ws):
+    """The call's eight flag words, the last of the workspace (256 bytes with their padding)."""
+    return ws[-256:-224].view(torch.int32).tolist()
+
+
+def inputs(rng, fg, hw, spread=0.2):
+    (H, W), A = hw, 9
+    scores = rng.random((1, 2 * A, H, W)).astype(np.float32)
+    scores[0, A:] = fg.reshape(H, W, A).transpose(2, 0, 1)
+    bbox = (rng.standard_normal((1, 4 * A, H, W)) * spread).astype(np.float32)
+    return scores, bbox, np.array([H * 16, W * 16, 1.0], np.float32)
 
 
 @pytest.mark.parametrize("hw,pre,post,order", [
@@ -84,3 +97,36 @@ def test_rows_equal_the_reference(K, hw, pre, post, order, seed):
     for steps in (False, True):
         rois, rs, _ = run(K, scores, bbox, im_info, pre, post, steps)
         assert np.array_equal(rois, want_rois) and np.array_equal(rs, want_scores), steps
+
+
+def best_valid(scores, bbox, im_info):
+    """Indices by (score descending, index ascending), boxes that are too small last."""
+    props = oracle.generate_proposals(scores[0, 9:], bbox[0], oracle.generate_anchors(), float(im_info[0]), float(im_info[1]), 16.0, 16)
+    return np.argsort(-props[:, 4], kind="stable")
+
+
+@pytest.mark.parametrize("hw,post", [((38, 63), 200), ((40, 63), 200), ((64, 64), 200), ((20, 20), 100), ((12, 10), 60),
+                                     ((11, 9), 40), ((6, 5), 20)])
+@pytest.mark.parametrize("seed", range(2))
+def test_the_head_replays_its_equal_scores(K, hw, post, seed):
+    """The two best proposals have one score, so their order is open whatever the boxes are: the
+    replay that starts from the head settles it (it would not with the general replay forced)."""
+    rng = np.random.default_rng(70 + 2 * seed)
+    n = 9 * hw[0] * hw[1]
+    fg = rng.permutation(n).astype(np.float32) / n * 0.9 + 0.05
+    args = scores, bbox, im_info = inputs(rng, fg, hw)
+    best = best_valid(*args)
+    fg[best[1]] = fg[best[0]]
+    fg[best[min(400, n // 2)]] = fg[best[min(401, n // 2 + 1)]]
+    scores[0, 9:] = fg.reshape(hw + (9,)).transpose(2, 0, 1)
+    want = oracle.proposal({"pre_nms_topn": 6000, "post_nms_topn": post, "nms_thresh": 0.7}, *args, 2)
+    for general in (0, 1):
+        K.check_mc(K.LIB.mcProposalForceGeneralReplay(general))
+        try:
+            for steps in (False, True):
+                rois, rs, ws = run(K, *args, 6000, post, steps)
+                assert np.array_equal(rois, want[0]) and np.array_equal(rs, want[1]), (general, steps)
+                f = flags(ws)
+                assert (f[3], f[5]) == (0 if general else 2, 1), (f, general, steps)
+        finally:
+            K.check_mc(K.LIB.mcProposalForceGeneralReplay(0))
