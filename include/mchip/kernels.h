@@ -345,8 +345,9 @@ int mcProposalContinue(const float* scores, const float* bbox, const float* im_i
  * stream.  mcProposalTimingCollect waits for them, adds up over the calls since the
  * last collect stage_ms[0] decode + ordering of the head, [1] overlap matrix, scan and
  * check of the head + roi gather, [2] full-size path: radix sort, replay of the
- * reference's order of equal scores, gather of the best pre_nms_topn boxes, [3]
- * full-size path: NMS proper (overlap bit matrix + greedy scan) + roi gather; returns
+ * reference's order of equal scores, gather of the best pre_nms_topn boxes and overlap
+ * matrix of the best 512, [3] full-size path: greedy scans, overlap matrix of all + roi gather;
+ * returns
  * the number of calls and clears the list. */
 int mcProposalTimingEnable(int on);
 /* Test knob (process-wide): 1 = replay the order of equal scores with the general

@@ -130,3 +130,66 @@ def test_the_head_replays_its_equal_scores(K, hw, post, seed):
                 assert (f[3], f[5]) == (0 if general else 2, 1), (f, general, steps)
         finally:
             K.check_mc(K.LIB.mcProposalForceGeneralReplay(0))
+
+
+@pytest.mark.parametrize("kind", ["crowds", "a pair at the cut", "too many proposals"])
+def test_overlaps_beyond_the_best_512_are_left_out_where_these_settle_it(K, kind):
+    """Where the head cannot be ordered by itself, the best 512 of the fully ordered table still come
+    first: of the 94 x 6000 words of the overlap matrix 8 x 512 are written, the others stay as they were."""
+    rng = np.random.default_rng(80)
+    hw, pre, post = ((64, 65) if kind == "too many proposals" else (38, 63)), 6000, 200
+    n = 9 * hw[0] * hw[1]
+    fg = rng.permutation(n).astype(np.float32) / n * 0.9 + 0.05
+    if kind == "crowds":
+        fg = (np.round(fg * 2000) / 2000).astype(np.float32)
+    args = scores, bbox, im_info = inputs(rng, fg, hw)
+    if kind == "a pair at the cut":
+        best = best_valid(*args)
+        fg[best[512]] = fg[best[511]]
+        scores[0, 9:] = fg.reshape(hw + (9,)).transpose(2, 0, 1)
+    want = oracle.proposal({"pre_nms_topn": pre, "post_nms_topn": post, "nms_thresh": 0.7}, *args, 2)
+    for steps in (False, True):
+        rois, rs, ws = run(K, *args, pre, post, steps)
+        assert np.array_equal(rois, want[0]) and np.array_equal(rs, want[1]), steps
+        assert len(rois) == post and flags(ws)[3] == 0
+        untouched = int((ws[:ws.numel() // 8 * 8].view(torch.int64) == -1).sum().item())
+        assert untouched > 0.95 * pre * 94, steps
+
+
+def kept_of(boxes, thr):
+    """Greedy suppression in order, as the layer's."""
+    area = (boxes[:, 2] - boxes[:, 0] + 1) * (boxes[:, 3] - boxes[:, 1] + 1)
+    kept = []
+    for i, b in enumerate(boxes):
+        k = boxes[kept]
+        w = np.maximum(0, np.minimum(b[2], k[:, 2]) - np.maximum(b[0], k[:, 0]) + 1)
+        h = np.maximum(0, np.minimum(b[3], k[:, 3]) - np.maximum(b[1], k[:, 1]) + 1)
+        if not (w * h / (area[i] + area[kept] - w * h) > thr).any():
+            kept.append(i)
+    return kept
+
+
+@pytest.mark.parametrize("seed", range(2))
+def test_replayed_order_keeps_fewer_than_asked_for(K, seed):
+    """Triples of equal scores, neighbours overlap, the outer two do not: in index order two of each
+    are kept, with the middle one first just one.  The scan of the best 512 then reaches post_nms_topn in index
+    order only, and the full-size path follows the replay."""
+    rng = np.random.default_rng(90 + seed)
+    hw, A = (38, 63), 9
+    H, W = hw
+    fg = (rng.permutation(A * H * W).astype(np.float32) / (A * H * W) * 0.9 + 0.05).reshape(H, W, A)
+    scores, bbox, im_info = inputs(rng, fg.reshape(-1), hw, 0.0)
+    anchors = oracle.generate_anchors()
+    square = int(np.argmin(np.abs(anchors[:, 2] - anchors[:, 0] - 127) + np.abs(anchors[:, 3] - anchors[:, 1] - 127)))
+    for i, (h, w) in enumerate([(h, w) for h in (10, 20, 28) for w in (10, 25, 40, 50)]):
+        scores[0, A:, h - 5:h + 6, w - 5:w + 8] *= 0.1    # (nothing else that the triple's members would suppress)
+        scores[0, A + square, h, w:w + 3] = 0.99 - 0.001 * i
+    props = oracle.generate_proposals(scores[0, A:], bbox[0], anchors, float(im_info[0]), float(im_info[1]), 16.0, 16)
+    first = props[np.argsort(-props[:, 4], kind="stable")[:512]]
+    post = len(kept_of(first[:, :4], 0.7))
+    want = oracle.proposal({"pre_nms_topn": 6000, "post_nms_topn": post, "nms_thresh": 0.7}, scores, bbox, im_info, 2)
+    for steps in (False, True):
+        rois, rs, ws = run(K, scores, bbox, im_info, 6000, post, steps)
+        assert np.array_equal(rois, want[0]) and np.array_equal(rs, want[1]), steps
+        f = flags(ws)
+        assert (f[3], f[5], f[6], f[7]) == (0, 1, 1, 0), f
