@@ -870,6 +870,7 @@ int least_chains(const mcConvPlan* plan, const SubProblem& s, int num) {
 // measured throughput on full launches (kSplitConfigs).
 struct LaunchChoice {
   int config, slices;
+  double us;  // estimated
 };
 
 // Whether igemm_small_kernel can run the launch: no tap table, and the offsets of a flagged
@@ -886,7 +887,7 @@ bool fits_small(const mcConvPlan* plan, const std::vector<const SubProblem*>& li
 // (forced_split: as in the plan, 0 = choose.)
 LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const SubProblem*>& live, int num,
                                int forced_split) {
-  LaunchChoice best = {3, 1};
+  LaunchChoice best = {3, 1, 1e30};
   double best_us = 1e30;
   int least = 1;
   const bool small_ok = fits_small(plan, live, num);
@@ -920,7 +921,7 @@ LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const S
       if (s > 1) us += 1.2 + 0.26 * s + 2e-6 * blocks * s * cfg.bm * cfg.bn;
       if (us < best_us) {
         best_us = us;
-        best = {c, s};
+        best = {c, s, us};
       }
     }
   }
@@ -955,7 +956,7 @@ LaunchChoice pick_split_launch(const mcConvPlan* plan, const std::vector<const S
       if (s > 1) us += 1.75 + 0.0021 * wgs;
       if (us < best_us) {
         best_us = us;
-        best = {c, s};
+        best = {c, s, us};
       }
     }
   }
@@ -1450,7 +1451,7 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
   // (a request for one slice means two where there are two tops, see below)
   const int forced_split = top_second && plan->forced_split == 1 ? 2 : plan->forced_split;
   const LaunchChoice choice =
-      plan->split ? pick_split_launch(plan, live, num, forced_split) : LaunchChoice{pick_config(plan, max_pixels), 0};
+      plan->split ? pick_split_launch(plan, live, num, forced_split) : LaunchChoice{pick_config(plan, max_pixels), 0, 0.};
   const int bm = plan->split ? kSplitConfigs[choice.config].bm : kConfigs[choice.config].bm;
   const int bn = plan->split ? kSplitConfigs[choice.config].bn : kConfigs[choice.config].bn;
   const int stage_kt = plan->split ? kSplitConfigs[choice.config].ks : kConfigs[choice.config].ks;
@@ -1661,11 +1662,30 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
   return 0;
 }
 
+// Estimated time of the direct path for a layer that may take the Winograd path.  Of tiles in K
+// slices pick_split_launch's estimate, which is to rank them, is high by an amount that follows
+// the workgroups on a CU (3x3 layers, measured / estimated: two 0.90, three 0.855, four 0.955, five
+// 0.885, each to 3 % rms; 128-row tiles 0.8); unsliced ones and the small-launch kernel are met.
+double direct_us(const mcConvPlan* plan, int num) {
+  const SubProblem& s = plan->subs[0];
+  const LaunchChoice c = pick_split_launch(plan, {&s}, num, 0);
+  const SplitConfig& cfg = kSplitConfigs[c.config];
+  if (cfg.waves || c.slices == 1) return c.us;
+  if (cfg.bm == 128) return 0.8 * c.us;
+  const long workgroups =
+      (long)ceil_div(plan->M, cfg.bm) * ceil_div((long)num * s.Hq * s.Wq, cfg.bn) * c.slices;
+  const long on_cu = ceil_div(workgroups, kNumCu);
+  return c.us * (on_cu == 3 ? 0.855 : on_cu == 4 ? 0.955 : on_cu == 5 ? 0.885 : 0.9);
+}
+
 // Whether a call with `num` images runs on the Winograd path.
 bool takes_winograd(const mcConvPlan* plan, int num) {
-  return plan->winograd && plan->winograd_mode != 0 && plan->forced_config < 0 &&
-         winograd_fits(plan->winograd, num) &&
-         (plan->winograd_mode == 1 || winograd_pays(plan->winograd, num));
+  if (!plan->winograd || plan->winograd_mode == 0 || plan->forced_config >= 0 || !winograd_fits(plan->winograd, num))
+    return false;
+  if (plan->winograd_mode == 1) return true;
+  const WinogradChoice choice = winograd_pays(plan->winograd, num);
+  return choice == kWinogradAlways || (choice == kWinogradIfAhead && plan->split &&
+                                       winograd_us(plan->winograd, num) < direct_us(plan, num));
 }
 
 // The reference convolves image by image and so takes any blob an int can count

@@ -64,7 +64,9 @@ WinogradState* winograd_create(const mcConvGeom& geom, int Ho, int Wo);
 void winograd_destroy(WinogradState* w);
 int winograd_set_weights(WinogradState* w, const float* weights, hipStream_t stream);
 bool winograd_fits(const WinogradState* w, int num);  // one image addressable by the kernel
-bool winograd_pays(const WinogradState* w, int num);  // the automatic choice
+enum WinogradChoice { kWinogradNever, kWinogradIfAhead, kWinogradAlways };
+WinogradChoice winograd_pays(const WinogradState* w, int num);  // the automatic choice by size
+double winograd_us(const WinogradState* w, int num);            // estimated time of a launch
 double winograd_issued_flops(const WinogradState* w, int num);  // of the sixteen products
 // top_second / c_first as in mcConvForwardTwoTops (null / ignored for one top);
 // images_per_run > 0 caps the images one launch takes, forced_slices > 0 fixes the

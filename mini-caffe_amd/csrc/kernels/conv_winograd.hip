@@ -562,26 +562,53 @@ bool winograd_fits(const WinogradState* w, int /*num*/) {
 // direct tile of all, this path still leads on launches that fill the chip: batch 64, 64 -> 64 @56
 // 100.5 us against 98.7 (even), 128 @28 86 / 93, 256 @14 80 / 88, 512 @7 86.5 / 88.7; batch 8, 64 @300
 // 295 / 322, 128 @150 236 / 258, 256 @75 236 / 259, 512 @38 239 / 269, 512 @19 84.6 / 85.8; RPN head
-// 108 / 130.  On smaller ones it does not.  Tile-rounds of a launch and us, this path against the
-// best direct kernel: 1344 (512 -> 150 @10 b8) 39 / 20, 1568 (64 @56, 128 @28, 256 @14 b8) 25 / 23, 27 / 23,
-// 29 / 22, 1968 (128 -> 192 @24 b9) 30 / 26, 2048 (512 @7 b8) 38 / 25, 2448 (284 -> 214 @46) 32 / 24; 3136 (128
-// @56 b4) 36 / 38, 3888 (64 -> 192 @48 b9) 32 / 42, 4704 (96 @56 b8) 39.5 / 40, 6144 (1024 -> 256 @38) 57 / 63,
-// 6272 (256 @28 b8) 53.5 / 53, 7980 (276 -> 251 @60 b2) 63 / 73, 9600 (1024 -> 150 @19 b8) 71 / 91.
+// 108 / 130.  On smaller ones it depends on how either kernel's tiles and slices fill the chip, so
+// that between 1200 and 2800 tile-rounds the estimated times decide (us, this path against the best
+// direct kernel: ahead 2368 (128 @28 b12) 30.9 / 33.2, 2304 (128 -> 208 @12 b32) 28.2 / 30.9, 2592 (192 @12 b32) 30.9 /
+// 32.2, 2760 (160 @75 b1) 30.2 / 35.0; behind 1344 (512 -> 150 @10 b8) 35 / 18, 1568 (64 @56, 128 @28 b8) 25 / 22, 26 / 23,
+// 1968 (128 -> 192 @24 b9) 30 / 24, 2048 (512 @7 b8) 38 / 25, 2432 (256 @14 b12) 32 / 27).  Of 112 launches
+// in that range the estimates choose the slower kernel by more than 2 % twice, by 4 % at most; all
+// together take 2775 us, 2803 without this path, 2772 with the better of the two each time.
 // What loses: 32 input channels (the loop is four rounds long: 56 / 47 us), an
 // output tile that is half padding (64 -> 32: 86 / 82), and launches of a few tiles,
 // whose time is this kernel's longer prologue and finish (256 -> 150 on 5x5 maps, 9
 // tiles: 25 / 19 us; one image of 256 channels on 14x14: 22 / 19; config 1's single
 // 64 -> 64 layer on one 56x56 image, 25 tiles of 8 rounds: 17 / 12).
-bool winograd_pays(const WinogradState* w, int num) {
+WinogradChoice winograd_pays(const WinogradState* w, int num) {
   const mcConvGeom& g = w->geom;
   const long blocks = (long)num * ((w->Ho + 1) / 2) * ((w->Wo + 1) / 2);
-  if (g.channels_in < 64) return false;
-  if (4 * g.channels_out < 3 * w->MT * kTileM) return false;
+  if (g.channels_in < 64) return kWinogradNever;
+  if (4 * g.channels_out < 3 * w->MT * kTileM) return kWinogradNever;
   // odd and tiny maps compute blocks that hang over the edge: a 3x3 map is four
   // blocks for nine outputs (16 x 4 products against 36 x 9 / 4 useful ones)
-  if (10L * w->Ho * w->Wo < 26L * ((w->Ho + 1) / 2) * ((w->Wo + 1) / 2)) return false;
+  if (10L * w->Ho * w->Wo < 26L * ((w->Ho + 1) / 2) * ((w->Wo + 1) / 2)) return kWinogradNever;
   const long tiles = (long)w->MT * ceil_div(blocks, kTileT);
-  return tiles * (w->KT / 2) >= 2800;
+  const long tile_rounds = tiles * (w->KT / 2);
+  return tile_rounds >= 2800 ? kWinogradAlways : tile_rounds >= 1200 ? kWinogradIfAhead : kWinogradNever;
+}
+
+// Channel rounds of a slice: a launch that leaves workgroup slots empty (two per CU) cuts its
+// rounds into slices, each at least four rounds long.
+static int rounds_per_slice(const WinogradState* w, long tiles, int forced_slices) {
+  const int rounds = w->KT / 2;
+  int slices = forced_slices > 0 ? forced_slices : static_cast<int>(2L * kNumCu / tiles);
+  slices = std::max(1, std::min(std::min(slices, 16), forced_slices > 0 ? rounds : rounds / 4));
+  return ceil_div(rounds, slices);
+}
+
+// A fixed part, per CU the rounds of its workgroups, two side by side (2.27 us a round) or one alone
+// (1.76), 1.8 us for each workgroup's prologue and finish, and what slices cost.  The constants
+// fit 330 launches of 20 to 100 us (800 to 9000 tile-rounds) to 4 % rms, 15 % at most.
+double winograd_us(const WinogradState* w, int num) {
+  const long blocks = (long)num * ((w->Ho + 1) / 2) * ((w->Wo + 1) / 2);
+  const long tiles = (long)w->MT * ceil_div(blocks, kTileT);
+  const int per = rounds_per_slice(w, tiles, 0);
+  const int slices = ceil_div(w->KT / 2, per);
+  const double workgroups = static_cast<double>(tiles) * slices;
+  const long on_cu = ceil_div(tiles * slices, kNumCu);
+  double us = 6.85 + per * (2.27 * (on_cu / 2) + 1.76 * (on_cu % 2)) + 1.8 * on_cu;
+  if (slices > 1) us += 1. + 0.8 * slices + 1.6 * workgroups / kNumCu;
+  return us;
 }
 
 int winograd_set_weights(WinogradState* w, const float* weights, hipStream_t st) {
@@ -665,13 +692,8 @@ int winograd_forward(WinogradState* w, int num, const float* bottom, float* top,
     make_fast_div(a.MT, (unsigned long long)a.MT * a.NT + 1, &a.div_mt_mul, &a.div_mt_shift);
     const long tiles = (long)a.MT * a.NT;
     MC_REQUIRE(tiles < (1L << 31), "mcConvForward: grid too large");
-    // A launch that leaves workgroup slots empty (two per CU) cuts the channel rounds
-    // into slices, each at least four rounds long.
-    const int rounds = w->KT / 2;
-    int slices = forced_slices > 0 ? forced_slices : static_cast<int>(2L * kNumCu / tiles);
-    slices = std::max(1, std::min(std::min(slices, 16), forced_slices > 0 ? rounds : rounds / 4));
-    a.rounds_per_slice = ceil_div(rounds, slices);
-    slices = ceil_div(rounds, a.rounds_per_slice);  // no empty slice
+    a.rounds_per_slice = rounds_per_slice(w, tiles, forced_slices);
+    const int slices = ceil_div(w->KT / 2, a.rounds_per_slice);  // no empty slice
     a.partial = nullptr;
     a.counters = nullptr;
     if (slices > 1) {
