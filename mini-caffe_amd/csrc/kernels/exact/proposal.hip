@@ -1276,17 +1276,16 @@ __global__ __launch_bounds__(kFastThreads) void tie_replay_fast_kernel(
 // wavefront c % 16), the original indices and the table of larger scores in LDS, and only
 // the elements that change places inside the followed partition move.  From 1024 places
 // on fast_levels goes on.  What bounds it: one CU's instruction issue in the
-// five passes over the partition per level (10 us for the first levels of 21 546 proposals, three to
-// nine levels), then the dependent levels below 1024 places (25 to 50 us).  21 546 proposals with two to
-// eight pairs among the best 512: 126 us on the average, where sorting the whole table and
-// replaying all its equal scores takes 81 + 205; 33 696 proposals, whose replay walked every
-// partition through memory: mcProposal 1500 -> 205 us.
+// five passes over the partition per level (21 to 25 us for all of 21 546 proposals; three to nine
+// levels, 1.2 to 4.4 times the table together), then the dependent levels below 1024 places (25 to 50
+// us).  21 546 proposals with four or five pairs among the best 512: mcProposal 167 us, where sorting the
+// whole table and replaying all its equal scores took 334; 33 480 proposals, whose replay
+// walked every partition through memory: 1500 -> 177 us.
 constexpr int kTieThreads = 1024, kTieWaves = kTieThreads / 64;
 // keys per thread, for the two sizes of table that the head takes
 constexpr int kTieSlots = kHeadPer / 2, kTieSlotsLarge = kHeadPerLarge / 2;
 static_assert(kTieThreads == 2 * kHeadThreads, "half as many keys per thread");
 constexpr int kTieStop = 1024;
-constexpr int kTieLevels = 64;                      // more (nearly sorted tables) are left to the full-size path
 static_assert(kTieThreads == kFastThreads, "fast_levels is for the same workgroup");
 
 template <int SLOTS>
@@ -1310,7 +1309,8 @@ __global__ __launch_bounds__(kTieThreads) void tie_head_kernel(
     FastLdsOf<unsigned long long, 2 * kTieThreads> fast;  // (whole keys: no dense ranks to find)
   } lds;
   __shared__ unsigned long long pairs[kHeadWant / 64];  // bit j: sorted places j and j + 1 are equal
-  __shared__ uint32_t pending[kTieLevels + 1];          // short partitions left behind (lo << 16 | hi)
+  // short partitions left behind (lo << 16 | hi): two places of the first `want` and more each
+  __shared__ uint32_t pending[kHeadWant / 2 + 1];
   TieChainLds<SLOTS>& s = lds.chain;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   auto below = [](unsigned long long m) {  // bits of lower lanes
@@ -1348,11 +1348,24 @@ __global__ __launch_bounds__(kTieThreads) void tie_head_kernel(
     return any;
   };
 
-  // All of what follows is uniform over the workgroup except the elements themselves.
-  int lo = 0, hi = n - 1, n_pending = 0, level = 0;
+  // All of what follows is uniform over the workgroup except the elements themselves.  Every level
+  // shortens the partition by its pivot at least, so n levels at most.  Four levels that neither
+  // shorten it by 1/128 nor bring its front 32 of the 512 places further are those of a nearly sorted
+  // table, with hundreds and more to come.  Where the full-size replay would run in LDS it gets such
+  // tables, since it walks those levels a little faster (20 us at full length, 21 to 25 here): 21 546
+  // scores in descending order 13.7 ms there, 13.9 with these four levels before, 15.1 with 64, 16.9 to
+  // the end here; in ascending order, where the front moves on, 0.84 there and 0.61 here.  Larger tables
+  // would be walked through memory and are always finished here: 33 480 descending scores 119 ms -> 34.
+  int window = 0, window_lo = 0, window_len = n;
+  int lo = 0, hi = n - 1, n_pending = 0;
   bool open = n >= 2;
   while (open && hi - lo + 1 > kTieStop) {
-    if (++level > kTieLevels) return;
+    if (++window == 5) {
+      if (n <= kFastMaxN && hi - lo + 1 > window_len - window_len / 128 && lo - window_lo < 32) return;
+      window = 1;
+      window_lo = lo;
+      window_len = hi - lo + 1;
+    }
     const int c_first = lo >> 6, c_last = hi >> 6;
 #pragma unroll
     for (int j = 0; j < SLOTS; ++j)
@@ -1416,7 +1429,7 @@ __global__ __launch_bounds__(kTieThreads) void tie_head_kernel(
       open = false;
       break;
     }
-    {
+    if (nB > 0) {
     MC_EACH_CHUNK
       const unsigned long long mb = __ballot(is_b);
       const int rank = nB - (static_cast<int>(s.cnt[c] >> 16) + below(mb));  // (its own bit not counted)
@@ -1425,7 +1438,7 @@ __global__ __launch_bounds__(kTieThreads) void tie_head_kernel(
     MC_END_CHUNK
     }
     __syncthreads();
-    {
+    if (nS > 0 && nB > 0) {
       // of the smaller scores: how many change places with a larger one (u), how many take the next
       // larger one in (t, with the first, which goes to the pivot's place), the last that moves
       int u = 0, t = 0, last = -1;
@@ -1452,7 +1465,7 @@ __global__ __launch_bounds__(kTieThreads) void tie_head_kernel(
     if ((t != u && t != u + 1) || h < lo || h > hi) return;  // cannot happen; the full-size path redoes the job
     const bool left = h - 1 > lo && touched(lo, h - 1), left_one = h - 1 == lo;
     const bool right = h + 1 < hi && h + 1 < want && touched(h + 1, hi), right_one = h + 1 == hi && h + 1 < want;
-    if (right || right_one) {
+    if ((right || right_one) && u > 0) {
       // (u <= h - lo < want: the places before the pivot's)
       MC_EACH_CHUNK
         const unsigned long long ms = __ballot(is_s);
@@ -1481,7 +1494,7 @@ __global__ __launch_bounds__(kTieThreads) void tie_head_kernel(
     // the places behind h: a larger score's is taken by the smaller one of its rank.  (These are the u
     // first larger scores from the right; counted from h on, because the places before it have
     // new scores by now.)
-    if (right || right_one) {
+    if ((right || right_one) && u > 0) {
       MC_EACH_CHUNK
         const unsigned long long mb = __ballot(is_b && q > h);
         const int before = c == (h >> 6) ? 0 : static_cast<int>(s.cnt[c] >> 16) - (nB - u);

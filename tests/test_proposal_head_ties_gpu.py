@@ -132,6 +132,38 @@ def test_the_head_replays_its_equal_scores(K, hw, post, seed):
             K.check_mc(K.LIB.mcProposalForceGeneralReplay(0))
 
 
+@pytest.mark.parametrize("order", ["descending", "ascending", "almost descending", "shuffled by 16", "organ pipe"])
+@pytest.mark.parametrize("hw", [(38, 63), (20, 20), (64, 64)])
+def test_sorted_tables(K, hw, order):
+    """Hundreds of levels with a pivot or two each.  The head's replay follows them where the table is too
+    large for the full-size one's LDS, or its front moves along quickly, and else gives up."""
+    rng = np.random.default_rng(60)
+    n = 9 * hw[0] * hw[1]
+    fg = np.arange(n, 0, -1).astype(np.float32) / n * 0.9 + 0.05
+    if order == "ascending":
+        fg = fg[::-1].copy()
+    elif order == "almost descending":
+        for i in rng.integers(0, n - 5, n // 50):
+            fg[i], fg[i + 4] = fg[i + 4], fg[i]
+    elif order == "shuffled by 16":
+        fg = rng.permuted(fg[:n // 16 * 16].reshape(-1, 16), axis=1).reshape(-1)
+        fg = np.concatenate([fg, np.full(n - fg.size, 0.05, np.float32)])
+    elif order == "organ pipe":
+        fg = np.concatenate([fg[::2][::-1], fg[1::2]])
+    args = scores, bbox, im_info = inputs(rng, fg, hw)
+    best = best_valid(*args)
+    for at in (0, 7, 100, 101, 300):
+        fg[best[at + 1]] = fg[best[at]]
+    scores[0, 9:] = fg.reshape(hw + (9,)).transpose(2, 0, 1)
+    post = 100
+    want = oracle.proposal({"pre_nms_topn": 6000, "post_nms_topn": post, "nms_thresh": 0.7}, *args, 2)
+    for steps in (False, True):
+        rois, rs, ws = run(K, *args, 6000, post, steps)
+        assert np.array_equal(rois, want[0]) and np.array_equal(rs, want[1]), steps
+        path = tuple(flags(ws)[k] for k in (3, 5, 7))
+        assert path == ((2, 1, 0) if n > 22528 else (0, 1, 1) if order == "descending" else path), steps
+
+
 @pytest.mark.parametrize("kind", ["crowds", "a pair at the cut", "too many proposals"])
 def test_overlaps_beyond_the_best_512_are_left_out_where_these_settle_it(K, kind):
     """Where the head cannot be ordered by itself, the best 512 of the fully ordered table still come
