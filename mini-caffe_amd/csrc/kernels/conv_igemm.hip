@@ -1448,10 +1448,8 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
     max_pixels = std::max(max_pixels, pixels);
   }
   if (live.empty()) return 0;
-  // (a request for one slice means two where there are two tops, see below)
-  const int forced_split = top_second && plan->forced_split == 1 ? 2 : plan->forced_split;
   const LaunchChoice choice =
-      plan->split ? pick_split_launch(plan, live, num, forced_split) : LaunchChoice{pick_config(plan, max_pixels), 0, 0.};
+      plan->split ? pick_split_launch(plan, live, num, plan->forced_split) : LaunchChoice{pick_config(plan, max_pixels), 0, 0.};
   const int bm = plan->split ? kSplitConfigs[choice.config].bm : kConfigs[choice.config].bm;
   const int bn = plan->split ? kSplitConfigs[choice.config].bn : kConfigs[choice.config].bn;
   const int stage_kt = plan->split ? kSplitConfigs[choice.config].ks : kConfigs[choice.config].ks;
@@ -1482,8 +1480,8 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
     return launch_small(plan, *live[0], choice, num, bottom, top, ep, st, top_second, c_first);
   // slices are chosen for the plan as a whole: all sub-problems of a launch run
   // side by side
-  // Two tops are told apart by the pass that sums the slices, so such a launch
-  // has at least two of them (a slice past the last K tile adds zeros).
+  // Two tops are told apart by the pass that sums the slices, so such a launch of the larger
+  // tiles has at least two of them (a slice past the last K tile adds zeros).
   int slices = thin ? 1 : plan->split ? choice.slices : pick_split(plan, total_blocks, min_kt);
   if (top_second && slices == 1) slices = 2;
   const long slice_stride = (out_count + 3) / 4 * 4;

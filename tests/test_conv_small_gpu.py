@@ -31,7 +31,8 @@ def conv64(x, w, **kw):
     (33, 9, 7, 65, 1, 2, 0, 1, 1, 3, 2), (160, 11, 11, 129, 1, 1, 0, 1, 1, 3, 3), (512, 6, 5, 31, 1, 1, 0, 1, 1, 1, 16),
     (4, 16, 16, 64, 3, 1, 1, 1, 1, 1, 1), (12, 13, 9, 130, 3, 2, 1, 1, 1, 2, 2), (20, 7, 7, 40, 5, 1, 2, 1, 1, 3, 5),
     (64, 1, 1, 24, 3, 1, 1, 1, 1, 5, 4), (8, 10, 11, 20, 3, 1, 2, 2, 1, 2, 1), (24, 12, 5, 96, 3, 1, 1, 1, 2, 2, 2),
-    (160, 9, 9, 70, 1, 1, 0, 1, 2, 2, 1), (36, 31, 3, 33, (1, 5), 1, (0, 2), 1, 1, 1, 1)])
+    (160, 9, 9, 70, 1, 1, 0, 1, 2, 2, 1), (36, 31, 3, 33, (1, 5), 1, (0, 2), 1, 1, 1, 1),
+    (1820, 3, 3, 20, 3, 1, 1, 1, 1, 1, 1)])          # 1024 K tiles, the longest table of taps
 def test_against_float64(K, case, config):
     cin, h, wd, cout, k, s, p, d, group, n, slices = case
     k = (k, k) if isinstance(k, int) else k
@@ -77,6 +78,7 @@ def test_special_values(K, geom, config, slices):
     plan = K.ConvPlan(K.conv_geom(cin, 13, 13, cout, k, s, p, d, g))
     plan.force_config(config)
     plan.force_split(slices)
+    assert "32x32" in plan.kernel_name(2)
     xd, wd = torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda()
     ho, wo = plan.output_shape()
     plan.set_weights(wd.data_ptr())
@@ -94,7 +96,7 @@ def test_special_values(K, geom, config, slices):
 
 @pytest.mark.parametrize("config", CONFIGS)
 @pytest.mark.parametrize("c_first", [1, 32, 45, 69])
-@pytest.mark.parametrize("slices", [2, 5])
+@pytest.mark.parametrize("slices", [1, 2, 5])
 def test_two_tops(K, config, c_first, slices):
     n, cin, h, cout = 3, 40, 7, 70
     g = torch.Generator(device="cuda").manual_seed(4)
@@ -104,6 +106,7 @@ def test_two_tops(K, config, c_first, slices):
     plan = K.ConvPlan(K.conv_geom(cin, h, h, cout, 3, 1, 1))
     plan.force_config(config)
     plan.force_split(slices)
+    assert "32x32" in plan.kernel_name(n)
     plan.set_weights(w.data_ptr())
     whole = torch.full((n, cout, h, h), float("nan"), device="cuda")
     first = torch.full((n, c_first, h, h), float("nan"), device="cuda")
