@@ -1448,8 +1448,12 @@ int conv_forward_images(const mcConvPlan* plan, int num, const float* bottom, fl
     max_pixels = std::max(max_pixels, pixels);
   }
   if (live.empty()) return 0;
+  // (a request for one slice means two where there are two tops, see below, unless it is for the
+  // small-launch kernel by name)
+  const bool small_asked = plan->split && plan->forced_config >= kNumConfigs && fits_small(plan, live, num);
+  const int forced_split = top_second && plan->forced_split == 1 && !small_asked ? 2 : plan->forced_split;
   const LaunchChoice choice =
-      plan->split ? pick_split_launch(plan, live, num, plan->forced_split) : LaunchChoice{pick_config(plan, max_pixels), 0, 0.};
+      plan->split ? pick_split_launch(plan, live, num, forced_split) : LaunchChoice{pick_config(plan, max_pixels), 0, 0.};
   const int bm = plan->split ? kSplitConfigs[choice.config].bm : kConfigs[choice.config].bm;
   const int bn = plan->split ? kSplitConfigs[choice.config].bn : kConfigs[choice.config].bn;
   const int stage_kt = plan->split ? kSplitConfigs[choice.config].ks : kConfigs[choice.config].ks;
