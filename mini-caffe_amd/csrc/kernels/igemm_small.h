@@ -10,14 +10,16 @@
 // barrier, DEPTH K tiles ahead; the NW blocks of sums then meet in LDS.  Four times as many
 // tiles and NW runs each occupy the chip with a quarter or less of the slices, and what a
 // slice leaves in memory is 4 KB.  The price is that every operand is fetched and split
-// by each wavefront that multiplies it (four times the traffic of a 64x64 tile per
-// product), which larger launches do not earn back: see pick_split_launch.
+// by each wavefront that multiplies it, and a 32x32 tile multiplies each value it fetches half as
+// often as a 64x64 tile (64 values for 1024 products, 128 for 4096: twice the traffic and twice the
+// splitting), which larger launches do not earn back: see pick_split_launch.
 //
 // What bounds it: on one image the fixed 3 us of a launch (dispatch, arguments, first loads, the
 // meeting of the wavefronts), 0.33 us per K tile of a wavefront, and 2 us where slices are summed.
-// us per launch, the 64x64 tile / this: 64 -> 64 3x3 on one 56x56 map 10.6 / 6.5, 128 -> 128 @28
-// 12.3 / 8.9, 256 -> 256 @14 14.0 / 9.4, 512 -> 512 @7 16.3 / 10.6, 256 -> 1024 1x1 @14 7.9 / 4.5,
-// 1024 -> 256 10.0 / 6.5, 512 -> 2048 @7 8.2 / 5.9, 2048 -> 512 11.3 / 7.8, 512 -> 24 3x3 @10 17.4 / 7.8.
+// us per launch, 64x64 tiles / this, launches of one layer one behind the other: 64 -> 64 3x3 on one 56x56 map
+// 10.2 / 7.0, 128 -> 128 @28 11.9 / 8.8, 256 -> 256 @14 13.8 / 9.3, 512 -> 512 @7 16.0 / 10.1, 256 -> 1024 1x1
+// @14 8.1 / 5.0, 1024 -> 256 10.2 / 7.2, 512 -> 2048 @7 8.5 / 5.8, 2048 -> 512 11.4 / 7.8, 512 -> 24 3x3 @10
+// 15.6 / 8.0.  Inside a network's forward, where the filters come from memory, 1 to 2 us more.
 // Sixteen wavefronts to a workgroup instead of slices: 13.6 us where four slices take 10.3.
 //
 // Lane l of the 32x32x16 product holds K rows 8 (l / 32) .. + 7 of filter row / pixel l % 32: of
@@ -56,13 +58,12 @@ struct SmallArgs {
 
 // TAIL: a pointwise launch whose K is not a multiple of 32, so that the last K tiles hold rows of padding.
 template <int NW, int MODE, bool TAIL>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 16 ? 4 : 2, 4))) void igemm_small_kernel(
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 4))) void igemm_small_kernel(
     const SmallArgs a) {
   static_assert(MODE == kModeOneMask || MODE == kModePointwise, "no tap table here");
   static_assert(MODE == kModePointwise || !TAIL, "taps: padding rows have a tap that no pixel has");
   constexpr bool PW = MODE == kModePointwise;
-  constexpr int TN = 1;                     // 32-pixel blocks of a tile (two measured no better anywhere)
-  constexpr int BN = 32 * TN;
+  constexpr int BN = 32;                    // pixels of a tile (64 measured no better anywhere)
   constexpr int EPT = 32 * BN / (NW * 64);  // sums a thread finishes: consecutive rows of a pixel
   constexpr int DEPTH = 3;                  // K tiles on their way
   __shared__ float sums[NW][32][BN];
@@ -154,12 +155,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 1
     }
   }
   const int n_dw = a.n_dw;
-  // byte offset of each pixel's origin, and (3x3 and the like) a bit per tap outside the image;
+  // byte offset of the pixel's origin, and (3x3 and the like) a bit per tap outside the image;
   // a column past the last pixel has no elements
-  unsigned voff[TN], bad[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int p = nt * BN + j * 32 + l32;
+  unsigned voff, bad = 0xFFFFFFFFu;
+  {
+    const int p = nt * BN + l32;
     const int n = fast_div(p, a.div_hw_mul, a.div_hw_shift);
     const int rem = p - n * a.HqWq;
     const int qh = fast_div(rem, a.div_w_mul, a.div_w_shift);
@@ -168,19 +168,18 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 1
     const int wi0 = qw * a.q_sw + a.in_ow;
     const unsigned origin = static_cast<unsigned>(
         ((n * a.x_nstride + g * a.x_gstride + (hi0 * a.W + wi0)) << 2) + a.pix_shift);
-    voff[j] = p < a.P ? origin : kNoElement;
-    bad[j] = 0xFFFFFFFFu;
+    voff = p < a.P ? origin : kNoElement;
     if constexpr (PW) {
-      voff[j] += static_cast<unsigned>(lhi) * 8u * x_cbytes;
+      voff += static_cast<unsigned>(lhi) * 8u * x_cbytes;
     } else if (p < a.P) {
       unsigned col_bad = 0u;
       for (int b = 0; b < n_dw; ++b)
         col_bad |= static_cast<unsigned>(static_cast<unsigned>(wi0 + b * a.dil_w) >= static_cast<unsigned>(a.W)) << b;
       const unsigned all_cols = (1u << n_dw) - 1u;
-      bad[j] = 0x80000000u;  // bit 31: the tap of K padding rows, never valid
+      bad = 0x80000000u;  // bit 31: the tap of K padding rows, never valid
       for (int b = 0; b < a.n_dh; ++b) {
         const bool row_bad = static_cast<unsigned>(hi0 + b * a.dil_h) >= static_cast<unsigned>(a.H);
-        bad[j] |= (row_bad ? all_cols : col_bad) << (b * n_dw);
+        bad |= (row_bad ? all_cols : col_bad) << (b * n_dw);
       }
     }
   }
@@ -197,7 +196,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 1
   if constexpr (!PW) __syncthreads();  // the taps
 
   u32x4 areg[DEPTH][3];
-  float breg[DEPTH][TN][8];
+  float breg[DEPTH][8];
 #define MC_LOADF(voff, soff) \
   __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xres, voff, soff, 0))
   // Rows past K (TAIL): their filter rows are zero.  They read what follows the last channel,
@@ -209,19 +208,17 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 1
     _Pragma("unroll") for (int q = 0; q < 3; ++q) areg[set][q] = __builtin_bit_cast(u32x4,    \
         __builtin_amdgcn_raw_buffer_load_b128(wres, avoff, static_cast<unsigned>(kt_) * wt_kt_bytes + q * a_plane, 0)); \
     if constexpr (PW) {                                                                       \
-      _Pragma("unroll") for (int j = 0; j < TN; ++j)                                          \
-        _Pragma("unroll") for (int e = 0; e < 8; ++e) breg[set][j][e] =                       \
-            MC_LOADF(small_lane_offset<TAIL>(voff[j], kt_, e, x_cbytes),                      \
-                     small_scalar_offset<TAIL>(kt_, e, x_cbytes));                            \
+      _Pragma("unroll") for (int e = 0; e < 8; ++e) breg[set][e] =                            \
+          MC_LOADF(small_lane_offset<TAIL>(voff, kt_, e, x_cbytes),                           \
+                   small_scalar_offset<TAIL>(kt_, e, x_cbytes));                              \
     } else {                                                                                  \
       const int4 two = taps[kt_ - kt_begin][lhi];                                             \
-      _Pragma("unroll") for (int h = 0; h < 2; ++h)                                           \
-        _Pragma("unroll") for (int j = 0; j < TN; ++j) {                                      \
-          const unsigned v = ((__builtin_amdgcn_ubfe(bad[j], h ? two.w : two.y, 1) << 31) | voff[j]) + \
-                             static_cast<unsigned>(h ? two.z : two.x);                        \
-          _Pragma("unroll") for (int e = 0; e < 4; ++e)                                       \
-            breg[set][j][4 * h + e] = MC_LOADF(v, e * x_cbytes);                              \
-        }                                                                                     \
+      _Pragma("unroll") for (int h = 0; h < 2; ++h) {                                         \
+        const unsigned v = ((__builtin_amdgcn_ubfe(bad, h ? two.w : two.y, 1) << 31) | voff) + \
+                           static_cast<unsigned>(h ? two.z : two.x);                          \
+        _Pragma("unroll") for (int e = 0; e < 4; ++e)                                         \
+          breg[set][4 * h + e] = MC_LOADF(v, e * x_cbytes);                                   \
+      }                                                                                       \
     }                                                                                         \
   }
   // h h' in two accumulators in turn, the five small products of terms in another
@@ -229,28 +226,26 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 1
   // on there, so the last tiles of an unfinished turn take one accumulator each: a run of up to two
   // tiles has no sum that goes on.
 #define MC_MULTIPLY(set, chain)                                                               \
-  _Pragma("unroll") for (int j = 0; j < TN; ++j) {                                            \
+  {                                                                                           \
     unsigned bt[3][4];                                                                        \
     _Pragma("unroll") for (int q = 0; q < 4; ++q)                                             \
-      split_pair(breg[set][j][2 * q], breg[set][j][2 * q + 1], bt[0][q], bt[1][q], bt[2][q]); \
+      split_pair(breg[set][2 * q], breg[set][2 * q + 1], bt[0][q], bt[1][q], bt[2][q]);       \
     bf16x8 av[3], bv[3];                                                                      \
     _Pragma("unroll") for (int q = 0; q < 3; ++q) {                                           \
       av[q] = __builtin_bit_cast(bf16x8, areg[set][q]);                                       \
       bv[q] = __builtin_bit_cast(bf16x8, u32x4{bt[q][0], bt[q][1], bt[q][2], bt[q][3]});      \
     }                                                                                         \
-    chain[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0], bv[0], chain[j], 0, 0, 0);      \
-    small[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0], bv[1], small[j], 0, 0, 0);      \
-    small[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[1], bv[0], small[j], 0, 0, 0);      \
-    small[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[1], bv[1], small[j], 0, 0, 0);      \
-    small[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0], bv[2], small[j], 0, 0, 0);      \
-    small[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[2], bv[0], small[j], 0, 0, 0);      \
+    chain = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0], bv[0], chain, 0, 0, 0);            \
+    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0], bv[1], small, 0, 0, 0);            \
+    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[1], bv[0], small, 0, 0, 0);            \
+    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[1], bv[1], small, 0, 0, 0);            \
+    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0], bv[2], small, 0, 0, 0);            \
+    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[2], bv[0], small, 0, 0, 0);            \
   }
 
-  acc16 acc[TN], odd[TN], small[TN];
+  acc16 acc, odd, small;
 #pragma unroll
-  for (int j = 0; j < TN; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[j][r] = odd[j][r] = small[j][r] = 0.f;
+  for (int r = 0; r < 16; ++r) acc[r] = odd[r] = small[r] = 0.f;
 
   if (w_end > w_begin) {
     // (a request past the run's end asks for its last tile again; nobody waits for it)
@@ -281,45 +276,37 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 1
 
   float probe = 0.f;  // NaN as soon as one sum of this lane is not finite
 #pragma unroll
-  for (int j = 0; j < TN; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      acc[j][r] = (acc[j][r] + (odd[j][r] + small[j][r])) * kSplitUnscale;
-      probe = __builtin_fmaf(acc[j][r], 0.f, probe);
-    }
+  for (int r = 0; r < 16; ++r) {
+    acc[r] = (acc[r] + (odd[r] + small[r])) * kSplitUnscale;
+    probe = __builtin_fmaf(acc[r], 0.f, probe);
+  }
   if (__any(probe != 0.f)) {
     // Rare, see igemm_split_kernel: the run again from fp32 values.
+    acc16 sum;
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      acc16 sum;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) sum[r] = 0.f;
-      for (int kt = w_begin; kt < w_end; ++kt) {
-        const uint16_t* w = reinterpret_cast<const uint16_t*>(wt_g + static_cast<size_t>(kt) * wt_kt_bytes + avoff);
+    for (int r = 0; r < 16; ++r) sum[r] = 0.f;
+    for (int kt = w_begin; kt < w_end; ++kt) {
+      const uint16_t* w = reinterpret_cast<const uint16_t*>(wt_g + static_cast<size_t>(kt) * wt_kt_bytes + avoff);
 #pragma unroll 2
-        for (int e = 0; e < 8; ++e) {
-          const int k = kt * BK + 8 * lhi + e;
-          unsigned off;
-          if constexpr (PW) {
-            off = k < a.K && !(voff[j] & kNoElement) ? voff[j] + static_cast<unsigned>(kt * BK + e) * x_cbytes
-                                                     : kNoElement;
-          } else {
-            const int4 tap = a.ktab[k];
-            off = (bad[j] >> tap.w) & 1u ? kNoElement : voff[j] + static_cast<unsigned>(tap.x);
-          }
-          const float wv = filter_value(w[e], w[a_plane / 2 + e], w[a_plane + e]);
-          sum = __builtin_amdgcn_mfma_f32_32x32x2f32(wv, MC_LOADF(off, 0), sum, 0, 0, 0);
+      for (int e = 0; e < 8; ++e) {
+        const int k = kt * BK + 8 * lhi + e;
+        unsigned off;
+        if constexpr (PW) {
+          off = k < a.K && !(voff & kNoElement) ? voff + static_cast<unsigned>(kt * BK + e) * x_cbytes : kNoElement;
+        } else {
+          const int4 tap = a.ktab[k];
+          off = (bad >> tap.w) & 1u ? kNoElement : voff + static_cast<unsigned>(tap.x);
         }
+        const float wv = filter_value(w[e], w[a_plane / 2 + e], w[a_plane + e]);
+        sum = __builtin_amdgcn_mfma_f32_32x32x2f32(wv, MC_LOADF(off, 0), sum, 0, 0, 0);
       }
-      acc[j] = sum;
     }
+    acc = sum;
   }
 #undef MC_LOADF
 
 #pragma unroll
-  for (int j = 0; j < TN; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) sums[wave][8 * (r / 4) + 4 * lhi + r % 4][j * 32 + l32] = acc[j][r];
+  for (int r = 0; r < 16; ++r) sums[wave][8 * (r / 4) + 4 * lhi + r % 4][l32] = acc[r];
   __syncthreads();
   float v[EPT];
 #pragma unroll
