@@ -296,30 +296,35 @@ int mcProposalWorkspaceSize(int num_proposals, int pre_nms_topn, int post_nms_to
  *            shape the top blob, as Forward_cpu's final Reshape does, :313-320)
  *   tie_flag optional device int: 0 when no order of equal scores had to be looked up,
  *            else 1 or 3 (see below).
- * Two steps, both queued by this call.  (1) The head of the table: the best 512
+ * Three steps, all queued by this call.  (1) The head of the table: the best 512
  * proposals are selected, ordered by (score descending, index ascending) and scanned;
  * the greedy pass usually reaches post_nms_topn kept boxes inside them.  Equal scores
  * among them matter only when two proposals of one score are both still alive when
  * the scan reaches them (the reference's quicksort SortBBox, :88-111, leaves equal
- * scores in an order of its own); a kernel checks that for every such group.  (2)
- * The full-size path, which skips itself on the device when step 1 settled the
- * result: all proposals are ordered by one radix sort; if equal scores reach into
+ * scores in an order of its own); a kernel checks that for every such group.
+ * (2) Where only that is open, SortBBox is replayed through the partitions that hold
+ * these groups, and the best 512 are scanned again (tie_flag 3).  (3) The full-size
+ * path: all proposals are ordered by one radix sort; if equal scores reach into
  * the first pre_nms_topn + 1 places, SortBBox is replayed on the device to give the
  * same row order (tie_flag 3 = by the kernel for inputs with few equal scores, which
  * follows only the partitions that hold equal scores, 1 = by the general kernel,
- * every partition, level by level); then the overlap bit matrix and the scan. */
+ * every partition, level by level); then the overlap bit matrix and the scan, of the
+ * best 512 first where no earlier step has scanned them in this order.  Steps 2 and 3
+ * skip themselves on the device once the result is settled. */
 int mcProposal(const float* scores, const float* bbox, const float* im_info, const float* anchors,
                int A, int H, int W, int feat_stride, float min_size, int pre_nms_topn,
                int post_nms_topn, float nms_thresh, void* workspace, size_t workspace_bytes,
                float* rois, float* roi_scores, int* num_rois, int* tie_flag, void* stream);
 
-/* The two steps of mcProposal as calls of their own, for a caller that reads num_rois
- * back anyway (the top's shape depends on it) and can read two more ints with it:
- * state[0] = tie_flag as above, state[1] = 1 when rois / num_rois are final.
- * mcProposalHead queues step 1 only (state[1] = 0: call mcProposalRest with the same
- * arguments, which starts over with the full-size path and always ends with
- * state[1] = 1).  Saves the launches of step 2 that would return at once.  No
- * counterpart in the reference. */
+/* The steps of mcProposal as calls of their own, for a caller that reads num_rois back
+ * anyway (the top's shape depends on it) and can read two more ints with it: state[0] =
+ * tie_flag as above, state[1] = 1 when rois / num_rois are final.
+ * mcProposalHead queues step 1 only.  state[1] = 0: call mcProposalContinue with the same
+ * arguments and the workspace as mcProposalHead left it; it queues steps 2 and 3 and
+ * always ends with state[1] = 1.  Saves the launches that would return at once.
+ * mcProposalRest needs no call before it: it decodes the proposals and takes step 3
+ * alone, and always ends with state[1] = 1 (behind mcProposalHead it does work twice
+ * that mcProposalContinue does not).  No counterpart in the reference. */
 int mcProposalHead(const float* scores, const float* bbox, const float* im_info, const float* anchors,
                    int A, int H, int W, int feat_stride, float min_size, int pre_nms_topn,
                    int post_nms_topn, float nms_thresh, void* workspace, size_t workspace_bytes,
@@ -328,17 +333,10 @@ int mcProposalRest(const float* scores, const float* bbox, const float* im_info,
                    int A, int H, int W, int feat_stride, float min_size, int pre_nms_topn,
                    int post_nms_topn, float nms_thresh, void* workspace, size_t workspace_bytes,
                    float* rois, float* roi_scores, int* num_rois, int* state, void* stream);
-/* What mcProposal queues behind step 1, for a caller of mcProposalHead that found
- * state[1] = 0: same arguments, and the workspace as mcProposalHead left it.  Where only the
- * order of equal scores among the best 512 proposals was open, SortBBox is replayed through
- * the partitions that hold them and the scan repeated; otherwise (and when that does not
- * settle the result) as mcProposalRest.  Always ends with state[1] = 1.  No counterpart in the
- * reference. */
 int mcProposalContinue(const float* scores, const float* bbox, const float* im_info, const float* anchors,
                        int A, int H, int W, int feat_stride, float min_size, int pre_nms_topn,
                        int post_nms_topn, float nms_thresh, void* workspace, size_t workspace_bytes,
                        float* rois, float* roi_scores, int* num_rois, int* state, void* stream);
-
 
 /* Measurement hook (no counterpart in the reference): while enabled on the calling
  * thread every mcProposal* call records HIP events between its stages on the launch
@@ -346,9 +344,8 @@ int mcProposalContinue(const float* scores, const float* bbox, const float* im_i
  * last collect stage_ms[0] decode + ordering of the head, [1] overlap matrix, scan and
  * check of the head + roi gather, [2] full-size path: radix sort, replay of the
  * reference's order of equal scores, gather of the best pre_nms_topn boxes and overlap
- * matrix of the best 512, [3] full-size path: greedy scans, overlap matrix of all + roi gather;
- * returns
- * the number of calls and clears the list. */
+ * matrix of the best 512, [3] full-size path: greedy scans, overlap matrix of all + roi
+ * gather; returns the number of calls and clears the list. */
 int mcProposalTimingEnable(int on);
 /* Test knob (process-wide): 1 = replay the order of equal scores with the general
  * level-by-level kernel on every input, also where the kernel for inputs with few
