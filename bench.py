@@ -23,7 +23,8 @@ sys.path.insert(0, os.path.join(ROOT, "mini-caffe_amd"))
 FP32_MFMA_PEAK_TFLOPS = 157.3
 HBM_PEAK_GBS = 8000.0
 CONV_SOURCES = [os.path.join(ROOT, "mini-caffe_amd", "csrc", "kernels", f)
-                for f in ("conv_igemm.hip", "igemm_split.h", "igemm_small.h", "igemm_finish.h", "conv_winograd.hip")]
+                for f in ("conv_igemm.hip", "igemm_split.h", "igemm_small.h", "small_rows.h", "igemm_finish.h",
+                          "conv_winograd.hip")]
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "igemm_resnet50_b64_pmc_traffic.txt")
 MFMA_PROFILE = os.path.join(ROOT, "profiles", "igemm_resnet50_b64_pmc_mfma_util.txt")
 

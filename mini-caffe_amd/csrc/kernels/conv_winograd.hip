@@ -569,6 +569,9 @@ bool winograd_fits(const WinogradState* w, int /*num*/) {
 // 1968 (128 -> 192 @24 b9) 30 / 24, 2048 (512 @7 b8) 38 / 25, 2432 (256 @14 b12) 32 / 27).  Of 112 launches
 // in that range the estimates choose the slower kernel by more than 2 % twice, by 4 % at most; all
 // together take 2775 us, 2803 without this path, 2772 with the better of the two each time.
+// In a network's forward the difference is smaller than in launches by themselves.  ms, with this path / without,
+// two nets in turn: ResNet-50 b64 3.845 / 3.899, b16 1.478 / 1.511, SSD300 b8 3.047 / 3.159, b2 1.283 / 1.258 (the one
+// of these that loses), RPN @38x63 0.190 / 0.218.
 // What loses: 32 input channels (the loop is four rounds long: 56 / 47 us), an
 // output tile that is half padding (64 -> 32: 86 / 82), and launches of a few tiles,
 // whose time is this kernel's longer prologue and finish (256 -> 150 on 5x5 maps, 9
