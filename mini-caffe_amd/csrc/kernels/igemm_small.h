@@ -19,7 +19,7 @@
 // us per launch, 64x64 tiles / this, launches of one layer one behind the other: 64 -> 64 3x3 on one 56x56 map
 // 10.2 / 7.0, 128 -> 128 @28 11.9 / 8.8, 256 -> 256 @14 13.8 / 9.3, 512 -> 512 @7 16.0 / 10.1, 256 -> 1024 1x1
 // @14 8.1 / 5.0, 1024 -> 256 10.2 / 7.2, 512 -> 2048 @7 8.5 / 5.8, 2048 -> 512 11.4 / 7.8, 512 -> 24 3x3 @10
-// 15.6 / 8.0.  Inside a network's forward, where the filters come from memory, 1 to 2 us more.
+// 15.6 / 8.0.  In the trace of a network's forward, where the filters come from memory, medians 0.6 to 0.8 us above these.
 // Sixteen wavefronts to a workgroup instead of slices: 13.6 us where four slices take 10.3.
 //
 // Lane l of the 32x32x16 product holds K rows 8 (l / 32) .. + 7 of filter row / pixel l % 32: of
