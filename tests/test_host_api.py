@@ -20,7 +20,7 @@ import wire
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 REF = "/root/reference"
-needs_ref = pytest.mark.skipif(not os.path.isdir(REF), reason="reference checkout not present")
+needs_ref = pytest.mark.skipif(not os.path.isdir(os.path.join(REF, "example")), reason="reference checkout not present")
 
 
 def declared_functions(header):
